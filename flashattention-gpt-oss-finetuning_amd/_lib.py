@@ -48,6 +48,7 @@ EXPORTS = (
     "fa_fwd_fp8",
     "fa_fwd_fp8_pv",
     "fa_bwd_workspace_bytes",
+    "fa_bwd_full_workspace_bytes",
     "fa_check_fwd",
     "fa_check_bwd",
     "fa_strerror",
@@ -154,6 +155,8 @@ def lib() -> ctypes.CDLL:
                 fn.restype = ctypes.c_int
             L.fa_bwd_workspace_bytes.argtypes = [ctypes.c_int32] * 7
             L.fa_bwd_workspace_bytes.restype = ctypes.c_size_t
+            L.fa_bwd_full_workspace_bytes.argtypes = [ctypes.c_int32] * 8
+            L.fa_bwd_full_workspace_bytes.restype = ctypes.c_size_t
             L.fa_check_fwd.argtypes = [ctypes.POINTER(FwdParams)]
             L.fa_check_fwd.restype = ctypes.c_int
             L.fa_check_bwd.argtypes = [ctypes.POINTER(BwdParams)]

@@ -73,6 +73,11 @@ struct Args {
   // B x n_kblocks blocks).
   int vl_units;
   int vl_kblocks;
+  // dK/dV split (kv_split > 1, see kv_split_plan in fa_capi.cpp): every key block's steps are cut into
+  // kv_split pieces, one workgroup each, whose fp32 sums go to kv_part [key block][piece][dK, dV]
+  // [64 D]; bwd_dkdv_fold_kernel adds the pieces in order.
+  int kv_split;
+  float* kv_part;
 };
 
 // Sequence b: its length and the row where it starts in the packed tensors (fixed-length
@@ -171,6 +176,9 @@ struct TailArgs {
   uint32_t fill[3];
 };
 
+// Compute units of the current device (fa_capi.cpp).
+int device_cus();
+
 // Launchers (return the hipError_t of the launch; launch_bwd_dkdv also launches the sink fold).
 hipError_t launch_fwd(const Args& a, int dtype, int D, int hpw, hipStream_t stream);
 // e4m3 q, k, v; bf16 o; fp8_pv: P V on the fp8 MFMA as well
@@ -181,6 +189,8 @@ hipError_t launch_bwd_dq_slide(const Args& a, int dtype, hipStream_t stream);
 // the sliding forward (the same, W <= 129; reads slide_ct / slide_ncu)
 hipError_t launch_fwd_slide(const Args& a, int dtype, hipStream_t stream);
 hipError_t launch_bwd_dkdv(const Args& a, int dtype, int D, hipStream_t stream);
+// does the 32-key dK/dV kernel serve this 16-bit backward on a device of `cus` compute units?
+bool dkdv4_eligible(const Args& a, int D, int cus);
 hipError_t launch_bwd_sink_logits(const Args& a, hipStream_t stream);  // after launch_bwd_dq
 hipError_t launch_varlen_tail(const TailArgs& t, hipStream_t stream);
 // float32 inputs (fa_f32.hip).  The dK/dV launch reads n_kblocks (32-key tiles), nsp (sink tiles

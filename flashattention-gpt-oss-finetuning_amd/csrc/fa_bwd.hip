@@ -737,9 +737,40 @@ __host__ __device__ inline bool dkdv_folds_in_kernel(const Args& a, int D, bool 
          ((a.dq_wgs + 3) & ~3) + 4 * 256 <= dkdv_lds_elems(D, kvl) / 2;
 }
 
+// Columns of a piece's sums in a.kv_part: a C tile is 32 columns wide, so D = 16 stores 32.
+template <int D>
+constexpr int kPartCols = D < 32 ? 32 : D;
+
+// Workgroup id -> piece, group and key block index of the split dK/dV grid (see bwd_dkdv_kernel):
+// `streams` = pieces x groups, `per` key blocks each.
+struct KvPiece {
+  int piece, group, p;
+};
+__device__ __forceinline__ KvPiece kv_piece(int id, int streams, int ns, int per) {
+  int stream, p;
+  if (streams % 8 == 0) {  // XCD id % 8 owns streams / 8 streams
+    const int spx = streams / 8, pos = id / 8;
+    p = pos / spx;
+    stream = id % 8 * spx + pos % spx;
+  } else {
+    p = id / streams;
+    stream = id % streams;
+  }
+  (void)per;
+  return KvPiece{stream % ns, stream / ns, p};
+}
+
 // D = 16 keeps four waves per SIMD (at most 128 VGPRs), D = 64 with KVL three (168); the wider
 // head dims need more registers.
-template <typename E, int D, bool KVL = false>
+//
+// SPLIT (a.kv_split > 1): a key block's steps are cut into kv_split contiguous pieces, one workgroup
+// each, which write their fp32 sums to a.kv_part; bwd_dkdv_fold_kernel adds them.  For grids whose
+// longest workgroup takes longer than the chip's average (full causal layers up to a few thousand
+// rows: key block 0 is seen by every row).  Piece s of a group (b, KV head) is a stream of
+// workgroups, one per key block; an XCD owns whole streams where their number allows (pieces are
+// whole query heads when kv_split divides G, so its L2 holds those heads' rows only) and takes
+// their key blocks together, the longest first.
+template <typename E, int D, bool KVL = false, bool SPLIT = false>
 __global__ __launch_bounds__(256, D == 16 ? 4 : KVL ? 3 : 1) void bwd_dkdv_kernel(const Args a) {
   constexpr int KS = D / 16;
   constexpr int DB = D >= 32 ? D / 32 : 1;
@@ -762,13 +793,38 @@ __global__ __launch_bounds__(256, D == 16 ? 4 : KVL ? 3 : 1) void bwd_dkdv_kerne
   // chunks.  A group's workgroups land on one XCD (they share its L2), and the short chunk
   // workgroups run last, filling the slots that the regular ones leave.
   const int per_group = a.n_kblocks + a.nsp * a.n_chunks;
-  const int id = xcd_remap(blockIdx.x, gridDim.x);
+  const int id = SPLIT ? int(blockIdx.x) : xcd_remap(blockIdx.x, gridDim.x);
   // groups in (KV head, batch) order, the KV head outermost: the XCDs then split over KV heads
   // before sequences, which keeps their work even for sequences of different lengths.  A packed
   // batch hands out only the key blocks with keys: per KV head, each sequence's blocks
   // (varlen_nth), then the sequences' chunk workgroups.
   int kvh, b, r;
-  if (a.vl_kblocks) {
+  int piece = 0;          // SPLIT: this workgroup's piece of its key block
+  int64_t part_slot = 0;  // SPLIT: and its slot in a.kv_part
+  if constexpr (SPLIT) {
+    const int ns = a.kv_split;
+    const int per = a.vl_kblocks ? a.vl_kblocks : a.n_kblocks;      // key blocks per stream
+    const int streams = ns * a.Hkv * (a.vl_kblocks ? 1 : a.B);
+    if (id < streams * per) {
+      const KvPiece t = kv_piece(id, streams, ns, per);
+      piece = t.piece;
+      part_slot = (int64_t(t.group) * per + t.p) * ns + piece;
+      if (a.vl_kblocks) {
+        kvh = t.group;
+        if (!varlen_nth(a, t.p, per, kKvKeys, 1, b, r)) return;
+      } else {
+        kvh = t.group / a.B;
+        b = t.group % a.B;
+        r = t.p;
+      }
+    } else {  // the sink-chunk workgroups
+      const int n_cw = a.nsp * a.n_chunks;
+      const int c = id - streams * per;
+      kvh = c / (a.B * n_cw);
+      b = c / n_cw % a.B;
+      r = a.n_kblocks + c % n_cw;
+    }
+  } else if (a.vl_kblocks) {
     const int n_cw = a.nsp * a.n_chunks;
     const int per_kv = a.vl_kblocks + a.B * n_cw;
     kvh = id / per_kv;
@@ -844,7 +900,15 @@ __global__ __launch_bounds__(256, D == 16 ? 4 : KVL ? 3 : 1) void bwd_dkdv_kerne
   const int qb_lo = qlo / 32;
   const int n_qb = qhi > qlo ? (qhi + 31) / 32 - qb_lo : 0;
   const int n_qp = (n_qb + 1) / 2;
-  const int n_steps = G * n_qp;
+  // this workgroup's steps [s_lo, s_lo + n_steps) of the G n_qp
+  int s_lo = 0, n_steps = G * n_qp;
+  if constexpr (SPLIT) {
+    if (!is_chunk) {
+      const int64_t n = n_steps;
+      s_lo = int(n * piece / a.kv_split);
+      n_steps = int(n * (piece + 1) / a.kv_split) - s_lo;
+    }
+  }
 
   // ---- staging.  Everything a step reads goes straight from memory into an LDS stage by DMA
   // (buffer_load ... lds): the four 32-row tiles (slot 0 Q, slot 0 dO, slot 1 Q, slot 1 dO; wave w
@@ -883,6 +947,12 @@ __global__ __launch_bounds__(256, D == 16 ? 4 : KVL ? 3 : 1) void bwd_dkdv_kerne
   const int s_slot = wave & 1;              // the slot whose statistics this wave loads
   // fetch side: the step (fh, fp) being loaded and the descriptors of head fh
   int fh = 0, fp = 0;
+  if constexpr (SPLIT) {
+    if (n_steps > 0) {
+      fh = s_lo / n_qp;
+      fp = s_lo % n_qp;
+    }
+  }
   rsrc_t rtile, rstat;
   auto set_head = [&]() {
     rtile = make_rsrc(tile_slice + int64_t(fh) * 2 * t_hs, nt_bytes);
@@ -997,7 +1067,8 @@ __global__ __launch_bounds__(256, D == 16 ? 4 : KVL ? 3 : 1) void bwd_dkdv_kerne
     // loads NSTG - 1 steps ahead; step s waits for its own
     for (int k = 0; k < NSTG - 1; ++k) issue(k);
     if constexpr (!KVL) kv_operands_ready(kf, vf);
-    int cp = 0, cur = 0, nxt = NSTG - 1;  // stage of step s, stage of step s + NSTG - 1
+    int cp = SPLIT ? s_lo % n_qp : 0;     // block pair of step s
+    int cur = 0, nxt = NSTG - 1;          // stage of step s, stage of step s + NSTG - 1
     for (int s = 0; s < n_steps; ++s) {
       wait_vm_lgkm0_barrier<(NSTG - 2) * PER>();  // step s landed everywhere
       // (D = 128 issues after its compute: measured 4% faster there, slower at D = 64)
@@ -1037,6 +1108,25 @@ __global__ __launch_bounds__(256, D == 16 ? 4 : KVL ? 3 : 1) void bwd_dkdv_kerne
         dk[db][e] += red[((kh * 2 + 0) * DB * 16 + db * 16 + e) * 64 + lane];
         dv[db][e] += red[((kh * 2 + 1) * DB * 16 + db * 16 + e) * 64 + lane];
       }
+  }
+
+  // ---- a piece's sums: 16-byte chunk (kh, db, e / 4) of lane l at [chunk][l], whole lines per store
+  if constexpr (SPLIT) {
+    if (!is_chunk) {
+      if (hh == 0) {
+        float* out = a.kv_part + part_slot * (2 * kKvKeys * kPartCols<D>) + kh * (DB * 16 * 64) + 4 * lane;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int e4 = 0; e4 < 4; ++e4) {
+            float* o = out + (db * 4 + e4) * 256;
+            *reinterpret_cast<f32x4*>(o) = f32x4{dk[db][4 * e4], dk[db][4 * e4 + 1], dk[db][4 * e4 + 2], dk[db][4 * e4 + 3]};
+            *reinterpret_cast<f32x4*>(o + kKvKeys * kPartCols<D>) =
+                f32x4{dv[db][4 * e4], dv[db][4 * e4 + 1], dv[db][4 * e4 + 2], dv[db][4 * e4 + 3]};
+          }
+      }
+      return;
+    }
   }
 
   // ---- outputs: lane (key, hf) holds head-dim indices 32db + 16hf + e (D == 16: hf == 0) ------
@@ -1603,6 +1693,59 @@ __global__ __launch_bounds__(256) void bwd_sink_fold_kernel(const Args a) {
   fold_sink_key<E, D>(b, kvh, key, sq, part);
 }
 
+// ---------------------------------------------------------------------------------------------
+// Adds the kv_split pieces of every key block's dK/dV (bwd_dkdv_kernel with SPLIT), piece by piece in
+// order, and writes dK and dV; the sink rows of a block whose later rows go elsewhere (key < S,
+// block < nsp) go to that block's own slot of the sink partials instead.  One thread per 8 columns
+// of a key row of dK or dV; bound by reading kv_split x 8 bytes per element once.
+// ---------------------------------------------------------------------------------------------
+template <typename E, int D>
+__global__ __launch_bounds__(256) void bwd_dkdv_fold_kernel(const Args a) {
+  constexpr int DB = D >= 32 ? D / 32 : 1;
+  constexpr int UNITS = 2 * 2 * DB * 2 * 64;  // [dK, dV][key half][db][16-byte chunk pair][lane]
+  static_assert(UNITS % 256 == 0, "whole workgroups per key block");
+  constexpr int WGS = UNITS / 256;
+  const int per = a.vl_kblocks ? a.vl_kblocks : a.n_kblocks;
+  const int blk = blockIdx.x / WGS;  // group * per + p
+  const int u = (blockIdx.x % WGS) * 256 + threadIdx.x;
+  const int lane = u & 63, c2 = (u >> 6) & 1, db = (u >> 7) % DB, kh = (u >> 7) / DB & 1, t = (u >> 7) / (2 * DB);
+  int kvh, b, kblk;
+  if (a.vl_kblocks) {
+    kvh = blk / per;
+    if (!varlen_nth(a, blk % per, per, kKvKeys, 1, b, kblk)) return;
+  } else {
+    const int grp = blk / per;
+    kblk = blk % per;
+    kvh = grp / a.B;
+    b = grp % a.B;
+  }
+  const Seq sq = seq_of(a, b);
+  const int r32 = lane & 31, hf = lane >> 5;
+  const int key = kKvKeys * kblk + 32 * kh + r32;
+  if (key >= sq.L || (D == 16 && hf == 1)) return;
+  const int ns = a.kv_split;
+  constexpr int HALF = kKvKeys * kPartCols<D>;  // floats of one tensor's sums
+  const float* src = a.kv_part + int64_t(blk) * ns * (2 * HALF) + t * HALF + ((kh * DB + db) * 4 + 2 * c2) * 256 + 4 * lane;
+  f32x4 x0 = {0.f, 0.f, 0.f, 0.f}, x1 = x0;
+  for (int s = 0; s < ns; ++s) {
+    x0 += *reinterpret_cast<const f32x4*>(src + int64_t(s) * (2 * HALF));
+    x1 += *reinterpret_cast<const f32x4*>(src + int64_t(s) * (2 * HALF) + 256);
+  }
+  const int d0 = 32 * db + (D >= 32 ? 16 * hf : 0) + 8 * c2;
+  if (kblk < a.nsp && key < a.S) {
+    const int64_t bk = (int64_t(b) * a.Hkv + kvh) * a.nsp + kblk;
+    float* o = a.partial + ((bk * (a.n_chunks + 1) + a.n_chunks) * 2 + t) * a.srows * D + (32 * kh + r32) * D + d0;
+    *reinterpret_cast<f32x4*>(o) = x0;
+    *reinterpret_cast<f32x4*>(o + 4) = x1;
+    return;
+  }
+  const float sc = t == 0 ? a.scale : 1.f;
+  const float v[8] = {x0[0] * sc, x0[1] * sc, x0[2] * sc, x0[3] * sc, x1[0] * sc, x1[1] * sc, x1[2] * sc, x1[3] * sc};
+  char* dst = t == 0 ? reinterpret_cast<char*>(a.dk) + 2 * slice_off(a.sdk, b, kvh, sq.row + key)
+                     : reinterpret_cast<char*>(a.dv) + 2 * slice_off(a.sdv, b, kvh, sq.row + key);
+  st16(dst + 2 * d0, pack8<E>(v));
+}
+
 // The D = 128 dQ and dK/dV kernels and the D = 64 dQ kernel without sink rows are instantiated in
 // fa_bwd_wide.hip, which includes this file
 // with FA_BWD_WIDE_TU defined and is compiled with another machine scheduler; everything below
@@ -1616,6 +1759,8 @@ extern template __global__ void bwd_dq_kernel<F16, 128, false>(const Args);
 extern template __global__ void bwd_dq_kernel<F16, 128, true>(const Args);
 extern template __global__ void bwd_dkdv_kernel<BF16, 128>(const Args);
 extern template __global__ void bwd_dkdv_kernel<F16, 128>(const Args);
+extern template __global__ void bwd_dkdv_kernel<BF16, 128, false, true>(const Args);
+extern template __global__ void bwd_dkdv_kernel<F16, 128, false, true>(const Args);
 
 // ---------------------------------------------------------------------------------------------
 // Gradient of the learned sink logits: dsink[h] = sum over (b, 32-row block) of the dQ kernel's
@@ -1689,14 +1834,6 @@ static int resident_per_cu() {
   return cached;
 }
 
-static int device_cus() {
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      n < 1)
-    n = 256;
-  return n;
-}
-
 // Grid of the dQ kernel: one resident wave of workgroups, a multiple of the 8 XCDs (the sink
 // fold recomputes it to find the dQ kernel's sink slots).
 template <typename E, int D, bool SINK>
@@ -1724,9 +1861,9 @@ static hipError_t launch_dq_d(const Args& a, int, hipStream_t stream) {
 // fewer rows and no idle waves, finish sooner (measured on MI355X: 19.5 us against 29.5 us at
 // L = 4096, W = 128, 8 heads).  On a full chip of 64-key workgroups bwd_dkdv_kernel is faster (its
 // two key halves share each staged tile), as for full causal and long windows.
-static bool dkdv4_eligible(const Args& a, int D) {
+bool dkdv4_eligible(const Args& a, int D, int cus) {
   return D <= 64 && a.G % 4 == 0 && a.W >= 1 && a.W <= 512 && (a.nsp == 0 || (a.sink_dq && a.n_chunks == 0)) &&
-         int64_t(a.B) * a.Hkv * ((a.L + kKvKeys - 1) / kKvKeys) <= device_cus();
+         int64_t(a.B) * a.Hkv * ((a.L + kKvKeys - 1) / kKvKeys) <= cus;
 }
 
 // The D = 64 dK/dV kernel with its K/V operands in LDS (three workgroups per CU instead of two)
@@ -1757,9 +1894,17 @@ static hipError_t launch_dkdv_d(const Args& a, hipStream_t stream) {
   // the in-kernel fold finds the dQ slots by the dQ grid (and sizes its run list in LDS by it)
   if (a.sink_dq) ad.dq_wgs = a.dq_slide ? (a.G / 8) * a.slide_ncu : dq_grid<E, D, true>(a);
   hipError_t e;
-  bool folded;
-  if constexpr (D <= 64) {
-    if (dkdv4_eligible(a, D)) {
+  bool folded = false;
+  if (a.kv_split > 1) {  // (kv_split_plan leaves dkdv4_eligible shapes alone)
+    const int blocks = a.Hkv * (a.vl_kblocks ? a.vl_kblocks : a.B * a.n_kblocks);
+    hipLaunchKernelGGL((bwd_dkdv_kernel<E, D, false, true>), dim3(a.kv_split * blocks + a.n_chunk_wgs), dim3(256), 0, stream, ad);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    constexpr int kWgs = 2 * (D >= 32 ? D / 32 : 1);  // workgroups per key block
+    hipLaunchKernelGGL((bwd_dkdv_fold_kernel<E, D>), dim3(kWgs * blocks), dim3(256), 0, stream, ad);
+    e = hipGetLastError();
+  } else if constexpr (D <= 64) {
+    if (dkdv4_eligible(a, D, device_cus())) {
       ad.n_kblocks = (a.L + 31) / 32;  // 32-key blocks
       const int grid = a.B * a.Hkv * ad.n_kblocks;
       const int nw = dkdv4_waves(a, D, grid);

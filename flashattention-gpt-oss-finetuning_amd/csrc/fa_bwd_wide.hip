@@ -18,4 +18,6 @@ template __global__ void bwd_dq_kernel<F16, 128, false>(const Args);
 template __global__ void bwd_dq_kernel<F16, 128, true>(const Args);
 template __global__ void bwd_dkdv_kernel<BF16, 128>(const Args);
 template __global__ void bwd_dkdv_kernel<F16, 128>(const Args);
+template __global__ void bwd_dkdv_kernel<BF16, 128, false, true>(const Args);
+template __global__ void bwd_dkdv_kernel<F16, 128, false, true>(const Args);
 }  // namespace fa

@@ -6,6 +6,7 @@
 // plus what the kernels assume (16-byte aligned rows, D in {16, 32, 64, 128}).  Nothing in
 // fa_check_* touches HIP, so the checks run on machines without a GPU.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -157,15 +158,6 @@ void copy3(int64_t dst[3], const int64_t src[3]) {
   for (int i = 0; i < 3; ++i) dst[i] = src[i];
 }
 
-// Compute units of the current device (256 on MI355X; 256 if the query fails).
-int device_cus() {
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      n < 1)
-    n = 256;
-  return n;
-}
-
 // Tiles per unit (slide_ct) of the sliding kernels, for `slots` resident units.  A fixed-length
 // batch spreads its B Hkv (G / 8) n_qt tiles evenly over the slots.  A packed batch holds at most
 // T = ceil(total_rows / 32) + B tiles with rows (each sequence adds at most one partial tile),
@@ -206,7 +198,7 @@ int vl_units(const fa::Args& a) {
 void plan_slide(fa::Args& a, int D) {
   if (D != 64 || a.G % 8 != 0 || a.W < 1 || a.W > fa::kSlideMaxW || a.S > 32 || a.L < 1) return;
   const int64_t n_qt = (int64_t(a.L) + 31) / 32;
-  const int64_t ct = slide_units_ct(a, device_cus());
+  const int64_t ct = slide_units_ct(a, fa::device_cus());
   a.dq_slide = 1;
   a.slide_ct = int(ct);
   a.slide_ncu = int((n_qt + ct - 1) / ct);
@@ -220,7 +212,7 @@ bool plan_fwd_slide(fa::Args& a, int D, int dtype) {
       a.L < 1)
     return false;
   const int64_t n_qt = (int64_t(a.L) + 31) / 32;
-  const int64_t ct = slide_units_ct(a, 2 * int64_t(device_cus()));
+  const int64_t ct = slide_units_ct(a, 2 * int64_t(fa::device_cus()));
   a.slide_ct = int(ct);
   a.slide_ncu = int((n_qt + ct - 1) / ct);
   a.vl_units = vl_units(a);
@@ -233,6 +225,92 @@ int vl_kblocks(const fa::Args& a) {
   if (!a.cu_seqlens) return 0;
   const int64_t bound = (int64_t(a.total_rows) + fa::kKvKeys - 1) / fa::kKvKeys + a.B;
   return bound < int64_t(a.B) * a.n_kblocks ? int(bound) : 0;
+}
+
+// Steps (pairs of 32-row blocks, times query heads) that the dK/dV kernel's workgroups of one (batch,
+// KV head) sweep: the longest workgroup's and all of them.  Blocks whose window ends inside the
+// sequence all sweep the same rows; the others sweep to the last row, one pair fewer per block.
+struct KvSteps {
+  double longest, total;
+};
+KvSteps kv_steps(double L, double W, double G) {
+  const double n_kb = std::ceil(L / fa::kKvKeys);
+  const double win = std::ceil((fa::kKvKeys - 1 + W) / 64.);  // pairs of a whole window
+  const double n_win = std::min(n_kb, std::max(0., std::floor((L - W + 1) / fa::kKvKeys)));
+  const double r = n_kb - n_win;
+  return KvSteps{G * (n_win > 0 ? win : n_kb), G * (n_win * win + r * (r + 1) / 2)};
+}
+
+// Pieces per key block of the dK/dV kernel (1: unsplit) for `nseq` sequences of L rows on `cus` compute
+// units: the power of two up to 32 with the least estimated time.  The kernel takes as long as its
+// longest workgroup (a full causal layer's key block 0 sweeps every row, twice the average), or as
+// the average work of a resident slot where that is more, or half of each, at the rate of full slots,
+// where the longest starts on a full chip; splitting shortens the first, and costs
+// writing and reading the pieces' fp32 sums, the launch that adds them, and the sink fold's launch
+// where the dK/dV kernel would have folded (`folds`).  Measured on MI355X, in us a step: longest
+// workgroups 0.55 / 0.58 / 0.8 / 1.15 at D = 16 / 32 / 64 / 128, full slots 1.3 / 1.5 / 1.14 / 1.25;
+// 5 us a launch, 0.35 us per MB of sums.  Full causal D = 64, Hq = 64, Hkv = 8, dK/dV in us by pieces
+// 1 / 2 / 4 / 8 / 16: L = 1024 106 / 61 / 41 / 39 / 50; L = 2048 207 / 122 / 90 / 101 / 124; L = 4096
+// 434 / 298 / 302 / 321 / 386; L = 8192 1137 / 1125 / 1140 / 1198 / 1339; Hq = 8, Hkv = 1, L = 2048
+// 202 / 106 / 59 / 38 / 31; D = 128, Hq = 32, Hkv = 8, L = 2048 149 / 102 / 113 / 142 / 220; with a
+// window of 1024 at L = 4096 (equal workgroups) 143 / 154 / 162 / 177 / 245.
+int kv_split_pieces(int D, int G, int Hkv, double nseq, double L, double W, bool folds, int cus) {
+  const int i = D == 16 ? 0 : D == 32 ? 1 : D == 64 ? 2 : 3;
+  const double t_long[4] = {0.55, 0.58, 0.8, 1.15}, t_slot[4] = {1.3, 1.5, 1.14, 1.25};
+  const int per_cu[4] = {4, 4, 2, 1};  // resident workgroups
+  const KvSteps st = kv_steps(L, W, G);
+  const double slot = t_slot[i] * st.total * nseq * Hkv / (double(cus) * per_cu[i]);
+  const double mb = nseq * Hkv * std::ceil(L / fa::kKvKeys) * fa::kKvKeys * (D < 32 ? 32 : D) * 8 * 1e-6;  // per piece
+  auto kernel_us = [&](double longest) {
+    return std::max({t_long[i] * longest, slot, 0.5 * (slot + t_slot[i] * longest)});
+  };
+  int best = 1;
+  double best_t = kernel_us(st.longest);
+  for (int ns = 2; ns <= 32 && ns <= st.longest; ns *= 2) {
+    const double t = kernel_us(st.longest / ns) + 5 + 0.35 * mb * ns + (folds ? 5 : 0);
+    if (t < 0.95 * best_t) {
+      best = ns;
+      best_t = t;
+    }
+  }
+  return best;
+}
+
+// bytes of kv_part for `blocks` key blocks (of every KV head) in `ns` pieces
+size_t kv_part_bytes(int D, int64_t blocks, int ns) {
+  return ns > 1 ? align256(size_t(blocks) * ns * 2 * fa::kKvKeys * (D < 32 ? 32 : D) * sizeof(float)) : 0;
+}
+
+// key blocks of every KV head that the dK/dV kernel's grid holds
+int64_t kv_blocks(const fa::Args& a) {
+  return int64_t(a.Hkv) * (a.vl_kblocks ? a.vl_kblocks : int64_t(a.B) * a.n_kblocks);
+}
+
+// Splits the dK/dV kernel (kv_split, kv_part) as far as the `spare` bytes of workspace at `ws` allow.
+// The rows of a packed batch are taken to be spread evenly over its sequences (the host does not
+// know their lengths).
+void plan_kv_split(fa::Args& a, int D, char* ws, size_t spare) {
+  a.kv_split = 1;
+  const int cus = fa::device_cus();
+  if (fa::dkdv4_eligible(a, D, cus)) return;
+  const double rows = a.cu_seqlens ? std::min(double(a.L), std::max(1., double(a.total_rows) / a.B)) : double(a.L);
+  int ns = kv_split_pieces(D, a.G, a.Hkv, a.B, rows, a.W, a.sink_dq != 0, cus);
+  const int64_t blocks = kv_blocks(a);
+  while (ns > 1 && (kv_part_bytes(D, blocks, ns) > spare || blocks * ns > (int64_t(1) << 24))) ns /= 2;
+  a.kv_split = ns;
+  a.kv_part = reinterpret_cast<float*>(ws);
+}
+
+// The kernel arguments that the 16-bit dK/dV kernel's plan reads.
+void set_kv_plan(fa::Args* a, int window, int sink) {
+  const SinkPlan sp = sink_plan(a->L, window, sink);
+  a->sink_dq = sp.dq;
+  a->n_kblocks = (a->L + fa::kKvKeys - 1) / fa::kKvKeys;
+  a->nsp = sp.nsp;
+  a->n_chunks = sp.n_chunks;
+  a->chunk_rows = kChunkRows;
+  a->srows = sp.srows;
+  a->n_chunk_wgs = a->B * a->Hkv * a->nsp * a->n_chunks;
 }
 
 fa::Args base_args(int32_t B, int32_t Hq, int32_t Hkv, int32_t L, int32_t D, int32_t W, int32_t S,
@@ -259,6 +337,18 @@ fa::Args base_args(int32_t B, int32_t Hq, int32_t Hkv, int32_t L, int32_t D, int
 }
 
 }  // namespace
+
+// Compute units of the current device (256 on MI355X; 256 if the query fails), looked up once per
+// device: launches plan with it several times a call.
+int fa::device_cus() {
+  static std::atomic<int> known[64];
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 256;
+  if (dev < 64 && (n = known[dev].load(std::memory_order_relaxed)) > 0) return n;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) return 256;
+  if (dev < 64) known[dev].store(n, std::memory_order_relaxed);
+  return n;
+}
 
 extern "C" {
 
@@ -482,12 +572,29 @@ size_t fa_bwd_workspace_bytes(int32_t batch, int32_t heads_q, int32_t heads_kv, 
          partial_region_bytes(batch, heads_q, heads_kv, seqlen, head_dim, window, sink);
 }
 
+size_t fa_bwd_full_workspace_bytes(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t seqlen, int32_t head_dim,
+                                   int32_t window, int32_t sink, int32_t total_rows) {
+  const size_t need = fa_bwd_workspace_bytes(batch, heads_q, heads_kv, seqlen, head_dim, window, sink);
+  if (need == 0) return 0;
+  fa::Args a = base_args(batch, heads_q, heads_kv, seqlen, head_dim, window, sink, 1.f);
+  set_kv_plan(&a, window, sink);
+  if (total_rows >= 0) {
+    a.cu_seqlens = &total_rows;  // (only whether there are offsets matters to the plan)
+    a.total_rows = total_rows;
+    a.vl_kblocks = vl_kblocks(a);
+  }
+  plan_kv_split(a, head_dim, nullptr, SIZE_MAX);
+  return need + kv_part_bytes(head_dim, kv_blocks(a), a.kv_split);
+}
+
 }  // extern "C"
 
 namespace {
 
 // Validates a backward call and fills the kernel arguments; returns FA_OK or an fa_status.
-int prepare_bwd(const fa_bwd_params* p, void* workspace, size_t workspace_bytes, fa::Args* out, int* hpw) {
+// cu_seqlens: a packed batch (checked by the caller).
+int prepare_bwd(const fa_bwd_params* p, void* workspace, size_t workspace_bytes, fa::Args* out, int* hpw,
+                const int32_t* cu_seqlens = nullptr, int32_t total_rows = 0) {
   const int rc = fa_check_bwd(p);
   if (rc != FA_OK) return rc;
   const size_t need = fa_bwd_workspace_bytes(p->batch, p->heads_q, p->heads_kv, p->seqlen, p->head_dim,
@@ -533,19 +640,19 @@ int prepare_bwd(const fa_bwd_params* p, void* workspace, size_t workspace_bytes,
     a.nsp = fp.nsp;
     a.n_chunks = fp.n_chunks;
     a.chunk_rows = kF32ChunkRows;
+    if (cu_seqlens) set_varlen(&a, cu_seqlens, total_rows);
     *out = a;
     return FA_OK;
   }
-  const SinkPlan sp = sink_plan(a.L, p->window, p->sink);
-  a.sink_dq = sp.dq;
-  if (sp.dq) a.dq_sink_part = a.partial + partial_bytes(a.B, a.Hkv, p->head_dim, sp) / sizeof(float);
-  a.n_kblocks = (a.L + fa::kKvKeys - 1) / fa::kKvKeys;
-  a.nsp = sp.nsp;
-  a.n_chunks = sp.n_chunks;
-  a.chunk_rows = kChunkRows;
-  a.srows = sp.srows;
-  a.n_chunk_wgs = a.B * a.Hkv * a.nsp * a.n_chunks;
+  set_kv_plan(&a, p->window, p->sink);
+  if (a.sink_dq)
+    a.dq_sink_part = a.partial + partial_bytes(a.B, a.Hkv, p->head_dim, sink_plan(a.L, p->window, p->sink)) / sizeof(float);
+  if (cu_seqlens) {
+    set_varlen(&a, cu_seqlens, total_rows);
+    a.vl_kblocks = vl_kblocks(a);
+  }
   plan_slide(a, p->head_dim);
+  plan_kv_split(a, p->head_dim, ws + need, workspace_bytes - need);
   *out = a;
   return FA_OK;
 }
@@ -597,14 +704,12 @@ int fa_bwd_varlen(const fa_bwd_params* p, const int32_t* cu_seqlens, int32_t tot
                   float* dsinks, void* workspace, size_t workspace_bytes, void* stream) {
   fa::Args a;
   int hpw = 1;
-  int rc = prepare_bwd(p, workspace, workspace_bytes, &a, &hpw);
-  if (rc == FA_OK) rc = check_varlen(cu_seqlens, total_rows);
+  const int vrc = check_varlen(cu_seqlens, total_rows);
+  int rc = prepare_bwd(p, workspace, workspace_bytes, &a, &hpw, vrc == FA_OK ? cu_seqlens : nullptr, total_rows);
+  if (rc == FA_OK) rc = vrc;
   if (rc != FA_OK) return rc;
   if (!sinks != !dsinks) return FA_ERR_NULL;
   if ((sinks && !aligned4(sinks)) || (dsinks && !aligned4(dsinks))) return FA_ERR_ALIGN;
-  set_varlen(&a, cu_seqlens, total_rows);
-  if (a.dq_slide) plan_slide(a, p->head_dim);  // size the units by the rows the batch holds
-  if (p->dtype != FA_DTYPE_F32) a.vl_kblocks = vl_kblocks(a);
   a.sink_logits = sinks;
   a.dsink = dsinks;
   const hipStream_t s = static_cast<hipStream_t>(stream);

@@ -4,7 +4,7 @@
 // caching allocator), the current HIP stream, filling fa_fwd_params / fa_bwd_params and the
 // launch -- in C++, so a forward + backward costs a few microseconds of host time instead of
 // the tens that per-field ctypes marshalling takes.  Every FLOP still runs in libfa_gfx950.so;
-// this module only calls fa_fwd / fa_bwd / fa_fwd_sinks / fa_bwd_sinks / fa_bwd_workspace_bytes /
+// this module only calls fa_fwd / fa_bwd / fa_fwd_sinks / fa_bwd_sinks / fa_bwd_full_workspace_bytes /
 // fa_strerror.  swda / swda_sinks are the autograd functions themselves in C++ (forward, saved
 // tensors, backward), which the functional forms of the Python package call.
 //
@@ -147,8 +147,8 @@ std::vector<at::Tensor> bwd(const at::Tensor& q_in, const at::Tensor& k_in, cons
   at::Tensor dq = at::empty_like(q);
   at::Tensor dk = at::empty_like(k);
   at::Tensor dv = at::empty_like(v);
-  const size_t ws_bytes = fa_bwd_workspace_bytes(clamp_i32(B), clamp_i32(Hq), clamp_i32(Hkv), clamp_i32(L),
-                                                 clamp_i32(D), clamp_i32(window), clamp_i32(sink));
+  const size_t ws_bytes = fa_bwd_full_workspace_bytes(clamp_i32(B), clamp_i32(Hq), clamp_i32(Hkv), clamp_i32(L),
+                                                      clamp_i32(D), clamp_i32(window), clamp_i32(sink), -1);
   at::Tensor ws = at::empty({int64_t(ws_bytes > 256 ? ws_bytes : 256)}, q.options().dtype(at::kByte));
   fa_bwd_params p{};
   p.q = q.data_ptr();

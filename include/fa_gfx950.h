@@ -130,9 +130,18 @@ int fa_fwd(const fa_fwd_params* p, void* stream);
 size_t fa_bwd_workspace_bytes(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t seqlen,
                               int32_t head_dim, int32_t window, int32_t sink);
 
+/* The workspace with which the backward is fastest, at least fa_bwd_workspace_bytes(): where one
+ * workgroup per 64 keys would leave compute units idle it adds room for the fp32 partial sums of a
+ * dK/dV kernel with several.  total_rows: the packed rows of fa_bwd_varlen (with seqlen the longest
+ * sequence), or -1 for a fixed-length batch.  fa_bwd* use what room they are given: dk and dv of a
+ * call with less room differ from those of one with more by the order of fp32 sums.  Returns 0
+ * for an invalid problem. */
+size_t fa_bwd_full_workspace_bytes(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t seqlen,
+                                   int32_t head_dim, int32_t window, int32_t sink, int32_t total_rows);
+
 /* Launches the backward kernels (fa_bwd_dq then fa_bwd_dkdv).  `workspace` must hold
- * fa_bwd_workspace_bytes() bytes of device memory, 256-byte aligned; its contents on entry do
- * not matter. */
+ * at least fa_bwd_workspace_bytes() bytes of device memory, 256-byte aligned; its contents on entry
+ * do not matter. */
 int fa_bwd(const fa_bwd_params* p, void* workspace, size_t workspace_bytes, void* stream);
 
 /* The two stages of fa_bwd, for callers that schedule or time them separately.
@@ -154,7 +163,7 @@ int fa_bwd_dkdv(const fa_bwd_params* p, void* workspace, size_t workspace_bytes,
  * until the process ends; the call itself allocates and frees nothing.  Its first call on a GPU looks
  * up the buffer's address there (hipGetSymbolAddress): make that call outside any graph capture,
  * after which calls may be captured.  Same arguments, checks, kernels and
- * results as fa_bwd (bitwise).  Returns FA_ERR_SCRATCH when fa_bwd_workspace_bytes() of the
+ * results as fa_bwd with a workspace of FA_SCRATCH_BYTES (bitwise).  Returns FA_ERR_SCRATCH when fa_bwd_workspace_bytes() of the
  * problem exceeds FA_SCRATCH_BYTES.  Every call on one GPU shares that GPU's buffer: calls that
  * overlap in time on one GPU (concurrent streams, or host threads launching without ordering)
  * race on it and must be serialised by the caller; calls in one stream are ordered and safe. */
@@ -196,7 +205,7 @@ int fa_bwd_sinks(const fa_bwd_params* p, const float* sinks, float* dsinks, void
  *     get o = 0 and lse = -inf from fa_fwd_varlen and zero dq, dk, dv from fa_bwd_varlen (one
  *     small extra launch, which exits at once when every row is covered).
  *   - sinks (float32 [Hq]) may be NULL; fa_bwd_varlen takes sinks and dsinks together or
- *     neither.  The workspace is fa_bwd_workspace_bytes(batch, Hq, Hkv, p->seqlen, D, W, S). */
+ *     neither.  The workspace is at least fa_bwd_workspace_bytes(batch, Hq, Hkv, p->seqlen, D, W, S). */
 int fa_fwd_varlen(const fa_fwd_params* p, const int32_t* cu_seqlens, int32_t total_rows, const float* sinks,
                   void* stream);
 int fa_bwd_varlen(const fa_bwd_params* p, const int32_t* cu_seqlens, int32_t total_rows, const float* sinks,
