@@ -155,7 +155,7 @@ def lib() -> ctypes.CDLL:
                 fn.restype = ctypes.c_int
             L.fa_bwd_workspace_bytes.argtypes = [ctypes.c_int32] * 7
             L.fa_bwd_workspace_bytes.restype = ctypes.c_size_t
-            L.fa_bwd_full_workspace_bytes.argtypes = [ctypes.c_int32] * 8
+            L.fa_bwd_full_workspace_bytes.argtypes = [ctypes.c_int32] * 9
             L.fa_bwd_full_workspace_bytes.restype = ctypes.c_size_t
             L.fa_check_fwd.argtypes = [ctypes.POINTER(FwdParams)]
             L.fa_check_fwd.restype = ctypes.c_int

@@ -257,11 +257,12 @@ def forward_fp8(q, k, v, window: int, sink: int, scale: float, descale=(1.0, 1.0
     return call.o, call.lse
 
 
-def workspace_bytes(B, Hq, Hkv, L, D, window, sink, device, total_rows: int = -1) -> int:
+def workspace_bytes(B, Hq, Hkv, L, D, window, sink, dtype, device, total_rows: int = -1) -> int:
     """The workspace with which the backward is fastest on `device` (fa_bwd_full_workspace_bytes);
     total_rows: the rows of a packed batch."""
     with _DeviceGuard(device):  # (it depends on the device's number of compute units)
-        return int(_lib.lib().fa_bwd_full_workspace_bytes(B, Hq, Hkv, L, D, _i32(window), _i32(sink), _i32(total_rows)))
+        return int(_lib.lib().fa_bwd_full_workspace_bytes(B, Hq, Hkv, L, D, _i32(window), _i32(sink),
+                                                          _DTYPES[dtype], _i32(total_rows)))
 
 
 class BwdCall:
@@ -279,7 +280,7 @@ class BwdCall:
         self.sinks = None if sinks is None else _sinks_ready(sinks, Hq, dev)
         self.dsinks = None if sinks is None else torch.empty(Hq, dtype=torch.float32, device=dev)
         self.dq, self.dk, self.dv = _out_like(q), _out_like(k), _out_like(v)
-        ws_bytes = workspace_bytes(B, Hq, Hkv, L, D, window, sink, dev)
+        ws_bytes = workspace_bytes(B, Hq, Hkv, L, D, window, sink, q.dtype, dev)
         self.ws = torch.empty((max(ws_bytes, 256),), dtype=torch.uint8, device=dev)
         self.inputs = (q, k, v, o, lse, do)
         self.device = dev
@@ -436,7 +437,7 @@ def backward_varlen(q, k, v, o, lse, do, cu_seqlens, max_seqlen: int, window: in
     dqv, dkv, dvv = (t.permute(1, 0, 2).unsqueeze(0) for t in (dq, dk, dv))
     sk = None if sinks is None else _sinks_ready(sinks, Hq, q.device)
     dsinks = None if sinks is None else torch.empty(Hq, dtype=torch.float32, device=q.device)
-    ws_bytes = workspace_bytes(B, Hq, Hkv, int(max_seqlen), D, window, sink, q.device, total)
+    ws_bytes = workspace_bytes(B, Hq, Hkv, int(max_seqlen), D, window, sink, q.dtype, q.device, total)
     ws = torch.empty((max(ws_bytes, 256),), dtype=torch.uint8, device=q.device)
     p = _lib.BwdParams()
     p.q, p.k, p.v, p.o, p.dout = qv.data_ptr(), kv.data_ptr(), vv.data_ptr(), ovw.data_ptr(), dov.data_ptr()

@@ -138,6 +138,24 @@ __device__ inline bool varlen_nth(const A& a, int p, int slots, int rows, int pe
   return false;
 }
 
+// Workgroup id -> piece, group and key block index of a split dK/dV grid (see bwd_dkdv_kernel): `streams`
+// = `ns` pieces x groups, each with one workgroup per key block.
+struct KvPiece {
+  int piece, group, p;
+};
+__device__ __forceinline__ KvPiece kv_piece(int id, int streams, int ns) {
+  int stream, p;
+  if (streams % 8 == 0) {  // XCD id % 8 owns streams / 8 streams
+    const int spx = streams / 8, pos = id / 8;
+    p = pos / spx;
+    stream = id % 8 * spx + pos % spx;
+  } else {
+    p = id / streams;
+    stream = id % streams;
+  }
+  return KvPiece{stream % ns, stream / ns, p};
+}
+
 // Element offset of row `row` of (batch b, head h) of a tensor with strides s[3] (a plain array
 // or one read through args_fresh()).
 template <typename S3>
@@ -193,8 +211,8 @@ hipError_t launch_bwd_dkdv(const Args& a, int dtype, int D, hipStream_t stream);
 bool dkdv4_eligible(const Args& a, int D, int cus);
 hipError_t launch_bwd_sink_logits(const Args& a, hipStream_t stream);  // after launch_bwd_dq
 hipError_t launch_varlen_tail(const TailArgs& t, hipStream_t stream);
-// float32 inputs (fa_f32.hip).  The dK/dV launch reads n_kblocks (32-key tiles), nsp (sink tiles
-// that may be split), n_chunks and chunk_rows (their chunk workgroups) and launches the fold.
+// float32 inputs (fa_f32.hip).  The dK/dV launch reads the same plan as launch_bwd_dkdv (key blocks,
+// pieces, sink blocks and their chunk workgroups) and launches the folds.
 hipError_t launch_fwd_f32(const Args& a, int D, hipStream_t stream);
 hipError_t launch_bwd_dq_f32(const Args& a, int D, hipStream_t stream);
 hipError_t launch_bwd_dkdv_f32(const Args& a, int D, hipStream_t stream);

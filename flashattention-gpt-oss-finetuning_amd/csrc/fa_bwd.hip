@@ -741,25 +741,6 @@ __host__ __device__ inline bool dkdv_folds_in_kernel(const Args& a, int D, bool 
 template <int D>
 constexpr int kPartCols = D < 32 ? 32 : D;
 
-// Workgroup id -> piece, group and key block index of the split dK/dV grid (see bwd_dkdv_kernel):
-// `streams` = pieces x groups, `per` key blocks each.
-struct KvPiece {
-  int piece, group, p;
-};
-__device__ __forceinline__ KvPiece kv_piece(int id, int streams, int ns, int per) {
-  int stream, p;
-  if (streams % 8 == 0) {  // XCD id % 8 owns streams / 8 streams
-    const int spx = streams / 8, pos = id / 8;
-    p = pos / spx;
-    stream = id % 8 * spx + pos % spx;
-  } else {
-    p = id / streams;
-    stream = id % streams;
-  }
-  (void)per;
-  return KvPiece{stream % ns, stream / ns, p};
-}
-
 // D = 16 keeps four waves per SIMD (at most 128 VGPRs), D = 64 with KVL three (168); the wider
 // head dims need more registers.
 //
@@ -806,7 +787,7 @@ __global__ __launch_bounds__(256, D == 16 ? 4 : KVL ? 3 : 1) void bwd_dkdv_kerne
     const int per = a.vl_kblocks ? a.vl_kblocks : a.n_kblocks;      // key blocks per stream
     const int streams = ns * a.Hkv * (a.vl_kblocks ? 1 : a.B);
     if (id < streams * per) {
-      const KvPiece t = kv_piece(id, streams, ns, per);
+      const KvPiece t = kv_piece(id, streams, ns);
       piece = t.piece;
       part_slot = (int64_t(t.group) * per + t.p) * ns + piece;
       if (a.vl_kblocks) {

@@ -124,9 +124,10 @@ size_t dq_sink_slot_bytes(int B, int Hq, int Hkv, int L, int D, const SinkPlan& 
   return sp.dq ? align256(size_t(dq_tiles(B, Hq, Hkv, L)) * 2 * sp.srows * D * sizeof(float)) : 0;
 }
 
-// float32 backward: 32-key tiles; the tiles holding sink keys whose rows extend past their window
-// (kv32_row_end in fa_f32.hip: min(L, 32 kt + 31 + max(W, 1))) split those rows into chunk
-// workgroups of kF32ChunkRows rows, with fp32 partials [B * Hkv][nsp][n_chunks + 1][dK, dV][32][D].
+// float32 backward: room for its sink-key partials, sized for 32-key tiles whose sink rows past the window
+// are cut into chunks of 256 rows, [B * Hkv][tiles][chunks + 1][dK, dV][32][D] fp32.  The kernel keeps
+// [B * Hkv][chunks + 1][dK, dV][S][D] for chunks of f32_chunk_rows rows laid out from its 64-key
+// blocks' window ends, which is never more.
 constexpr int kF32ChunkRows = 256;
 struct F32Plan {
   int n_kt, nsp, n_chunks;
@@ -140,6 +141,17 @@ F32Plan f32_plan(int L, int W, int S) {
   p.n_chunks = (S > 0 && row_end0 < L) ? (L - row_end0 + kF32ChunkRows - 1) / kF32ChunkRows : 0;
   p.nsp = p.n_chunks > 0 ? (S + 31) / 32 : 0;
   return p;
+}
+// Rows per sink-chunk workgroup of the float32 dK/dV kernel: 64, so that short workgroups even out the
+// end of the launch (c2's backward with chunks of 64 / 128 / 256 rows: 502 / 509 / 596 us), or as few
+// more as the room for partials needs.
+int f32_chunk_rows(int L, int W, int S) {
+  const F32Plan fp = f32_plan(L, W, S);
+  int rows = 64;
+  while (rows < kF32ChunkRows &&
+         int64_t(fa::kv_n_chunks(L, W, S, rows) + 1) * S > int64_t(fp.n_chunks + 1) * 32 * fp.nsp)
+    rows *= 2;
+  return rows;
 }
 size_t f32_partial_bytes(int B, int Hkv, int D, const F32Plan& fp) {
   return align256(size_t(B) * Hkv * fp.nsp * (fp.n_chunks + 1) * 2 * 32 * D * sizeof(float));
@@ -254,10 +266,13 @@ KvSteps kv_steps(double L, double W, double G) {
 // 434 / 298 / 302 / 321 / 386; L = 8192 1137 / 1125 / 1140 / 1198 / 1339; Hq = 8, Hkv = 1, L = 2048
 // 202 / 106 / 59 / 38 / 31; D = 128, Hq = 32, Hkv = 8, L = 2048 149 / 102 / 113 / 142 / 220; with a
 // window of 1024 at L = 4096 (equal workgroups) 143 / 154 / 162 / 177 / 245.
-int kv_split_pieces(int D, int G, int Hkv, double nseq, double L, double W, bool folds, int cus) {
-  const int i = D == 16 ? 0 : D == 32 ? 1 : D == 64 ? 2 : 3;
-  const double t_long[4] = {0.55, 0.58, 0.8, 1.15}, t_slot[4] = {1.3, 1.5, 1.14, 1.25};
-  const int per_cu[4] = {4, 4, 2, 1};  // resident workgroups
+// The float32 kernel (the last four of each table): L = 2048, Hq = 64, Hkv = 8, D = 64 by pieces 1 / 2 / 4 /
+// 8 / 16 1260 / 849 / 650 / 603 / 644; D = 128, Hq = 16, Hkv = 8 610 / 361 / 377 / 431 / 536.
+int kv_split_pieces(bool f32, int D, int G, int Hkv, double nseq, double L, double W, bool folds, int cus) {
+  const int i = (D == 16 ? 0 : D == 32 ? 1 : D == 64 ? 2 : 3) + (f32 ? 4 : 0);
+  const double t_long[8] = {0.55, 0.58, 0.8, 1.15, 2.9, 2.9, 4.9, 9.3};
+  const double t_slot[8] = {1.3, 1.5, 1.14, 1.25, 6.5, 6.5, 8.8, 9.6};
+  const int per_cu[8] = {4, 4, 2, 1, 4, 3, 2, 1};  // resident workgroups
   const KvSteps st = kv_steps(L, W, G);
   const double slot = t_slot[i] * st.total * nseq * Hkv / (double(cus) * per_cu[i]);
   const double mb = nseq * Hkv * std::ceil(L / fa::kKvKeys) * fa::kKvKeys * (D < 32 ? 32 : D) * 8 * 1e-6;  // per piece
@@ -289,27 +304,32 @@ int64_t kv_blocks(const fa::Args& a) {
 // Splits the dK/dV kernel (kv_split, kv_part) as far as the `spare` bytes of workspace at `ws` allow.
 // The rows of a packed batch are taken to be spread evenly over its sequences (the host does not
 // know their lengths).
-void plan_kv_split(fa::Args& a, int D, char* ws, size_t spare) {
+void plan_kv_split(fa::Args& a, int D, bool f32, char* ws, size_t spare) {
   a.kv_split = 1;
   const int cus = fa::device_cus();
-  if (fa::dkdv4_eligible(a, D, cus)) return;
+  if (!f32 && fa::dkdv4_eligible(a, D, cus)) return;
   const double rows = a.cu_seqlens ? std::min(double(a.L), std::max(1., double(a.total_rows) / a.B)) : double(a.L);
-  int ns = kv_split_pieces(D, a.G, a.Hkv, a.B, rows, a.W, a.sink_dq != 0, cus);
+  int ns = kv_split_pieces(f32, D, a.G, a.Hkv, a.B, rows, a.W, a.sink_dq != 0, cus);
   const int64_t blocks = kv_blocks(a);
   while (ns > 1 && (kv_part_bytes(D, blocks, ns) > spare || blocks * ns > (int64_t(1) << 24))) ns /= 2;
   a.kv_split = ns;
   a.kv_part = reinterpret_cast<float*>(ws);
 }
 
-// The kernel arguments that the 16-bit dK/dV kernel's plan reads.
-void set_kv_plan(fa::Args* a, int window, int sink) {
-  const SinkPlan sp = sink_plan(a->L, window, sink);
-  a->sink_dq = sp.dq;
+// The kernel arguments that describe the dK/dV kernel's key blocks and sink chunks.
+void set_kv_plan(fa::Args* a, bool f32) {
   a->n_kblocks = (a->L + fa::kKvKeys - 1) / fa::kKvKeys;
+  const SinkPlan sp = sink_plan(a->L, a->W, a->S);
   a->nsp = sp.nsp;
-  a->n_chunks = sp.n_chunks;
-  a->chunk_rows = kChunkRows;
-  a->srows = sp.srows;
+  if (f32) {
+    a->chunk_rows = f32_chunk_rows(a->L, a->W, a->S);
+    a->n_chunks = fa::kv_n_chunks(a->L, a->W, a->S, a->chunk_rows);
+  } else {
+    a->sink_dq = sp.dq;
+    a->n_chunks = sp.n_chunks;
+    a->chunk_rows = kChunkRows;
+    a->srows = sp.srows;
+  }
   a->n_chunk_wgs = a->B * a->Hkv * a->nsp * a->n_chunks;
 }
 
@@ -453,15 +473,16 @@ int run_fwd(const fa_fwd_params* p, const float* sinks, void* stream, const int3
   copy3(a.so_out, p->o_stride);
   copy3(a.slse, p->lse_stride);
   if (cu_seqlens) set_varlen(&a, cu_seqlens, total_rows);
-  if (p->dtype == FA_DTYPE_F32)
-    return fa::launch_fwd_f32(a, p->head_dim, static_cast<hipStream_t>(stream)) == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
   if (plan_fwd_slide(a, p->head_dim, p->dtype))
     return fa::launch_fwd_slide(a, p->dtype, static_cast<hipStream_t>(stream)) == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
+  const bool f32 = p->dtype == FA_DTYPE_F32;
   int hpw, wh, wq;
-  choose_qmajor(a.G, p->head_dim <= 64 ? 2 : 1, &hpw, &wh, &wq);
+  choose_qmajor(a.G, p->head_dim <= 64 && !f32 ? 2 : 1, &hpw, &wh, &wq);
   a.wh = wh;
   a.wq = wq;
   a.n_qtiles = (a.L + 32 * wq - 1) / (32 * wq);
+  if (f32)
+    return fa::launch_fwd_f32(a, p->head_dim, static_cast<hipStream_t>(stream)) == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
   const hipError_t e = fa::launch_fwd(a, p->dtype, p->head_dim, hpw, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
 }
@@ -573,17 +594,18 @@ size_t fa_bwd_workspace_bytes(int32_t batch, int32_t heads_q, int32_t heads_kv, 
 }
 
 size_t fa_bwd_full_workspace_bytes(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t seqlen, int32_t head_dim,
-                                   int32_t window, int32_t sink, int32_t total_rows) {
+                                   int32_t window, int32_t sink, int32_t dtype, int32_t total_rows) {
   const size_t need = fa_bwd_workspace_bytes(batch, heads_q, heads_kv, seqlen, head_dim, window, sink);
   if (need == 0) return 0;
+  const bool f32 = dtype == FA_DTYPE_F32;
   fa::Args a = base_args(batch, heads_q, heads_kv, seqlen, head_dim, window, sink, 1.f);
-  set_kv_plan(&a, window, sink);
+  set_kv_plan(&a, f32);
   if (total_rows >= 0) {
     a.cu_seqlens = &total_rows;  // (only whether there are offsets matters to the plan)
     a.total_rows = total_rows;
     a.vl_kblocks = vl_kblocks(a);
   }
-  plan_kv_split(a, head_dim, nullptr, SIZE_MAX);
+  plan_kv_split(a, head_dim, f32, nullptr, SIZE_MAX);
   return need + kv_part_bytes(head_dim, kv_blocks(a), a.kv_split);
 }
 
@@ -634,25 +656,16 @@ int prepare_bwd(const fa_bwd_params* p, void* workspace, size_t workspace_bytes,
   const size_t off_dsink = delta_bytes(a.B, a.Hq, a.L);
   a.dsink_part = reinterpret_cast<float*>(ws + off_dsink);
   a.partial = reinterpret_cast<float*>(ws + off_dsink + dsink_part_bytes(a.B, a.Hq, a.L));
-  if (p->dtype == FA_DTYPE_F32) {
-    const F32Plan fp = f32_plan(a.L, p->window, p->sink);
-    a.n_kblocks = fp.n_kt;
-    a.nsp = fp.nsp;
-    a.n_chunks = fp.n_chunks;
-    a.chunk_rows = kF32ChunkRows;
-    if (cu_seqlens) set_varlen(&a, cu_seqlens, total_rows);
-    *out = a;
-    return FA_OK;
-  }
-  set_kv_plan(&a, p->window, p->sink);
+  const bool f32 = p->dtype == FA_DTYPE_F32;
+  set_kv_plan(&a, f32);
   if (a.sink_dq)
-    a.dq_sink_part = a.partial + partial_bytes(a.B, a.Hkv, p->head_dim, sink_plan(a.L, p->window, p->sink)) / sizeof(float);
+    a.dq_sink_part = a.partial + partial_bytes(a.B, a.Hkv, p->head_dim, sink_plan(a.L, a.W, a.S)) / sizeof(float);
   if (cu_seqlens) {
     set_varlen(&a, cu_seqlens, total_rows);
     a.vl_kblocks = vl_kblocks(a);
   }
-  plan_slide(a, p->head_dim);
-  plan_kv_split(a, p->head_dim, ws + need, workspace_bytes - need);
+  if (!f32) plan_slide(a, p->head_dim);
+  plan_kv_split(a, p->head_dim, f32, ws + need, workspace_bytes - need);
   *out = a;
   return FA_OK;
 }

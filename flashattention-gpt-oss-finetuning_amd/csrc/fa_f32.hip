@@ -4,7 +4,7 @@
 // (flash_attention_gpt_oss.py:356-357: o = empty_like(q); benchmark_backward_speed.py:28-37:
 // dtype "fp32").  These kernels compute that case in float32 throughout: every product runs on
 // v_mfma_f32_32x32x2_f32 (exact fp32 products, fp32 sums), P and dS stay fp32, and q, k, v, o,
-// dq, dk, dv are fp32 tensors.  The mathematics, masks, visit order of key blocks, workspace row
+// dq, dk, dv are fp32 tensors.  The mathematics, masks, visit order of key tiles, workspace row
 // statistics and the sink-key partial sums follow the 16-bit kernels (fa_fwd.hip, fa_bwd.hip).
 //
 // The instruction: a wave64 multiplies a 32x2 A tile by a 2x32 B tile into a 32x32 fp32 C tile;
@@ -15,8 +15,21 @@
 //    head-dim index h D / 2 + t, so each lane reads one contiguous half row;
 //  * a C tile feeds the next product as its B operand unchanged: in step t the reduction index
 //    of lane half h is crow(t, h), which is register t of every lane.
-// Each workgroup is one wave: 32 query rows of one head (forward, dQ) or 32 keys of one KV head
-// (dK/dV).  Operands come straight from memory (L1/L2), no LDS.
+//
+// What bounds them: the instruction takes 64 cycles for 4096 operations (157 TFLOP/s over the
+// chip), so a 32x32 tile at D = 64 is 64 (forward), 96 (dQ) or 128 (dK/dV) of them, 4096-8192 cycles
+// against a few hundred for its elementwise work: the matrix cores, once a wave's operands are at hand.
+// So the tiles that the waves of a workgroup share (K and V, or a query head's Q and dO) come by
+// LDS DMA, one tile ahead, and every operand is read from LDS, where it costs a small share of
+// the matrix time; the waves' own rows stay in registers.  Against one wave per workgroup with
+// operands straight from memory, in us (B = 1, Hq = 64, Hkv = 8, D = 64): L = 4096, W = 128, S = 4
+// forward 240 -> 133, dQ 338 -> 205, dK/dV 1119 -> 299; L = 2048 full causal 1007 -> 334,
+// 1390 -> 489, 4862 -> 620 (105 TFLOP/s of allowed pairs).
+//
+// The head-dim order of a product whose A rows are head-dim indices (O^T, dQ^T, dV^T, dK^T) is free:
+// A row m of its C tile db (DB = D / 32 of them) stands for index DB m + db, so a lane reads the DB
+// operands of one tile row with one LDS read of DB consecutive floats, and holds 4 DB
+// consecutive outputs per four registers.
 #include "fa_args.h"
 #include "fa_common.h"
 
@@ -32,14 +45,18 @@ __device__ __forceinline__ f32x4 ld4f(const float* p) { return *reinterpret_cast
 __device__ __forceinline__ void st4f(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
 __device__ __forceinline__ float other_half(float x) { return __shfl_xor(x, 32); }
 
-// Key tiles of 32 that rows [q0, q0 + 32) of a sequence of L rows visit: the sink tiles [0, nsink)
+// 32-column C tiles of a head dim
+template <int D>
+constexpr int kDB = D >= 32 ? D / 32 : 1;
+
+// Key tiles of 32 that rows [q0, q0 + bm) of a sequence of L rows visit: the sink tiles [0, nsink)
 // (keys below S that lie before the window tiles) and the window tiles [ws, we).
 struct Plan32 {
   int nsink, ws, we;
 };
-__device__ __forceinline__ Plan32 plan32(int q0, int L, int W, int S) {
+__device__ __forceinline__ Plan32 plan32(int q0, int bm, int L, int W, int S) {
   Plan32 p;
-  const int q_end = min(q0 + 32, L);
+  const int q_end = min(q0 + bm, L);
   const int wlo = max(0, q0 - W + 1);  // first key in any row's window
   p.ws = wlo / 32;
   p.we = q_end > wlo ? (q_end - 1) / 32 + 1 : p.ws;
@@ -63,24 +80,134 @@ __device__ __forceinline__ void load_half_row(const float* base, int64_t stride,
   }
 }
 
+// ---- [32][D] fp32 tiles in LDS ------------------------------------------------------------------
+// Row-major without padding; 16-byte chunk j of row r is stored at chunk j ^ swz32(r), so that the
+// same chunk of 8 consecutive rows (a half-row read) lies in 8 different bank groups and a row
+// read across lanes still covers whole rows.
+template <int D>
+__device__ __forceinline__ int swz32(int r) {
+  return D >= 32 ? r & 7 : (r >> 1) & 3;
+}
+// chunk u of lane (r, h)'s half row: columns h D / 2 + 4u .. + 3 of row r
+template <int D>
+__device__ __forceinline__ f32x4 tile_half(const float* t, int r, int h, int u) {
+  return ld4f(t + r * D + 4 * ((h * (D / 8) + u) ^ swz32<D>(r)));
+}
+// columns DB c .. DB c + DB - 1 of row r (D = 16 has 16 columns: lanes past them repeat the others)
+template <int D>
+__device__ __forceinline__ void tile_cols(const float* t, int r, int c, float (&out)[kDB<D>]) {
+  const int col = D >= 32 ? kDB<D> * c : c & 15;
+  const float* p = t + r * D + 4 * ((col >> 2) ^ swz32<D>(r)) + (col & 3);
+  if constexpr (kDB<D> == 4) {
+    const f32x4 x = ld4f(p);
+#pragma unroll
+    for (int db = 0; db < 4; ++db) out[db] = x[db];
+  } else if constexpr (kDB<D> == 2) {
+    const f32x2 x = *reinterpret_cast<const f32x2*>(p);
+    out[0] = x[0];
+    out[1] = x[1];
+  } else {
+    out[0] = *p;
+  }
+}
+// DMA instruction p (of D / 8: 1 KiB each) of the tile at rows [row0, row0 + 32) of a slice: lane l
+// loads the chunk that the swizzle places at 16-byte position 64 p + l; rows past the slice read as 0
+template <int D>
+__device__ __forceinline__ void dma_tile(rsrc_t rs, float* tile, int row0, int64_t stride, int p) {
+  const int pos = 64 * p + int(threadIdx.x & 63), row = pos / (D / 4), chunk = (pos % (D / 4)) ^ swz32<D>(row);
+  buf_dma16(rs, reinterpret_cast<uint16_t*>(tile + 256 * p), uint32_t((int64_t(row0 + row) * stride + 4 * chunk) * 4));
+}
+__device__ __forceinline__ rsrc_t slice_rsrc(const float* base, int L, int64_t stride, int D) {
+  return make_rsrc(base, span_bytes(L, stride, D, 4));
+}
+
+// Stores a 32-row output: this lane's row at `row`, C tiles acc (A row m of tile db = column DB m +
+// db) times mul.
+template <int D>
+__device__ __forceinline__ void store_cols(float* row, const f32x16 (&acc)[kDB<D>], int h, float mul) {
+  constexpr int DB = kDB<D>;
+#pragma unroll
+  for (int j = 0; j < (D >= 32 ? 4 : 2); ++j) {
+    float v[4 * DB];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int db = 0; db < DB; ++db) v[DB * i + db] = acc[db][4 * j + i] * mul;
+#pragma unroll
+    for (int x = 0; x < DB; ++x)
+      st4f(row + DB * (8 * j + 4 * h) + 4 * x, f32x4{v[4 * x], v[4 * x + 1], v[4 * x + 2], v[4 * x + 3]});
+  }
+}
+
+// Workgroup -> rows and heads of the query-major kernels: wq x wh waves of 32 rows x 1 head of one KV
+// group.  An XCD owns whole (batch, head group)s where their number allows (their tiles share K/V
+// rows in its L2), takes their row tiles together and the last rows, which see the most keys, first.
+struct QTile {
+  int b, kvh, hq, q0, qw;
+};
+__device__ __forceinline__ QTile q_tile(const Args& a) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int groups = a.B * (a.Hq / a.wh), id = blockIdx.x;
+  int grp, qt;
+  if (groups % 8 == 0) {
+    const int gpx = groups / 8, pos = id / 8;
+    grp = id % 8 * gpx + pos % gpx;
+    qt = pos / gpx;
+  } else {
+    grp = id % groups;
+    qt = id / groups;
+  }
+  const int gpk = a.G / a.wh;  // head groups per KV head
+  QTile t;
+  t.kvh = grp / gpk / a.B;
+  t.b = grp / gpk % a.B;
+  t.hq = t.kvh * a.G + grp % gpk * a.wh + wave / a.wq;
+  t.q0 = (a.n_qtiles - 1 - qt) * 32 * a.wq;
+  t.qw = t.q0 + 32 * (wave % a.wq);
+  return t;
+}
+
+// The K and V tiles of a query-major workgroup: two LDS buffers of [K, V] tiles, wave w issuing DMA
+// instructions [w D / 16, (w + 1) D / 16) of the D / 4.
+template <int D>
+struct KvTiles {
+  static constexpr int kTile = 32 * D, kBuf = 2 * kTile;
+  rsrc_t rk, rv;
+  int64_t sk, sv;
+  float* lds;
+  __device__ __forceinline__ void load(int buf, int ks0) const {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+    for (int n = 0; n < D / 16; ++n) {
+      const int i = wave * (D / 16) + n;
+      if (i < D / 8) dma_tile<D>(rk, lds + buf * kBuf, ks0, sk, i);
+      else dma_tile<D>(rv, lds + buf * kBuf + kTile, ks0, sv, i - D / 8);
+    }
+  }
+};
+
 // ---------------------------------------------------------------------------------------------
 // Forward: O = softmax(mask(s)) V with s = scale q.k, online softmax in the log2 domain (q is
-// pre-multiplied by scale * log2(e)).  Grid (row tiles, Hq, B), one wave each.
+// pre-multiplied by scale * log2(e)).
 // ---------------------------------------------------------------------------------------------
 template <int D>
-__global__ __launch_bounds__(64) void fwd32_kernel(const Args a) {
+__global__ __launch_bounds__(256, 2) void fwd32_kernel(const Args a) {
   constexpr int HD = D / 2;
-  constexpr int DB = D >= 32 ? D / 32 : 1;
-  const int lane = threadIdx.x, r = lane & 31, h = lane >> 5;
-  const int hq = blockIdx.y, b = blockIdx.z;
-  const Seq sq = seq_of(a, b);
-  const int L = sq.L, q0 = 32 * int(blockIdx.x);
-  if (q0 >= L) return;
-  const int kvh = hq / a.G, W = a.W, S = a.S;
+  constexpr int DB = kDB<D>;
+  __shared__ __attribute__((aligned(16))) float lds[2 * KvTiles<D>::kBuf];
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  const QTile t = q_tile(a);
+  const Seq sq = seq_of(a, t.b);
+  const int L = sq.L, W = a.W, S = a.S, hq = t.hq, b = t.b, qw = t.qw;
+  if (t.q0 >= L) return;
   const float* Q = static_cast<const float*>(a.q) + slice_off(a.sq, b, hq, sq.row);
-  const float* K = static_cast<const float*>(a.k) + slice_off(a.sk, b, kvh, sq.row);
-  const float* V = static_cast<const float*>(a.v) + slice_off(a.sv, b, kvh, sq.row);
-  const int q = q0 + r;
+  const float* K = static_cast<const float*>(a.k) + slice_off(a.sk, b, t.kvh, sq.row);
+  const float* V = static_cast<const float*>(a.v) + slice_off(a.sv, b, t.kvh, sq.row);
+  const KvTiles<D> kv{slice_rsrc(K, L, a.sk[2], D), slice_rsrc(V, L, a.sv[2], D), a.sk[2], a.sv[2], lds};
+  const Plan32 pl = plan32(t.q0, 32 * a.wq, L, W, S);
+  const int nt = pl.nsink + (pl.we - pl.ws);
+  if (nt > 0) kv.load(0, 32 * plan32_tile(pl, 0));
+  const int q = qw + r;
   float qf[HD];
   load_half_row<D>(Q, a.sq[2], q, L, h, a.scale * kLog2e, qf);
 
@@ -88,46 +215,55 @@ __global__ __launch_bounds__(64) void fwd32_kernel(const Args a) {
   f32x16 acc[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) acc[db] = f32x16{};
-  const Plan32 pl = plan32(q0, L, W, S);
-  const int nt = pl.nsink + (pl.we - pl.ws);
+  wait_vm_lgkm0_barrier<0>();
   for (int it = 0; it < nt; ++it) {
+    // the other buffer was last read before the barrier that ended the tile before
+    if (it + 1 < nt) kv.load((it + 1) & 1, 32 * plan32_tile(pl, it + 1));
     const int ks0 = 32 * plan32_tile(pl, it);
-    // S^T = K Q^T (keys x queries): lane (r, h) supplies K[ks0 + r][h HD + t]
-    float kf[HD];
-    load_half_row<D>(K, a.sk[2], ks0 + r, L, h, 1.f, kf);
-    f32x16 s = f32x16{};
+    if (qw < L && wave_needs(ks0, qw, L, W, S)) {
+      const float* Kt = lds + (it & 1) * KvTiles<D>::kBuf;
+      const float* Vt = Kt + KvTiles<D>::kTile;
+      // S^T = K Q^T (keys x queries): lane (r, h) supplies K[ks0 + r][h HD + t]
+      f32x16 s = f32x16{};
 #pragma unroll
-    for (int t = 0; t < HD; ++t) s = mfma32(kf[t], qf[t], s);
-    float mx = kNegInf;
+      for (int u = 0; u < D / 8; ++u) {
+        const f32x4 kf = tile_half<D>(Kt, r, h, u);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      s[i] = allowed32(q, ks0 + crow(i, h), W, S) ? s[i] : kNegInf;
-      mx = fmaxf(mx, s[i]);
-    }
-    mx = fmaxf(mx, other_half(mx));
-    const float mnew = fmaxf(m, mx);
-    const float alpha = mnew == kNegInf ? 1.f : exp2f(m - mnew);
-    const float ms = mnew == kNegInf ? 0.f : mnew;
-    m = mnew;
-    lsum *= alpha;
-    float p[16];
+        for (int j = 0; j < 4; ++j) s = mfma32(kf[j], qf[4 * u + j], s);
+      }
+      if (!tile_full(ks0, qw, W, S)) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      p[i] = exp2f(s[i] - ms);
-      lsum += p[i];
-    }
-    // O^T += V^T P^T: lane (r, h) supplies V[ks0 + crow(t, h)][32 db + r]
+        for (int i = 0; i < 16; ++i) s[i] = allowed32(q, ks0 + crow(i, h), W, S) ? s[i] : kNegInf;
+      }
+      float mx = s[0];
 #pragma unroll
-    for (int db = 0; db < DB; ++db) {
-      acc[db] *= alpha;
-      const int d = 32 * db + r;
+      for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+      mx = max_halves(mx);
+      if (wave_any(mx > m)) {  // some row's maximum moves (otherwise the factor is 1)
+        const float mnew = fmaxf(m, mx);
+        const float alpha = mnew == kNegInf ? 1.f : exp2f(m - mnew);
+        m = mnew;
+        lsum *= alpha;
 #pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        const int kk = ks0 + crow(t, h);
-        const float va = (d < D && kk < L) ? V[int64_t(kk) * a.sv[2] + d] : 0.f;
-        acc[db] = mfma32(va, p[t], acc[db]);
+        for (int db = 0; db < DB; ++db) acc[db] *= alpha;
+      }
+      const float ms = m == kNegInf ? 0.f : m;
+      float p[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        p[i] = exp2f(s[i] - ms);
+        lsum += p[i];
+      }
+      // O^T += V^T P^T: lane (r, h) supplies V[ks0 + crow(t, h)][DB r + db]
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        float va[DB];
+        tile_cols<D>(Vt, crow(i, h), r, va);
+#pragma unroll
+        for (int db = 0; db < DB; ++db) acc[db] = mfma32(va[db], p[i], acc[db]);
       }
     }
+    wait_vm_lgkm0_barrier<0>();
   }
   float lt = lsum + other_half(lsum);
   float rs = 1.f;
@@ -140,15 +276,7 @@ __global__ __launch_bounds__(64) void fwd32_kernel(const Args a) {
   }
   if (q >= L) return;
   const float inv = lt > 0.f ? rs / lt : 0.f;
-  float* O = static_cast<float*>(a.o_out) + slice_off(a.so_out, b, hq, sq.row + q);
-#pragma unroll
-  for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int d = 32 * db + 8 * j + 4 * h;
-      if (d < D) st4f(O + d, f32x4{acc[db][4 * j] * inv, acc[db][4 * j + 1] * inv, acc[db][4 * j + 2] * inv,
-                                   acc[db][4 * j + 3] * inv});
-    }
+  store_cols<D>(static_cast<float*>(a.o_out) + slice_off(a.so_out, b, hq, sq.row + q), acc, h, inv);
   if (h == 0) a.lse_out[slice_off(a.slse, b, hq, sq.row + q)] = (m + log2f(lt)) * kLn2;
 }
 
@@ -156,143 +284,205 @@ __global__ __launch_bounds__(64) void fwd32_kernel(const Args a) {
 // dQ: delta = rowsum(dO o O), P = exp2(s - lse2), dS = P (dP - delta), dQ = scale dS K.  Also
 // stores the row statistics the dK/dV kernel reads (lse * log2(e), -delta per 32-row block, the
 // layout of the 16-bit backward) and, with learned sinks, the per-block partials of their
-// gradient.  Grid (row tiles, Hq, B), one wave each.
+// gradient.
 // ---------------------------------------------------------------------------------------------
 template <int D>
-__global__ __launch_bounds__(64) void dq32_kernel(const Args a) {
+__global__ __launch_bounds__(256, D == 128 ? 1 : 2) void dq32_kernel(const Args a) {
   constexpr int HD = D / 2;
-  constexpr int DB = D >= 32 ? D / 32 : 1;
-  const int lane = threadIdx.x, r = lane & 31, h = lane >> 5;
-  const int hq = blockIdx.y, b = blockIdx.z;
-  const Seq sq = seq_of(a, b);
-  const int L = sq.L, q0 = 32 * int(blockIdx.x);
-  if (q0 >= L) return;
-  const int kvh = hq / a.G, W = a.W, S = a.S;
+  constexpr int DB = kDB<D>;
+  __shared__ __attribute__((aligned(16))) float lds[2 * KvTiles<D>::kBuf];
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  const QTile t = q_tile(a);
+  const Seq sq = seq_of(a, t.b);
+  const int L = sq.L, W = a.W, S = a.S, hq = t.hq, b = t.b, qw = t.qw;
+  if (t.q0 >= L) return;
   const float* Q = static_cast<const float*>(a.q) + slice_off(a.sq, b, hq, sq.row);
-  const float* K = static_cast<const float*>(a.k) + slice_off(a.sk, b, kvh, sq.row);
-  const float* V = static_cast<const float*>(a.v) + slice_off(a.sv, b, kvh, sq.row);
+  const float* K = static_cast<const float*>(a.k) + slice_off(a.sk, b, t.kvh, sq.row);
+  const float* V = static_cast<const float*>(a.v) + slice_off(a.sv, b, t.kvh, sq.row);
   const float* O = static_cast<const float*>(a.o) + slice_off(a.so, b, hq, sq.row);
   const float* dO = static_cast<const float*>(a.dout) + slice_off(a.sdo, b, hq, sq.row);
-  const int q = q0 + r;
-  float qf[HD], dof[HD], of[HD];
+  const KvTiles<D> kv{slice_rsrc(K, L, a.sk[2], D), slice_rsrc(V, L, a.sv[2], D), a.sk[2], a.sv[2], lds};
+  const Plan32 pl = plan32(t.q0, 32 * a.wq, L, W, S);
+  const int nt = pl.nsink + (pl.we - pl.ws);
+  if (nt > 0) kv.load(0, 32 * plan32_tile(pl, 0));
+  const int q = qw + r;
+  float qf[HD], dof[HD];
   load_half_row<D>(Q, a.sq[2], q, L, h, a.scale * kLog2e, qf);
   load_half_row<D>(dO, a.sdo[2], q, L, h, 1.f, dof);
-  load_half_row<D>(O, a.so[2], q, L, h, 1.f, of);
   float dsum = 0.f;
+  {
+    float of[HD];
+    load_half_row<D>(O, a.so[2], q, L, h, 1.f, of);
 #pragma unroll
-  for (int t = 0; t < HD; ++t) dsum = fmaf(dof[t], of[t], dsum);
+    for (int i = 0; i < HD; ++i) dsum = fmaf(dof[i], of[i], dsum);
+  }
   const float delta = dsum + other_half(dsum);
   const float lse2 = q < L ? a.lse[slice_off(a.slse, b, hq, sq.row + q)] * kLog2e : __builtin_inff();
-  if (h == 0) {
-    float* st = a.delta + ((int64_t(b) * a.Hq + hq) * (a.Lp / 32) + q0 / 32) * 64;
-    st[r] = lse2;
-    st[32 + r] = -delta;
-  }
-  if (a.sink_logits) {
-    float v = (q < L && h == 0) ? exp2f(a.sink_logits[hq] * kLog2e - lse2) * delta : 0.f;
+  if (qw < L) {
+    const int64_t blk = (int64_t(b) * a.Hq + hq) * (a.Lp / 32) + qw / 32;
+    if (h == 0) {
+      float* st = a.delta + blk * 64;
+      st[r] = lse2;
+      st[32 + r] = -delta;
+    }
+    if (a.sink_logits) {
+      float v = (q < L && h == 0) ? exp2f(a.sink_logits[hq] * kLog2e - lse2) * delta : 0.f;
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-    if (lane == 0) a.dsink_part[(int64_t(b) * a.Hq + hq) * (a.Lp / 32) + q0 / 32] = -v;
+      for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+      if (lane == 0) a.dsink_part[blk] = -v;
+    }
   }
 
   f32x16 acc[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) acc[db] = f32x16{};
-  const Plan32 pl = plan32(q0, L, W, S);
-  const int nt = pl.nsink + (pl.we - pl.ws);
+  wait_vm_lgkm0_barrier<0>();
   for (int it = 0; it < nt; ++it) {
+    if (it + 1 < nt) kv.load((it + 1) & 1, 32 * plan32_tile(pl, it + 1));
     const int ks0 = 32 * plan32_tile(pl, it);
-    float kf[HD], vf[HD];
-    load_half_row<D>(K, a.sk[2], ks0 + r, L, h, 1.f, kf);
-    load_half_row<D>(V, a.sv[2], ks0 + r, L, h, 1.f, vf);
-    // S^T = K Q^T and dP^T - delta = V dO^T - delta (keys x queries)
-    f32x16 s = f32x16{}, dp;
+    if (qw < L && wave_needs(ks0, qw, L, W, S)) {
+      const float* Kt = lds + (it & 1) * KvTiles<D>::kBuf;
+      const float* Vt = Kt + KvTiles<D>::kTile;
+      // S^T = K Q^T and dP^T - delta = V dO^T - delta (keys x queries)
+      f32x16 s = f32x16{}, dp;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) dp[i] = -delta;
+      for (int i = 0; i < 16; ++i) dp[i] = -delta;
 #pragma unroll
-    for (int t = 0; t < HD; ++t) {
-      s = mfma32(kf[t], qf[t], s);
-      dp = mfma32(vf[t], dof[t], dp);
-    }
-    float ds[16];
+      for (int u = 0; u < D / 8; ++u) {
+        const f32x4 kf = tile_half<D>(Kt, r, h, u), vf = tile_half<D>(Vt, r, h, u);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float p = allowed32(q, ks0 + crow(i, h), W, S) ? exp2f(s[i] - lse2) : 0.f;
-      ds[i] = p * dp[i];
-    }
-    // dQ^T += K^T dS^T: lane (r, h) supplies K[ks0 + crow(t, h)][32 db + r]
+        for (int j = 0; j < 4; ++j) {
+          s = mfma32(kf[j], qf[4 * u + j], s);
+          dp = mfma32(vf[j], dof[4 * u + j], dp);
+        }
+      }
+      const bool full = tile_full(ks0, qw, W, S);
+      float ds[16];
 #pragma unroll
-    for (int db = 0; db < DB; ++db) {
-      const int d = 32 * db + r;
+      for (int i = 0; i < 16; ++i) {
+        float p = exp2f(s[i] - lse2);
+        if (!full) p = allowed32(q, ks0 + crow(i, h), W, S) ? p : 0.f;
+        ds[i] = p * dp[i];
+      }
+      // dQ^T += K^T dS^T: lane (r, h) supplies K[ks0 + crow(t, h)][DB r + db]
 #pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        const int kk = ks0 + crow(t, h);
-        const float ka = (d < D && kk < L) ? K[int64_t(kk) * a.sk[2] + d] : 0.f;
-        acc[db] = mfma32(ka, ds[t], acc[db]);
+      for (int i = 0; i < 16; ++i) {
+        float ka[DB];
+        tile_cols<D>(Kt, crow(i, h), r, ka);
+#pragma unroll
+        for (int db = 0; db < DB; ++db) acc[db] = mfma32(ka[db], ds[i], acc[db]);
       }
     }
+    wait_vm_lgkm0_barrier<0>();
   }
   if (q >= L) return;
-  float* dQ = static_cast<float*>(a.dq) + slice_off(a.sdq, b, hq, sq.row + q);
-  const float sc = a.scale;
-#pragma unroll
-  for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int d = 32 * db + 8 * j + 4 * h;
-      if (d < D) st4f(dQ + d, f32x4{acc[db][4 * j] * sc, acc[db][4 * j + 1] * sc, acc[db][4 * j + 2] * sc,
-                                    acc[db][4 * j + 3] * sc});
-    }
+  store_cols<D>(static_cast<float*>(a.dq) + slice_off(a.sdq, b, hq, sq.row + q), acc, h, a.scale);
 }
 
-// Rows a key tile's regular workgroup covers: [ks0, kv32_row_end) -- every row whose window
-// reaches a key of the tile (and the tile's own 32 rows, for its sink keys).  Sink keys are also
-// seen by every later row; those rows go to chunk workgroups of kF32ChunkRows rows.
-__device__ __forceinline__ int kv32_row_end(int ks0, int L, int W) { return min(L, ks0 + 31 + max(W, 1)); }
-
 // ---------------------------------------------------------------------------------------------
-// dK / dV: a wave owns 32 keys of one KV head and sweeps the (query head, 32-row block) items
-// that can see them: dV^T += dO^T P, dK^T += Q^T dS (keys as the C columns).  Grid (items, Hkv,
-// B): blockIdx.x < n_kblocks is key tile x with its window rows; the rest are chunk workgroups,
-// (sink tile st, chunk c) = ((x - n_kblocks) % nsp, (x - n_kblocks) / nsp), with the rows past
-// the window of sink tile st.  Sink tiles write fp32 partials to the workspace (slot 0: the
-// regular rows, slot c + 1: chunk c); fold32_kernel adds them.
+// dK / dV: a workgroup owns 64 keys of one KV head; wave (kh, hh) owns the 32-key half kh and takes
+// item 2s + hh of step s, an item being a (query head, 32-row block) that can see the keys: dV^T +=
+// dO^T P, dK^T += Q^T dS (keys as the C columns).  A step's two items (Q and dO tiles and row
+// statistics) are staged in LDS by DMA, one step ahead.  As in bwd_dkdv_kernel, a key block's steps
+// can be cut into kv_split pieces, one workgroup each, and the rows past the window of a block with
+// sink keys (block < nsp) go to chunk workgroups of chunk_rows rows; those and the block's own
+// workgroup write fp32 sums of its sink rows, [slot][dK, dV][S][D] per (batch, KV head), slot c for
+// chunk c and n_chunks for the block's own rows, and fold32_kernel adds them.
+// A chunk workgroup whose sink keys all lie in half 0 has its two waves of an item both take half 0
+// and half of the head-dim columns each (kh is then the column half).
 // ---------------------------------------------------------------------------------------------
 template <int D>
-__global__ __launch_bounds__(64) void dkdv32_kernel(const Args a) {
+constexpr int kDkdv32Slot = 2 * 32 * D + 64;  // floats of an item: Q tile, dO tile, lse2[32], -delta[32]
+
+template <int D>
+__global__ __launch_bounds__(256, D == 128 ? 1 : 2) void dkdv32_kernel(const Args a) {
   constexpr int HD = D / 2;
-  constexpr int DB = D >= 32 ? D / 32 : 1;
-  const int lane = threadIdx.x, r = lane & 31, h = lane >> 5;
-  const int kvh = blockIdx.y, b = blockIdx.z;
+  constexpr int DB = kDB<D>;
+  constexpr int SLOT = kDkdv32Slot<D>, STAGE = 2 * SLOT;
+  static_assert(2 * STAGE >= 2 * 2 * DB * 16 * 64, "the item slots' sums fit the stages");
+  __shared__ __attribute__((aligned(16))) float lds[2 * STAGE];
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kh = wave & 1, hh = wave >> 1;
+  const int W = a.W, S = a.S, G = a.G, ns = a.kv_split;
+  const int per = a.vl_kblocks ? a.vl_kblocks : a.n_kblocks;
+  const int streams = ns * a.Hkv * (a.vl_kblocks ? 1 : a.B);
+  const int id = blockIdx.x;
+  int kvh, b, kblk, piece = 0, chunk = -1;
+  int64_t part_slot = 0;
+  if (id < streams * per) {
+    const KvPiece t = kv_piece(id, streams, ns);
+    piece = t.piece;
+    part_slot = (int64_t(t.group) * per + t.p) * ns + piece;
+    if (a.vl_kblocks) {
+      kvh = t.group;
+      if (!varlen_nth(a, t.p, per, kKvKeys, 1, b, kblk)) return;
+    } else {
+      kvh = t.group / a.B;
+      b = t.group % a.B;
+      kblk = t.p;
+    }
+  } else {
+    const int n_cw = a.nsp * a.n_chunks, c = id - streams * per;
+    kvh = c / (a.B * n_cw);
+    b = c / n_cw % a.B;
+    kblk = c % n_cw % a.nsp;
+    chunk = c % n_cw / a.nsp;
+  }
   const Seq sq = seq_of(a, b);
-  const int L = sq.L, W = a.W, S = a.S, G = a.G;
-  int kt, chunk = -1;
-  if (int(blockIdx.x) < a.n_kblocks) {
-    kt = blockIdx.x;
-  } else {
-    const int x = blockIdx.x - a.n_kblocks;
-    kt = x % a.nsp;
-    chunk = x / a.nsp;
-  }
-  const int ks0 = 32 * kt;
-  if (ks0 >= L) return;
-  const int row_end = kv32_row_end(ks0, L, W);
-  const bool split = ks0 < S && row_end < L && kt < a.nsp;  // a sink tile with rows past its window
+  const int L = sq.L;
+  if (kKvKeys * kblk >= L) return;
+  const bool is_chunk = chunk >= 0, partial_block = kblk < a.nsp;
   int lo, hi;
-  if (chunk < 0) {
-    lo = ks0;
-    hi = row_end;
+  if (is_chunk) {
+    lo = kv_chunk_lo(kblk, chunk, a.chunk_rows, L, W);
+    hi = kv_chunk_hi(kblk, chunk, a.chunk_rows, L, W);
+    if (lo >= hi) return;  // (the fold reads no slot of it)
   } else {
-    if (!split) return;  // (this tile's rows all lie in its window: no chunk rows)
-    lo = row_end + chunk * a.chunk_rows;
-    hi = min(L, lo + a.chunk_rows);
+    lo = kKvKeys * kblk;
+    hi = kv_window_end(kblk, L, W);  // > lo
   }
+  const bool col_split = DB >= 2 && is_chunk && S <= kKvKeys * kblk + 32;
+  const int ks0 = kKvKeys * kblk + (col_split ? 0 : 32 * kh);  // this wave's keys
   const int key = ks0 + r;
+  const bool wave_on = ks0 < L && (!is_chunk || ks0 < S);
+  const int wlo = is_chunk ? lo : max(lo, ks0);
+
+  // the steps [s_lo, s_hi) of this workgroup over the items (g, qb), qb fastest
+  const int qb_lo = lo / 32, n_qb = (hi + 31) / 32 - qb_lo;
+  const int n_items = G * n_qb, all_steps = (n_items + 1) / 2;
+  int s_lo = 0, s_hi = all_steps;
+  if (!is_chunk) {
+    s_lo = int(int64_t(all_steps) * piece / ns);
+    s_hi = int(int64_t(all_steps) * (piece + 1) / ns);
+  }
+
+  // staging: wave w loads tile w of a step (item slot w / 2, Q or dO) and slot w % 2's statistics (waves
+  // w and w + 2 the same bytes to the same place)
+  const int t_slot = wave >> 1, t_do = wave & 1;
+  const int64_t t_rs = t_do ? a.sdo[2] : a.sq[2], t_hs = t_do ? a.sdo[1] : a.sq[1];
+  const float* tensor = t_do ? static_cast<const float*>(a.dout) + slice_off(a.sdo, b, kvh * G, sq.row)
+                             : static_cast<const float*>(a.q) + slice_off(a.sq, b, kvh * G, sq.row);
+  const int nblk = a.Lp / 32;
+  const float* stats = a.delta + (int64_t(b) * a.Hq + int64_t(kvh) * G) * nblk * 64;
+  auto issue = [&](int step) {
+    float* st = lds + (step & 1) * STAGE;
+    const int i = min(2 * step + t_slot, n_items - 1);  // (past the last item: loaded, not used)
+    const int g = i / n_qb, row0 = 32 * (qb_lo + i % n_qb);
+    const rsrc_t rs = slice_rsrc(tensor + g * t_hs, L, t_rs, D);
+#pragma unroll
+    for (int p = 0; p < D / 8; ++p) dma_tile<D>(rs, st + t_slot * SLOT + t_do * 32 * D, row0, t_rs, p);
+    const int i2 = min(2 * step + (wave & 1), n_items - 1);
+    const int blk = i2 / n_qb * nblk + qb_lo + i2 % n_qb;
+    buf_dma4(make_rsrc(stats + int64_t(blk) * 64, 256), reinterpret_cast<uint16_t*>(st + (wave & 1) * SLOT + 64 * D), 4u * lane);
+  };
+  if (s_lo < s_hi) issue(s_lo);
+
   const float c2 = a.scale * kLog2e;
   const float* K = static_cast<const float*>(a.k) + slice_off(a.sk, b, kvh, sq.row);
   const float* V = static_cast<const float*>(a.v) + slice_off(a.sv, b, kvh, sq.row);
   float kf[HD], vf[HD];
-  load_half_row<D>(K, a.sk[2], key, L, h, 1.f, kf);
+  load_half_row<D>(K, a.sk[2], key, L, h, c2, kf);
   load_half_row<D>(V, a.sv[2], key, L, h, 1.f, vf);
   f32x16 dk[DB], dv[DB];
 #pragma unroll
@@ -300,159 +490,263 @@ __global__ __launch_bounds__(64) void dkdv32_kernel(const Args a) {
     dk[db] = f32x16{};
     dv[db] = f32x16{};
   }
-  for (int g = 0; g < G && lo < hi; ++g) {
-    const int hq = kvh * G + g;
-    const float* Q = static_cast<const float*>(a.q) + slice_off(a.sq, b, hq, sq.row);
-    const float* dO = static_cast<const float*>(a.dout) + slice_off(a.sdo, b, hq, sq.row);
-    const float* stat = a.delta + (int64_t(b) * a.Hq + hq) * (a.Lp / 32) * 64;
-    for (int qr0 = lo / 32 * 32; qr0 < hi; qr0 += 32) {
-      // S = Q K^T and dP - delta = dO V^T - delta (queries x keys): lane (r, h) supplies row
-      // qr0 + r of Q (times scale log2 e) and of dO
-      float qa[HD], da[HD];
-      load_half_row<D>(Q, a.sq[2], qr0 + r, L, h, c2, qa);
-      load_half_row<D>(dO, a.sdo[2], qr0 + r, L, h, 1.f, da);
-      const float* st = stat + (qr0 / 32) * 64;
-      float l2[16];
-      f32x16 s = f32x16{}, dp;
+  // the mask as one unsigned compare, row - mref < lim (see bwd_dkdv_kernel)
+  unsigned lim;
+  if (is_chunk) lim = key < S ? unsigned(hi - lo) : 0u;
+  else lim = key < S ? (partial_block ? unsigned(max(hi - key, 0)) : 0x80000000u) : unsigned(W);
+  const int mref = is_chunk ? lo : key;
+
+  for (int s = s_lo; s < s_hi; ++s) {
+    wait_vm_lgkm0_barrier<0>();  // step s has landed, and nobody reads the other stage any more
+    if (s + 1 < s_hi) issue(s + 1);
+    const int i = 2 * s + hh;
+    const int qr0 = 32 * (qb_lo + i % n_qb);
+    if (!(wave_on && i < n_items && qr0 + 32 > wlo && qr0 < hi && kv_half_needs(qr0, ks0, L, W, S))) continue;
+    const float* Qt = lds + (s & 1) * STAGE + hh * SLOT;
+    const float* Dt = Qt + 32 * D;
+    const float* st = Qt + 64 * D;
+    // S = Q K^T and dP - delta = dO V^T - delta (queries x keys): lane (r, h) supplies rows qr0 + r
+    f32x16 sc = f32x16{}, dp;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 nv = ld4f(st + 32 + 8 * j + 4 * h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dp[4 * j + e] = nv[e];
+    }
+#pragma unroll
+    for (int u = 0; u < D / 8; ++u) {
+      const f32x4 qa = tile_half<D>(Qt, r, h, u), da = tile_half<D>(Dt, r, h, u);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const f32x4 lv = ld4f(st + 8 * j + 4 * h), nv = ld4f(st + 32 + 8 * j + 4 * h);
+        sc = mfma32(qa[j], kf[4 * u + j], sc);
+        dp = mfma32(da[j], vf[4 * u + j], dp);
+      }
+    }
+    const bool full = !is_chunk && qr0 >= wlo && qr0 + 32 <= hi && tile_full(ks0, qr0, W, S);
+    const int m0 = qr0 + 4 * h - mref;
+    float p[16], ds[16];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          l2[4 * j + i] = lv[i];
-          dp[4 * j + i] = nv[i];
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 l4 = ld4f(st + 8 * j + 4 * h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int x = 4 * j + e;
+        float pe = exp2f(sc[x] - l4[e]);
+        if (!full) pe = unsigned(m0 + 8 * j + e) < lim ? pe : 0.f;
+        p[x] = pe;
+        ds[x] = pe * dp[x];
+      }
+    }
+    // dV^T += dO^T P and dK^T += Q^T dS: lane (r, h) supplies dO / Q[qr0 + crow(t, h)][DB r + db]
+    if (col_split) {
+#pragma unroll
+      for (int x = 0; x < 16; ++x) {
+        float oa[DB], qa[DB];
+        tile_cols<D>(Dt, crow(x, h), r, oa);
+        tile_cols<D>(Qt, crow(x, h), r, qa);
+        // this wave's half of the column tiles, in the accumulators of the first half
+#pragma unroll
+        for (int db = 0; db < DB / 2; ++db) {
+          dv[db] = mfma32(kh ? oa[DB / 2 + db] : oa[db], p[x], dv[db]);
+          dk[db] = mfma32(kh ? qa[DB / 2 + db] : qa[db], ds[x], dk[db]);
         }
       }
+    } else {
 #pragma unroll
-      for (int t = 0; t < HD; ++t) {
-        s = mfma32(qa[t], kf[t], s);
-        dp = mfma32(da[t], vf[t], dp);
-      }
-      float p[16], ds[16];
+      for (int x = 0; x < 16; ++x) {
+        float oa[DB], qa[DB];
+        tile_cols<D>(Dt, crow(x, h), r, oa);
+        tile_cols<D>(Qt, crow(x, h), r, qa);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int qq = qr0 + crow(i, h);
-        const bool ok = qq >= lo && qq < hi && allowed32(qq, key, W, S);
-        p[i] = ok ? exp2f(s[i] - l2[i]) : 0.f;
-        ds[i] = p[i] * dp[i];
-      }
-      // dV^T += dO^T P and dK^T += Q^T dS: lane (r, h) supplies dO / Q[qr0 + crow(t, h)][32 db + r]
-#pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        const int d = 32 * db + r;
-#pragma unroll
-        for (int t = 0; t < 16; ++t) {
-          const int qq = qr0 + crow(t, h);
-          const bool in = d < D && qq < L;
-          const float doa = in ? dO[int64_t(qq) * a.sdo[2] + d] : 0.f;
-          const float qa2 = in ? Q[int64_t(qq) * a.sq[2] + d] : 0.f;
-          dv[db] = mfma32(doa, p[t], dv[db]);
-          dk[db] = mfma32(qa2, ds[t], dk[db]);
+        for (int db = 0; db < DB; ++db) {
+          dv[db] = mfma32(oa[db], p[x], dv[db]);
+          dk[db] = mfma32(qa[db], ds[x], dk[db]);
         }
       }
     }
   }
-  // outputs: lane (r, h) register i of tile db holds head-dim index 32 db + crow(i, h) of key ks0 + r
-  if (key >= L) return;
-  if (split) {
-    const int64_t slot = ((int64_t(b) * a.Hkv + kvh) * a.nsp + kt) * (a.n_chunks + 1) + (chunk + 1);
-    float* pk = a.partial + slot * 2 * 32 * D + r * D;
-    float* pv = pk + 32 * D;
+
+  // the two item slots' sums (hh = 0 gets hh = 1's), fixed order; the stages are reused
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  float* red = lds + kh * (2 * DB * 16 * 64) + lane;
+  if (hh == 1) {
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        red[(db * 16 + e) * 64] = dk[db][e];
+        red[((DB + db) * 16 + e) * 64] = dv[db][e];
+      }
+  }
+  __syncthreads();
+  if (hh == 1) return;
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      dk[db][e] += red[(db * 16 + e) * 64];
+      dv[db][e] += red[((DB + db) * 16 + e) * 64];
+    }
+
+  if (!is_chunk && ns > 1) {  // a piece: register quads in lane order, whole lines per store
+    float* out = a.kv_part + part_slot * (2 * kKvKeys * 32 * DB) + kh * (DB * 16 * 64) + 4 * lane;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int d = 32 * db + 8 * j + 4 * h;
-        if (d < D) {
-          st4f(pk + d, f32x4{dk[db][4 * j], dk[db][4 * j + 1], dk[db][4 * j + 2], dk[db][4 * j + 3]});
-          st4f(pv + d, f32x4{dv[db][4 * j], dv[db][4 * j + 1], dv[db][4 * j + 2], dv[db][4 * j + 3]});
-        }
+        float* o = out + (db * 4 + j) * 256;
+        st4f(o, f32x4{dk[db][4 * j], dk[db][4 * j + 1], dk[db][4 * j + 2], dk[db][4 * j + 3]});
+        st4f(o + kKvKeys * 32 * DB, f32x4{dv[db][4 * j], dv[db][4 * j + 1], dv[db][4 * j + 2], dv[db][4 * j + 3]});
       }
     return;
   }
-  float* dK = static_cast<float*>(a.dk) + slice_off(a.sdk, b, kvh, sq.row + key);
-  float* dV = static_cast<float*>(a.dv) + slice_off(a.sdv, b, kvh, sq.row + key);
-  const float sc = a.scale;
+  if (key >= L) return;
+  if (partial_block && key < S) {
+    float* pk = a.partial + ((int64_t(b) * a.Hkv + kvh) * (a.n_chunks + 1) + (is_chunk ? chunk : a.n_chunks)) * 2 * S * D + key * D;
+    float* pv = pk + S * D;
+    if (col_split) {
 #pragma unroll
-  for (int db = 0; db < DB; ++db)
+      for (int db = 0; db < DB / 2; ++db)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int d = 32 * db + 8 * j + 4 * h;
-      if (d < D) {
-        st4f(dK + d, f32x4{dk[db][4 * j] * sc, dk[db][4 * j + 1] * sc, dk[db][4 * j + 2] * sc, dk[db][4 * j + 3] * sc});
-        st4f(dV + d, f32x4{dv[db][4 * j], dv[db][4 * j + 1], dv[db][4 * j + 2], dv[db][4 * j + 3]});
-      }
+        for (int e = 0; e < 16; ++e) {
+          const int d = DB * crow(e, h) + kh * (DB / 2) + db;
+          pk[d] = dk[db][e];
+          pv[d] = dv[db][e];
+        }
+      return;
     }
+    store_cols<D>(pk, dk, h, 1.f);
+    store_cols<D>(pv, dv, h, 1.f);
+    return;
+  }
+  if (is_chunk) return;
+  store_cols<D>(static_cast<float*>(a.dk) + slice_off(a.sdk, b, kvh, sq.row + key), dk, h, a.scale);
+  store_cols<D>(static_cast<float*>(a.dv) + slice_off(a.sdv, b, kvh, sq.row + key), dv, h, 1.f);
 }
 
-// Adds the partial sums of the split sink tiles, slot by slot in order (deterministic).  Grid
-// (32 nsp, Hkv, B): one workgroup of D threads per key of a split tile.
+// Adds the kv_split pieces of every key block, piece by piece in order, and writes dK and dV, or a sink
+// row's sums to its block's own slot of the sink partials.  One thread per register quad of a key
+// row (4 DB columns).
+template <int D>
+__global__ __launch_bounds__(256) void fold_pieces32_kernel(const Args a) {
+  constexpr int DB = kDB<D>;
+  constexpr int WGS = 2 * 2 * 4 * 64 / 256;  // [dK, dV][key half][quad][lane]
+  const int per = a.vl_kblocks ? a.vl_kblocks : a.n_kblocks, ns = a.kv_split;
+  const int blk = blockIdx.x / WGS, u = blockIdx.x % WGS * 256 + threadIdx.x;
+  const int lane = u & 63, j = (u >> 6) & 3, kh = (u >> 8) & 1, t = u >> 9;
+  int kvh, b, kblk;
+  if (a.vl_kblocks) {
+    kvh = blk / per;
+    if (!varlen_nth(a, blk % per, per, kKvKeys, 1, b, kblk)) return;
+  } else {
+    kblk = blk % per;
+    kvh = blk / per / a.B;
+    b = blk / per % a.B;
+  }
+  const Seq sq = seq_of(a, b);
+  const int r = lane & 31, h = lane >> 5, key = kKvKeys * kblk + 32 * kh + r;
+  if (key >= sq.L || (D == 16 && j >= 2)) return;
+  constexpr int HALF = kKvKeys * 32 * DB;
+  const float* src = a.kv_part + int64_t(blk) * ns * (2 * HALF) + t * HALF + kh * (DB * 16 * 64) + j * 256 + 4 * lane;
+  f32x4 x[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db) x[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < ns; ++s)
+#pragma unroll
+    for (int db = 0; db < DB; ++db) x[db] += ld4f(src + int64_t(s) * (2 * HALF) + db * 1024);
+  float* dst;
+  float sc = 1.f;
+  if (kblk < a.nsp && key < a.S) {
+    dst = a.partial + (((int64_t(b) * a.Hkv + kvh) * (a.n_chunks + 1) + a.n_chunks) * 2 + t) * a.S * D + key * D;
+  } else if (t == 0) {
+    dst = static_cast<float*>(a.dk) + slice_off(a.sdk, b, kvh, sq.row + key);
+    sc = a.scale;
+  } else {
+    dst = static_cast<float*>(a.dv) + slice_off(a.sdv, b, kvh, sq.row + key);
+  }
+  dst += DB * (8 * j + 4 * h);
+#pragma unroll
+  for (int y = 0; y < DB; ++y) {
+    f32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = x[(4 * y + e) % DB][(4 * y + e) / DB] * sc;
+    st4f(dst + 4 * y, v);
+  }
+}
+
+// Adds the partial sums of the sink rows of the blocks below nsp, slot by slot in order
+// (deterministic).  Grid (sink rows, Hkv, B): one workgroup of 128 threads per key.
 template <int D>
 __global__ __launch_bounds__(128) void fold32_kernel(const Args a) {
   const int kvh = blockIdx.y, b = blockIdx.z;
   const Seq sq = seq_of(a, b);
-  const int kt = blockIdx.x / 32, r = blockIdx.x % 32, d = threadIdx.x;
-  const int ks0 = 32 * kt, key = ks0 + r;
+  const int key = blockIdx.x, d = threadIdx.x, kblk = key / kKvKeys;
   if (key >= sq.L || d >= D) return;
-  if (!(ks0 < a.S && kv32_row_end(ks0, sq.L, a.W) < sq.L && kt < a.nsp)) return;  // not split: written directly
-  const int64_t slot0 = ((int64_t(b) * a.Hkv + kvh) * a.nsp + kt) * (a.n_chunks + 1);
-  float sk = 0.f, sv = 0.f;
-  for (int c = 0; c <= a.n_chunks; ++c) {
-    const float* pk = a.partial + (slot0 + c) * 2 * 32 * D + r * D + d;
-    // chunks that start past the sequence's end wrote nothing: skip them
-    if (c > 0 && kv32_row_end(ks0, sq.L, a.W) + (c - 1) * a.chunk_rows >= sq.L) break;
-    sk += pk[0];
-    sv += pk[32 * D];
+  const float* src = a.partial + (int64_t(b) * a.Hkv + kvh) * (a.n_chunks + 1) * 2 * a.S * D + key * D + d;
+  const int64_t slot = int64_t(2) * a.S * D;
+  // chunks that start past the sequence's end wrote nothing
+  const int rows = sq.L - kv_chunk_base(kblk, sq.L, a.W);
+  const int n = kv_window_end(kblk, sq.L, a.W) < sq.L ? (rows + a.chunk_rows - 1) / a.chunk_rows : 0;
+  float sk = src[a.n_chunks * slot], sv = src[a.n_chunks * slot + a.S * D];
+  constexpr int kBatch = 16;  // loads in flight (one at a time, c2's 62 chunks took 17 us)
+  for (int c0 = 0; c0 < n; c0 += kBatch) {
+    float xk[kBatch], xv[kBatch];
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      const float* p = src + min(c0 + j, n - 1) * slot;
+      xk[j] = p[0];
+      xv[j] = p[a.S * D];
+    }
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      sk += c0 + j < n ? xk[j] : 0.f;
+      sv += c0 + j < n ? xv[j] : 0.f;
+    }
   }
   static_cast<float*>(a.dk)[slice_off(a.sdk, b, kvh, sq.row + key) + d] = sk * a.scale;
   static_cast<float*>(a.dv)[slice_off(a.sdv, b, kvh, sq.row + key) + d] = sv;
 }
 
+template <int D>
+hipError_t fwd_d(const Args& a, hipStream_t s) {
+  hipLaunchKernelGGL(fwd32_kernel<D>, dim3(a.n_qtiles * a.B * (a.Hq / a.wh)), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+template <int D>
+hipError_t dq_d(const Args& a, hipStream_t s) {
+  hipLaunchKernelGGL(dq32_kernel<D>, dim3(a.n_qtiles * a.B * (a.Hq / a.wh)), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+template <int D>
+hipError_t dkdv_d(const Args& a, hipStream_t s) {
+  const int blocks = a.Hkv * (a.vl_kblocks ? a.vl_kblocks : a.B * a.n_kblocks);
+  hipLaunchKernelGGL(dkdv32_kernel<D>, dim3(a.kv_split * blocks + a.n_chunk_wgs), dim3(256), 0, s, a);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess && a.kv_split > 1) {
+    hipLaunchKernelGGL(fold_pieces32_kernel<D>, dim3(4 * blocks), dim3(256), 0, s, a);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess && a.nsp > 0) {
+    hipLaunchKernelGGL(fold32_kernel<D>, dim3(min(a.S, kKvKeys * a.nsp), a.Hkv, a.B), dim3(128), 0, s, a);
+    e = hipGetLastError();
+  }
+  return e;
+}
+
 }  // namespace
 
-hipError_t launch_fwd_f32(const Args& a, int D, hipStream_t s) {
-  const dim3 grid((a.L + 31) / 32, a.Hq, a.B), block(64);
-  switch (D) {
-    case 16: hipLaunchKernelGGL(fwd32_kernel<16>, grid, block, 0, s, a); break;
-    case 32: hipLaunchKernelGGL(fwd32_kernel<32>, grid, block, 0, s, a); break;
-    case 64: hipLaunchKernelGGL(fwd32_kernel<64>, grid, block, 0, s, a); break;
-    case 128: hipLaunchKernelGGL(fwd32_kernel<128>, grid, block, 0, s, a); break;
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
+#define FA_F32_D(FN)                  \
+  switch (D) {                        \
+    case 16: return FN<16>(a, s);     \
+    case 32: return FN<32>(a, s);     \
+    case 64: return FN<64>(a, s);     \
+    case 128: return FN<128>(a, s);   \
+  }                                   \
+  return hipErrorInvalidValue;
 
-hipError_t launch_bwd_dq_f32(const Args& a, int D, hipStream_t s) {
-  const dim3 grid((a.L + 31) / 32, a.Hq, a.B), block(64);
-  switch (D) {
-    case 16: hipLaunchKernelGGL(dq32_kernel<16>, grid, block, 0, s, a); break;
-    case 32: hipLaunchKernelGGL(dq32_kernel<32>, grid, block, 0, s, a); break;
-    case 64: hipLaunchKernelGGL(dq32_kernel<64>, grid, block, 0, s, a); break;
-    case 128: hipLaunchKernelGGL(dq32_kernel<128>, grid, block, 0, s, a); break;
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
-
-hipError_t launch_bwd_dkdv_f32(const Args& a, int D, hipStream_t s) {
-  const dim3 grid(a.n_kblocks + a.nsp * a.n_chunks, a.Hkv, a.B), block(64);
-  switch (D) {
-    case 16: hipLaunchKernelGGL(dkdv32_kernel<16>, grid, block, 0, s, a); break;
-    case 32: hipLaunchKernelGGL(dkdv32_kernel<32>, grid, block, 0, s, a); break;
-    case 64: hipLaunchKernelGGL(dkdv32_kernel<64>, grid, block, 0, s, a); break;
-    case 128: hipLaunchKernelGGL(dkdv32_kernel<128>, grid, block, 0, s, a); break;
-    default: return hipErrorInvalidValue;
-  }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || a.nsp == 0) return e;
-  const dim3 fgrid(32 * a.nsp, a.Hkv, a.B), fblock(128);
-  switch (D) {
-    case 16: hipLaunchKernelGGL(fold32_kernel<16>, fgrid, fblock, 0, s, a); break;
-    case 32: hipLaunchKernelGGL(fold32_kernel<32>, fgrid, fblock, 0, s, a); break;
-    case 64: hipLaunchKernelGGL(fold32_kernel<64>, fgrid, fblock, 0, s, a); break;
-    case 128: hipLaunchKernelGGL(fold32_kernel<128>, fgrid, fblock, 0, s, a); break;
-  }
-  return hipGetLastError();
-}
+hipError_t launch_fwd_f32(const Args& a, int D, hipStream_t s) { FA_F32_D(fwd_d) }
+hipError_t launch_bwd_dq_f32(const Args& a, int D, hipStream_t s) { FA_F32_D(dq_d) }
+hipError_t launch_bwd_dkdv_f32(const Args& a, int D, hipStream_t s) { FA_F32_D(dkdv_d) }
 
 }  // namespace fa

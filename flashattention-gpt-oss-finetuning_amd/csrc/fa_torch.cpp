@@ -148,7 +148,7 @@ std::vector<at::Tensor> bwd(const at::Tensor& q_in, const at::Tensor& k_in, cons
   at::Tensor dk = at::empty_like(k);
   at::Tensor dv = at::empty_like(v);
   const size_t ws_bytes = fa_bwd_full_workspace_bytes(clamp_i32(B), clamp_i32(Hq), clamp_i32(Hkv), clamp_i32(L),
-                                                      clamp_i32(D), clamp_i32(window), clamp_i32(sink), -1);
+                                                      clamp_i32(D), clamp_i32(window), clamp_i32(sink), dtype_code(q), -1);
   at::Tensor ws = at::empty({int64_t(ws_bytes > 256 ? ws_bytes : 256)}, q.options().dtype(at::kByte));
   fa_bwd_params p{};
   p.q = q.data_ptr();

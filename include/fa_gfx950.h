@@ -137,7 +137,8 @@ size_t fa_bwd_workspace_bytes(int32_t batch, int32_t heads_q, int32_t heads_kv, 
  * call with less room differ from those of one with more by the order of fp32 sums.  Returns 0
  * for an invalid problem. */
 size_t fa_bwd_full_workspace_bytes(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t seqlen,
-                                   int32_t head_dim, int32_t window, int32_t sink, int32_t total_rows);
+                                   int32_t head_dim, int32_t window, int32_t sink, int32_t dtype,
+                                   int32_t total_rows);
 
 /* Launches the backward kernels (fa_bwd_dq then fa_bwd_dkdv).  `workspace` must hold
  * at least fa_bwd_workspace_bytes() bytes of device memory, 256-byte aligned; its contents on entry

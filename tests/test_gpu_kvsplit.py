@@ -34,8 +34,9 @@ CASES = [
 ]
 
 
-def full_bytes(L, *shape, total=-1):
-    return int(L.fa_bwd_full_workspace_bytes(*shape, total))
+def full_bytes(L, *shape, dtype, total=-1):
+    code = load_mod("_ops")._DTYPES[dtype]
+    return int(L.fa_bwd_full_workspace_bytes(*shape, code, total))
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,L,D,W,S,dtype,pieces", CASES)
@@ -46,7 +47,7 @@ def test_split_dkdv(gpu, B, Hq, Hkv, L, D, W, S, dtype, pieces):
     sc = 1.0 / math.sqrt(D)
     o, lse = ops.forward(q, k, v, W, S, sc)
     base = int(lib.fa_bwd_workspace_bytes(B, Hq, Hkv, L, D, W, S))
-    full = full_bytes(lib, B, Hq, Hkv, L, D, W, S)
+    full = full_bytes(lib, B, Hq, Hkv, L, D, W, S, dtype=dtype)
     per_piece = B * Hkv * ((L + 63) // 64) * 2 * 64 * max(D, 32) * 4
     assert full - base == pieces * per_piece  # the plan's number of pieces
     ref = naive.attention_fwd_bwd(q, k, v, do, W, S, scale=sc, compute_dtype=torch.float32, row_chunk=2048)
@@ -94,7 +95,7 @@ def test_split_dkdv_packed(gpu, D, dtype):
     sc = 1.0 / math.sqrt(D)
     o, lse = ops.forward_varlen(q, k, v, cu_dev, max_len, W, S, sc)
     base = int(lib.fa_bwd_workspace_bytes(B, Hq, Hkv, max_len, D, W, S))
-    full = full_bytes(lib, B, Hq, Hkv, max_len, D, W, S, total=total)
+    full = full_bytes(lib, B, Hq, Hkv, max_len, D, W, S, dtype=dtype, total=total)
     assert full > base
     split = ops.backward_varlen(q, k, v, o, lse, do, cu_dev, max_len, W, S, sc)
     real, ops.workspace_bytes = ops.workspace_bytes, lambda *a: base
