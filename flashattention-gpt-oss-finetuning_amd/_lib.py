@@ -47,6 +47,8 @@ EXPORTS = (
     "fa_bwd_varlen",
     "fa_fwd_fp8",
     "fa_fwd_fp8_pv",
+    "fa_quantize_fp8",
+    "fa_quantize_fp8_amax",
     "fa_bwd_workspace_bytes",
     "fa_bwd_full_workspace_bytes",
     "fa_check_fwd",
@@ -155,6 +157,9 @@ def lib() -> ctypes.CDLL:
                 fn.restype = ctypes.c_int
             L.fa_bwd_workspace_bytes.argtypes = [ctypes.c_int32] * 7
             L.fa_bwd_workspace_bytes.restype = ctypes.c_size_t
+            L.fa_quantize_fp8.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64, ctypes.c_void_p,
+                                          ctypes.c_double, ctypes.c_void_p]
+            L.fa_quantize_fp8_amax.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64] + [ctypes.c_void_p] * 5
             L.fa_bwd_full_workspace_bytes.argtypes = [ctypes.c_int32] * 9
             L.fa_bwd_full_workspace_bytes.restype = ctypes.c_size_t
             L.fa_check_fwd.argtypes = [ctypes.POINTER(FwdParams)]

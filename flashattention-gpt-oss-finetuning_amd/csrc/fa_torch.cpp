@@ -248,6 +248,38 @@ at::Tensor swda_sinks(const at::Tensor& q, const at::Tensor& k, const at::Tensor
   return SwdaSinksFunction::apply(q, k, v, sinks, window, sink, scale);
 }
 
+// Per-tensor e4m3 quantisation of a GPU tensor (quantize_fp8 in attention.py): (x8, descale), x8 with x's
+// strides; without a given descale it is max |x| / 448.  The host waits for the maximum only: the codes
+// are written by a kernel behind it that reads the maximum on the device.  Returns None for tensors
+// the kernels do not take (other dtypes, strides with gaps, unaligned or empty).
+py::object quantize_fp8(const at::Tensor& x_in, c10::optional<double> descale) {
+  const at::Tensor x = x_in.detach();
+  const auto st = x.scalar_type();
+  const int dtype = st == at::kBFloat16 ? FA_DTYPE_BF16 : st == at::kHalf ? FA_DTYPE_F16 : st == at::kFloat ? FA_DTYPE_F32 : 0;
+  if (!x.is_cuda() || dtype == 0 || x.numel() == 0 || !x.is_non_overlapping_and_dense() ||
+      (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) != 0)
+    return py::none();
+  const c10::DeviceGuard guard(x.device());
+  at::Tensor x8 = at::empty_like(x, x.options().dtype(at::kFloat8_e4m3fn));
+  void* stream = current_stream(x);
+  if (descale.has_value()) {
+    raise_for_status(fa_quantize_fp8(x.data_ptr(), dtype, x.numel(), x8.data_ptr(), *descale, stream),
+                     "fa_quantize_fp8");
+    return py::make_tuple(x8, *descale);
+  }
+  at::Tensor parts = at::empty({FA_AMAX_PARTS}, x.options().dtype(at::kFloat));
+  at::Tensor host = at::empty({FA_AMAX_PARTS}, at::TensorOptions().dtype(at::kFloat).pinned_memory(true));
+  float amax = 0.f;
+  int rc;
+  {
+    py::gil_scoped_release nogil;
+    rc = fa_quantize_fp8_amax(x.data_ptr(), dtype, x.numel(), x8.data_ptr(), parts.data_ptr<float>(),
+                              host.data_ptr<float>(), &amax, stream);
+  }
+  raise_for_status(rc, "fa_quantize_fp8_amax");
+  return py::make_tuple(x8, amax > 0.f ? double(amax) / 448.0 : 1.0);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -257,6 +289,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("swda_sinks", &swda_sinks,
         "autograd forward with learned sink logits: (q, k, v, sinks, window, sink, scale) -> o", py::arg("q"),
         py::arg("k"), py::arg("v"), py::arg("sinks"), py::arg("window"), py::arg("sink"), py::arg("scale"));
+  m.def("quantize_fp8", &quantize_fp8, "per-tensor e4m3 quantisation: (x, descale=None) -> (x8, descale) or None",
+        py::arg("x"), py::arg("descale") = py::none());
   m.doc() = "PyTorch binding of libfa_gfx950.so (fa_fwd / fa_bwd)";
   m.def("fwd", &fwd, "forward: (q, k, v, window, sink, scale, sinks=None) -> (o, lse)", py::arg("q"), py::arg("k"),
         py::arg("v"), py::arg("window"), py::arg("sink"), py::arg("scale"), py::arg("sinks") = py::none());

@@ -212,6 +212,18 @@ int fa_fwd_varlen(const fa_fwd_params* p, const int32_t* cu_seqlens, int32_t tot
 int fa_bwd_varlen(const fa_bwd_params* p, const int32_t* cu_seqlens, int32_t total_rows, const float* sinks,
                   float* dsinks, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Per-tensor e4m3 quantisation for the FP8 forward, over the n elements of a dense bf16, fp16 or fp32
+ * tensor x: the codes of clamp(x / descale, -448, 448) to `out` (both 16-byte aligned), dividing as a
+ * product with the reciprocal of descale rounded to float32.  fa_quantize_fp8_amax takes descale = max |x| / 448 (1 where
+ * that maximum is 0 or NaN) and returns the maximum (NaN if x holds one) in *amax: it enqueues
+ * everything, then blocks the host until the maximum is known, while the codes are still being
+ * written.  `parts` is FA_AMAX_PARTS floats of device memory, `host_parts` as many of pinned host
+ * memory; both are free again when the codes are written (stream order) and at return. */
+#define FA_AMAX_PARTS 1024
+int fa_quantize_fp8(const void* x, int32_t dtype, int64_t n, void* out, double descale, void* stream);
+int fa_quantize_fp8_amax(const void* x, int32_t dtype, int64_t n, void* out, float* parts, float* host_parts,
+                         float* amax, void* stream);
+
 /* FP8 forward: q, k and v hold OCP float8 e4m3 values (p->dtype = FA_DTYPE_FP8_E4M3, strides in
  * elements, i.e. bytes, multiples of 16, bases 16-byte aligned); the values they stand for are
  * q_descale * q, k_descale * k and v_descale * v.  o is written in bf16 (strides in bf16

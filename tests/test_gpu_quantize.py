@@ -1,0 +1,63 @@
+"""GPU test of quantize_fp8's kernels: the codes and the scale are those of the PyTorch expression
+(x.float() / descale).clamp(-448, 448).to(float8_e4m3fn), bit for bit, over every 16-bit pattern,
+NaNs, infinities, the tensor sizes around a kernel's 16-element unit, and strided layouts."""
+import pytest
+import torch
+
+from conftest import load_pkg
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(x, descale=None):
+    xf = x.detach().float()
+    if descale is None:
+        amax = float(xf.abs().max()) if xf.numel() else 0.0
+        descale = amax / 448.0 if amax > 0.0 else 1.0
+    return (xf / descale).clamp(-448.0, 448.0).to(torch.float8_e4m3fn), float(descale)
+
+
+def check(x, descale=None):
+    got, gd = load_pkg().quantize_fp8(x, descale)
+    ref, rd = reference(x, descale)
+    assert gd == rd and isinstance(gd, float)
+    assert got.dtype == torch.float8_e4m3fn and got.shape == ref.shape and got.stride() == ref.stride()
+    assert not got.requires_grad
+    nan = torch.isnan(ref.float())
+    assert torch.equal(torch.isnan(got.float()), nan)
+    g, r = got.view(torch.uint8), ref.view(torch.uint8)
+    assert torch.equal(g[~nan], r[~nan])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("descale", [None, 1.0, 0.0123, 7.0, 3e-5])
+def test_every_16_bit_value(gpu, dtype, descale):
+    x = torch.arange(65536, dtype=torch.int32, device=gpu).to(torch.int16).view(dtype)
+    check(x, descale)  # NaNs and infinities included
+    check(x[torch.isfinite(x.float())], descale)
+
+
+@pytest.mark.parametrize("n", [1, 3, 7, 8, 15, 16, 17, 31, 255, 4096, 4099, 1 << 20, (1 << 20) + 5])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_sizes(gpu, n, dtype):
+    g = torch.Generator(device=gpu).manual_seed(n)
+    x = (torch.randn(n, generator=g, device=gpu) * 3).to(dtype)
+    for d in (None, 0.01):
+        check(x, d)
+    x[n // 2] = -1000.0  # the maximum is a negative element, wherever it lies
+    check(x)
+    x[n - 1] = float("nan")
+    check(x)
+
+
+def test_layouts_and_special_tensors(gpu):
+    x = torch.randn(2, 100, 8, 64, device=gpu).bfloat16().requires_grad_()
+    check(x.transpose(1, 2))  # dense: kept in its layout
+    check(x[:, :, :4])  # gaps: the PyTorch expression
+    check(torch.randn(1025, device=gpu).bfloat16()[1:])  # not 16-byte aligned
+    check(torch.zeros(40, device=gpu, dtype=torch.float16))
+    check(torch.zeros(0, 4, device=gpu))
+    check(torch.randn(64, device=gpu, dtype=torch.float64))
+    check(torch.full((33,), float("inf"), device=gpu))
+    check(torch.full((33,), 1e-44, device=gpu))
+    check(torch.tensor([0.0, -0.0, 1e-30, -3e38], device=gpu))
