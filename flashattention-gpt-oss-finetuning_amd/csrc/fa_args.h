@@ -156,6 +156,21 @@ __device__ __forceinline__ KvPiece kv_piece(int id, int streams, int ns) {
   return KvPiece{stream % ns, stream / ns, p};
 }
 
+// Workgroup id -> (stream, position) of the query-major kernels that run one tile per workgroup: a stream
+// is one (KV head, batch, head group), positions count its row tiles from the last.  An XCD owns whole
+// streams where their number allows (their tiles share K/V rows in its L2) and takes their tiles
+// together, the last rows, which see the most keys, first.
+struct QStream {
+  int stream, pos;
+};
+__device__ __forceinline__ QStream q_stream(int id, int streams) {
+  if (streams % 8 == 0) {
+    const int spx = streams / 8, pos = id / 8;
+    return QStream{id % 8 * spx + pos % spx, pos / spx};
+  }
+  return QStream{id % streams, id / streams};
+}
+
 // Element offset of row `row` of (batch b, head h) of a tensor with strides s[3] (a plain array
 // or one read through args_fresh()).
 template <typename S3>
@@ -198,9 +213,12 @@ struct TailArgs {
 int device_cus();
 
 // Launchers (return the hipError_t of the launch; launch_bwd_dkdv also launches the sink fold).
-hipError_t launch_fwd(const Args& a, int dtype, int D, int hpw, hipStream_t stream);
+hipError_t launch_fwd(const Args& a, int dtype, int D, hipStream_t stream);
 // e4m3 q, k, v; bf16 o; fp8_pv: P V on the fp8 MFMA as well
 hipError_t launch_fwd_fp8(const Args& a, int D, int hpw, bool fp8_pv, hipStream_t stream);
+// the forward with one tile per workgroup, whose keys are split over `ksp` waves: 1, 2 or 4 (D < 128);
+// reads wq, wh (wq wh ksp = 4) and n_qtiles (tiles of 32 wq rows)
+hipError_t launch_fwd_split(const Args& a, int dtype, int D, int hpw, int ksp, hipStream_t stream);
 hipError_t launch_bwd_dq(const Args& a, int dtype, int D, int hpw, hipStream_t stream);
 // the sliding dQ kernel (D = 64, 16-bit, G a multiple of 8, 1 <= W <= 161, S <= 32)
 hipError_t launch_bwd_dq_slide(const Args& a, int dtype, hipStream_t stream);

@@ -253,8 +253,8 @@ KvSteps kv_steps(double L, double W, double G) {
   return KvSteps{G * (n_win > 0 ? win : n_kb), G * (n_win * win + r * (r + 1) / 2)};
 }
 
-// Pieces per key block of the dK/dV kernel (1: unsplit) for `nseq` sequences of L rows on `cus` compute
-// units: the power of two up to 32 with the least estimated time.  The kernel takes as long as its
+// Pieces per key block of the dK/dV kernel (1: unsplit) for `nseq` sequences of L rows on average and
+// max_L at most on `cus` compute units: the power of two up to 32 with the least estimated time.  The kernel takes as long as its
 // longest workgroup (a full causal layer's key block 0 sweeps every row, twice the average), or as
 // the average work of a resident slot where that is more, or half of each, at the rate of full slots,
 // where the longest starts on a full chip; splitting shortens the first, and costs
@@ -268,12 +268,13 @@ KvSteps kv_steps(double L, double W, double G) {
 // window of 1024 at L = 4096 (equal workgroups) 143 / 154 / 162 / 177 / 245.
 // The float32 kernel (the last four of each table): L = 2048, Hq = 64, Hkv = 8, D = 64 by pieces 1 / 2 / 4 /
 // 8 / 16 1260 / 849 / 650 / 603 / 644; D = 128, Hq = 16, Hkv = 8 610 / 361 / 377 / 431 / 536.
-int kv_split_pieces(bool f32, int D, int G, int Hkv, double nseq, double L, double W, bool folds, int cus) {
+int kv_split_pieces(bool f32, int D, int G, int Hkv, double nseq, double L, double max_L, double W, bool folds,
+                    int cus) {
   const int i = (D == 16 ? 0 : D == 32 ? 1 : D == 64 ? 2 : 3) + (f32 ? 4 : 0);
   const double t_long[8] = {0.55, 0.58, 0.8, 1.15, 2.9, 2.9, 4.9, 9.3};
   const double t_slot[8] = {1.3, 1.5, 1.14, 1.25, 6.5, 6.5, 8.8, 9.6};
   const int per_cu[8] = {4, 4, 2, 1, 4, 3, 2, 1};  // resident workgroups
-  const KvSteps st = kv_steps(L, W, G);
+  const KvSteps st{kv_steps(max_L, W, G).longest, kv_steps(L, W, G).total};
   const double slot = t_slot[i] * st.total * nseq * Hkv / (double(cus) * per_cu[i]);
   const double mb = nseq * Hkv * std::ceil(L / fa::kKvKeys) * fa::kKvKeys * (D < 32 ? 32 : D) * 8 * 1e-6;  // per piece
   auto kernel_us = [&](double longest) {
@@ -309,11 +310,75 @@ void plan_kv_split(fa::Args& a, int D, bool f32, char* ws, size_t spare) {
   const int cus = fa::device_cus();
   if (!f32 && fa::dkdv4_eligible(a, D, cus)) return;
   const double rows = a.cu_seqlens ? std::min(double(a.L), std::max(1., double(a.total_rows) / a.B)) : double(a.L);
-  int ns = kv_split_pieces(f32, D, a.G, a.Hkv, a.B, rows, a.W, a.sink_dq != 0, cus);
+  int ns = kv_split_pieces(f32, D, a.G, a.Hkv, a.B, rows, a.L, a.W, a.sink_dq != 0, cus);
   const int64_t blocks = kv_blocks(a);
   while (ns > 1 && (kv_part_bytes(D, blocks, ns) > spare || blocks * ns > (int64_t(1) << 24))) ns /= 2;
   a.kv_split = ns;
   a.kv_part = reinterpret_cast<float*>(ws);
+}
+
+// The 16-bit forward with one tile per workgroup (fwd_split_kernel): how many waves share a tile's keys
+// (1, 2 or 4; wq, wh and n_qtiles are set), or 0 for fwd_kernel.  The least estimated time over the
+// choices, as for the dK/dV split: the longest tile alone on its CU, or the average work of a resident
+// slot plus part of the longest tile's excess, and each workgroup's fixed time (its Q rows and first
+// keys, the merge).  In us per step of a workgroup, alone / with full slots; measured over Hq = 8 .. 64,
+// G = 1 .. 16, L = 257 .. 8192, W = 128 .. full (fwd_split_kernel's comment has the D = 64 figures; G = 1,
+// Hq = 16, L = 4096 full causal: D = 64 81 / 60 / 74 for 1 / 2 / 4 waves against 88 for fwd_kernel, D = 16
+// at L = 2048 34 / 20 / 14 against 27).
+// fwd_kernel keeps what it still does better: D <= 32 with one head per wave and short windows, whose
+// tiles' key blocks it fetches at once (the D = 16, W = 256 default case 10.9 against 12.2 us), and D = 128
+// with one head per KV group (B = 2, Hq = 32, L = 2048 full causal 81.5 against 85 us).
+int plan_fwd_split(fa::Args& a, int D, int hpw) {
+  struct Cost {
+    int per_cu;
+    double alone, full;
+  };
+  static const Cost costs[4][2][3] = {
+      // [D][heads per wave - 1][KSP = 1, 2, 4]
+      {{{7, 0.47, 1.5}, {7, 0.5, 1.5}, {7, 0.6, 1.55}}, {{4, 0.5, 1.3}, {4, 0.6, 1.4}, {4, 0.75, 1.5}}},
+      {{{5, 0.5, 1.6}, {5, 0.6, 1.6}, {4, 0.8, 1.4}}, {{4, 0.63, 1.6}, {4, 0.77, 1.6}, {4, 1.0, 1.8}}},
+      {{{4, 0.56, 1.34}, {4, 0.7, 1.38}, {2, 0.9, 1.15}}, {{3, 0.75, 1.57}, {3, 0.85, 1.72}, {2, 1.1, 1.43}}},
+      {{{2, 0.83, 1.04}, {2, 1.2, 1.3}, {0, 0, 0}}, {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}}};
+  const double fixed[3] = {3, D == 64 ? 4.5 : 3.5, 3};  // one launch's, merge included
+  const int di = D == 16 ? 0 : D == 32 ? 1 : D == 64 ? 2 : 3;
+  if (D <= 32 && hpw == 1 && a.W <= 320) return 0;
+  if (D == 128 && a.G % 2 != 0) return 0;
+  const double rows = a.cu_seqlens ? std::min(double(a.L), std::max(1., double(a.total_rows) / a.B)) : double(a.L);
+  const int cus = fa::device_cus();
+  // steps of one head set's tiles over `n` rows in tiles of 32 wq, for `ksp` waves on a tile's halves
+  auto steps = [&](double n, int wq, int ksp, double* longest) {
+    const double nt = std::ceil(n / (32 * wq));
+    const double n1 = std::min(nt, std::floor((a.W - 1) / (32. * wq)) + 1);  // tiles that see key 0's half
+    const double win = std::ceil((wq + std::ceil((a.W - 1) / 32.) + std::ceil(std::min(a.S, 64) / 32.)) / ksp);
+    *longest = std::max(std::ceil(n1 * wq / ksp), nt > n1 ? win : 0.);
+    return n1 * (n1 + 1) / 2 * wq / ksp + n1 * (ksp - 1) / (2. * ksp) + (nt - n1) * win;
+  };
+  int best = 0, best_wh = 0;
+  double best_t = 0;
+  for (int k = 0; k < 3; ++k) {
+    const Cost& c = costs[di][hpw - 1][k];
+    if (!c.per_cu) continue;
+    const int ksp = 1 << k;
+    int wh = 4 / ksp;
+    while (a.G % (hpw * wh) != 0) wh /= 2;
+    const int wq = 4 / ksp / wh;
+    const double streams = double(a.B) * (a.Hq / (hpw * wh)), slots = double(cus) * c.per_cu;
+    double longest;
+    const double slot = c.full * streams * steps(rows, wq, ksp, &longest) / slots;
+    steps(a.L, wq, ksp, &longest);  // (a packed batch's longest sequence)
+    const double wgs = streams * std::ceil(rows / (32 * wq));
+    const double t = std::max(c.alone * longest, slot + 0.3 * std::max(0., c.full * longest - slot)) +
+                     fixed[k] + (hpw == 2 ? 4. : 3.) * wgs / slots;
+    if (!best || t < 0.97 * best_t) {
+      best = ksp;
+      best_wh = wh;
+      best_t = t;
+    }
+  }
+  a.wh = best_wh;
+  a.wq = 4 / best / best_wh;
+  a.n_qtiles = (a.L + 32 * a.wq - 1) / (32 * a.wq);
+  return best;
 }
 
 // The kernel arguments that describe the dK/dV kernel's key blocks and sink chunks.
@@ -481,9 +546,15 @@ int run_fwd(const fa_fwd_params* p, const float* sinks, void* stream, const int3
   a.wh = wh;
   a.wq = wq;
   a.n_qtiles = (a.L + 32 * wq - 1) / (32 * wq);
-  if (f32)
-    return fa::launch_fwd_f32(a, p->head_dim, static_cast<hipStream_t>(stream)) == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
-  const hipError_t e = fa::launch_fwd(a, p->dtype, p->head_dim, hpw, static_cast<hipStream_t>(stream));
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  hipError_t e;
+  if (f32) {
+    e = fa::launch_fwd_f32(a, p->head_dim, s);
+  } else if (const int ksp = plan_fwd_split(a, p->head_dim, hpw)) {
+    e = fa::launch_fwd_split(a, p->dtype, p->head_dim, hpw, ksp, s);
+  } else {
+    e = fa::launch_fwd(a, p->dtype, p->head_dim, s);
+  }
   return e == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
 }
 

@@ -49,21 +49,6 @@ __device__ __forceinline__ float other_half(float x) { return __shfl_xor(x, 32);
 template <int D>
 constexpr int kDB = D >= 32 ? D / 32 : 1;
 
-// Key tiles of 32 that rows [q0, q0 + bm) of a sequence of L rows visit: the sink tiles [0, nsink)
-// (keys below S that lie before the window tiles) and the window tiles [ws, we).
-struct Plan32 {
-  int nsink, ws, we;
-};
-__device__ __forceinline__ Plan32 plan32(int q0, int bm, int L, int W, int S) {
-  Plan32 p;
-  const int q_end = min(q0 + bm, L);
-  const int wlo = max(0, q0 - W + 1);  // first key in any row's window
-  p.ws = wlo / 32;
-  p.we = q_end > wlo ? (q_end - 1) / 32 + 1 : p.ws;
-  p.nsink = (min(S, 32 * p.ws) + 31) / 32;
-  return p;
-}
-__device__ __forceinline__ int plan32_tile(const Plan32& p, int i) { return i < p.nsink ? i : p.ws + (i - p.nsink); }
 __device__ __forceinline__ bool allowed32(int q, int k, int W, int S) { return k <= q && (q - k < W || k < S); }
 
 // One fp32 half row (D / 2 values starting at column h D / 2) of row `row` of a [rows][stride]
@@ -140,29 +125,19 @@ __device__ __forceinline__ void store_cols(float* row, const f32x16 (&acc)[kDB<D
 }
 
 // Workgroup -> rows and heads of the query-major kernels: wq x wh waves of 32 rows x 1 head of one KV
-// group.  An XCD owns whole (batch, head group)s where their number allows (their tiles share K/V
-// rows in its L2), takes their row tiles together and the last rows, which see the most keys, first.
+// group (see q_stream).
 struct QTile {
   int b, kvh, hq, q0, qw;
 };
 __device__ __forceinline__ QTile q_tile(const Args& a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int groups = a.B * (a.Hq / a.wh), id = blockIdx.x;
-  int grp, qt;
-  if (groups % 8 == 0) {
-    const int gpx = groups / 8, pos = id / 8;
-    grp = id % 8 * gpx + pos % gpx;
-    qt = pos / gpx;
-  } else {
-    grp = id % groups;
-    qt = id / groups;
-  }
   const int gpk = a.G / a.wh;  // head groups per KV head
+  const QStream s = q_stream(blockIdx.x, a.B * a.Hkv * gpk);
   QTile t;
-  t.kvh = grp / gpk / a.B;
-  t.b = grp / gpk % a.B;
-  t.hq = t.kvh * a.G + grp % gpk * a.wh + wave / a.wq;
-  t.q0 = (a.n_qtiles - 1 - qt) * 32 * a.wq;
+  t.kvh = s.stream / gpk / a.B;
+  t.b = s.stream / gpk % a.B;
+  t.hq = t.kvh * a.G + s.stream % gpk * a.wh + wave / a.wq;
+  t.q0 = (a.n_qtiles - 1 - s.pos) * 32 * a.wq;
   t.qw = t.q0 + 32 * (wave % a.wq);
   return t;
 }

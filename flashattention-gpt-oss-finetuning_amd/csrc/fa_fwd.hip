@@ -70,7 +70,8 @@ constexpr int kQFrags = F8 ? D / 32 : D / 16;
 
 // Masked scores S^T = K Q^T of one 32-key half [ks0, ks0 + 32) -- the swizzled K tile at Kl --
 // for the HPW heads of a wave whose 32 rows start at qw (this lane's row q).
-template <typename E, int D, int HPW, int F8>
+// PAT: the workgroup has the recurring masks at `pat` (otherwise every partial mask is computed).
+template <typename E, int D, int HPW, int F8, bool PAT = true>
 __device__ __forceinline__ void half_scores(const Args& a, const uint16_t* Kl, int ks0, int qw, int q,
                                             const u32x4 (&qf)[HPW][kQFrags<D, F8>], const float* pat,
                                             EdgeOffsets eo, f32x16 (&s)[HPW]) {
@@ -115,7 +116,7 @@ __device__ __forceinline__ void half_scores(const Args& a, const uint16_t* Kl, i
   } else {
     f32x16 bias;
     const int dl = qw - ks0;
-    const int pi = ks0 >= S ? (dl == 0 ? 0 : dl == eo.e1 ? 1 : dl == eo.e2 ? 2 : -1)
+    const int pi = !PAT ? -1 : ks0 >= S ? (dl == 0 ? 0 : dl == eo.e1 ? 1 : dl == eo.e2 ? 2 : -1)
                             : (ks0 == 0 && S < 32 && qw - 31 >= W ? 3 : -1);
     const int dq0 = q - ks0 - 4 * hf;
     if (pi >= 0) {  // a recurring pattern: four 16-byte LDS reads
@@ -145,14 +146,14 @@ __device__ __forceinline__ void half_scores(const Args& a, const uint16_t* Kl, i
 
 // One 32-key half of the 16-bit P V path: masked scores, the online-softmax update of (m2, lsum,
 // acc) and O^T += V^T P^T, V^T read transposed from the swizzled [32][D] 16-bit V tile at Vl.
-template <typename E, int D, int HPW, int F8>
+template <typename E, int D, int HPW, int F8, bool PAT = true>
 __device__ __forceinline__ void fwd_half(const Args& a, const uint16_t* Kl, const uint16_t* Vl, int ks0, int qw, int q,
                                          const u32x4 (&qf)[HPW][kQFrags<D, F8>], float (&m2)[HPW], float (&lsum)[HPW],
                                          f32x16 (&acc)[HPW][D >= 32 ? D / 32 : 1], const float* pat,
                                          EdgeOffsets eo) {
   constexpr int DB = D >= 32 ? D / 32 : 1;
   f32x16 s[HPW];
-  half_scores<E, D, HPW, F8>(a, Kl, ks0, qw, q, qf, pat, eo, s);
+  half_scores<E, D, HPW, F8, PAT>(a, Kl, ks0, qw, q, qf, pat, eo, s);
   // The softmax below is vector work; at a higher priority than the score products of a wave
   // that shares the SIMD, it issues while that wave's products wait for the matrix core (a wave
   // whose next product cannot issue otherwise holds up the other wave's vector instructions).
@@ -735,6 +736,196 @@ __global__ __launch_bounds__(256) void fwd_kernel(const Args a) {
 }
 
 // ---------------------------------------------------------------------------------------------
+// Forward with the keys of a tile split over waves (16-bit inputs), for grids whose longest tile
+// would set the time: full causal layers up to a few thousand rows, and packed batches of them.
+// A workgroup is 4 = wq x wh x KSP waves on one tile of 32 wq query rows x HPW wh query heads of a KV group:
+// wave (qi, hi, g) takes 32 rows of HPW heads and every KSP-th 32-key half, half KSP s + g in step s,
+// with the online softmax of its own halves; at the end the KSP waves of a head set merge their (maximum, sum, O)
+// through LDS, each writing out a part of O.  A workgroup runs one tile; the tiles with the most
+// keys (the last rows of the longest sequences) are dispatched first, so the slots that finish
+// early pick up the short ones.  An XCD owns whole (batch, head set)s where their number allows.
+// K/V halves are double-buffered in LDS by DMA, one step ahead.
+// ---------------------------------------------------------------------------------------------
+// ROWS: more than one row tile per workgroup (wq > 1), whose waves skip halves outside their own rows.
+//
+// Against fwd_kernel, which walks tiles with resident workgroups (register-staged key blocks, Q stashed in
+// LDS, mask patterns: 64 KB of LDS, 208 VGPRs, two workgroups per CU at D = 64): one tile per workgroup
+// needs 16 KB and 168 VGPRs, three per CU, and the dispatcher evens out the tiles' lengths.  In us, bf16,
+// D = 64, Hq = 64, Hkv = 8, full causal, KSP = 1 / 2 / 4: L = 512 17.8 / 13.0 / 11.5 (fwd_kernel 18.8);
+// L = 1024 29.7 / 23.4 / 25.0 (31.4); L = 2048 63 / 48 / 65 (69); L = 4096 152 / 160 / 206 (160); L = 8192
+// 551 / 582 / 734 (600).  KSP = 1 gives fwd_kernel's results bit for bit.
+template <typename E, int D, int HPW, int KSP, bool ROWS>
+__global__ __launch_bounds__(256, D == 128 || KSP == 4 ? 2 : 3) void fwd_split_kernel(const Args a) {
+  constexpr int KS = D / 16;
+  constexpr int DB = D >= 32 ? D / 32 : 1;
+  constexpr int TILE = 32 * D;              // a K or V half, swizzled row-major [key][d]
+  constexpr int STAGE = KSP * 2 * TILE;     // the halves of a step: K, V of each
+  constexpr int NC = HPW * DB;              // C tiles of O per wave
+  constexpr int RING = 2 * STAGE;           // 16-bit units
+  // C tiles that a wave hands over in the merge: all but its own (c % KSP == g)
+  constexpr int NM = NC < KSP ? NC : (NC / KSP) * (KSP - 1);
+  constexpr int MERGE = KSP > 1 ? 4 * NM * 16 * 64 * 2 : 0;
+  constexpr int CPR = D / 8;                // 16-byte chunks per K or V row
+  __shared__ __attribute__((aligned(16))) uint16_t lds[RING > MERGE ? RING : MERGE];
+  __shared__ float ml[KSP > 1 ? 4 * HPW * 2 * 32 : 1];  // per wave and head: maxima, sums of the 32 rows
+  const int lane = threadIdx.x & 63, r32 = lane & 31, hf = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // wave -> 32 rows, head set, key share: wq x wh x KSP
+  const int wq = ROWS ? a.wq : 1, wh = a.wh;
+  const int qi = ROWS ? wave % wq : 0, hi = wave / wq % wh, g = KSP == 1 ? 0 : wave / (wq * wh);
+  const int W = a.W, S = a.S;
+
+  // workgroup -> row tile, batch, head set (see q_stream)
+  const int gpk = a.G / (HPW * wh);
+  const QStream qs = q_stream(blockIdx.x, a.B * a.Hkv * gpk);
+  const int kvh = qs.stream / gpk / a.B, b = qs.stream / gpk % a.B;
+  const int hw = kvh * a.G + (qs.stream % gpk * wh + hi) * HPW;
+  const Seq sq = seq_of(a, b);
+  const int L = sq.L, q0 = 32 * wq * (a.n_qtiles - 1 - qs.pos), qw = q0 + 32 * qi, q = qw + r32;
+  if (q0 >= L) return;
+  const Plan32 pl = plan32(q0, 32 * wq, L, W, S);
+  const int nh = pl.nsink + (pl.we - pl.ws), n_steps = (nh + KSP - 1) / KSP;
+
+  const rsrc_t rk = make_rsrc(reinterpret_cast<const char*>(a.k) + 2 * slice_off(a.sk, b, kvh, sq.row), span_bytes(L, a.sk[2], D));
+  const rsrc_t rv = make_rsrc(reinterpret_cast<const char*>(a.v) + 2 * slice_off(a.sv, b, kvh, sq.row), span_bytes(L, a.sv[2], D));
+  const uint32_t bk = uint32_t(2 * a.sk[2]), bv = uint32_t(2 * a.sv[2]);
+  // DMA instructions of a step: D / 8 of 1 KiB per half (K, then V), shared out over the waves
+  constexpr int NI = KSP * D / 8, NIW = (NI + 3) / 4;
+  auto issue = [&](int step) {
+    uint16_t* stage = lds + (step & 1) * STAGE;
+#pragma unroll
+    for (int n = 0; n < NIW; ++n) {
+      const int ii = wave * NIW + n, half = ii / (D / 8), i = ii % (D / 8);
+      const int is_v = i >= D / 16, p = is_v ? i - D / 16 : i;
+      if (ii >= NI || step * KSP + half >= nh) continue;
+      const int pos = 64 * p + lane, row = pos / CPR, col = (pos % CPR) ^ swz<D>(row);
+      const int key = 32 * plan32_tile(pl, step * KSP + half) + row;
+      uint16_t* dst = stage + (2 * half + is_v) * TILE + 512 * p;
+      const uint32_t off = uint32_t(int64_t(key) * (is_v ? bv : bk)) + 16u * uint32_t(col);
+      if (is_v) buf_dma16(rv, dst, off);
+      else buf_dma16(rk, dst, off);
+    }
+  };
+  if (n_steps > 0) issue(0);
+
+  u32x4 qf[HPW][KS];
+#pragma unroll
+  for (int h = 0; h < HPW; ++h) {
+    const rsrc_t rq = make_rsrc(reinterpret_cast<const char*>(a.q) + 2 * slice_off(a.sq, b, hw + h, sq.row), span_bytes(L, a.sq[2], D));
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      qf[h][ks] = buf_ld16(rq, uint32_t((int64_t(q) * a.sq[2] + hf * (D / 2) + 8 * ks) * 2)) ^ a.qsign;
+  }
+  float m2[HPW], lsum[HPW];
+  f32x16 acc[HPW][DB];
+#pragma unroll
+  for (int h = 0; h < HPW; ++h) {
+    m2[h] = kNegInf;
+    lsum[h] = 0.f;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) acc[h][db] = f32x16{};
+  }
+  wait_vm_lgkm0_barrier<0>();
+  for (int s = 0; s < n_steps; ++s) {
+    if (s + 1 < n_steps) issue(s + 1);  // (into the stage that step s - 1 read, before the barrier)
+    const int i = s * KSP + g;
+    if (i < nh) {
+      const int ks0 = 32 * plan32_tile(pl, i);
+      const uint16_t* Kl = lds + (s & 1) * STAGE + 2 * g * TILE;
+      if (!ROWS || (qw < L && wave_needs(ks0, qw, L, W, S)))
+        fwd_half<E, D, HPW, 0, false>(a, Kl, Kl + TILE, ks0, qw, q, qf, m2, lsum, acc, nullptr, EdgeOffsets{-1, -1});
+    }
+    wait_vm_lgkm0_barrier<0>();
+  }
+
+  // merge the KSP waves of a head set: O C tile c = (head, 32 columns) goes to wave c % KSP
+  float lt[HPW];
+#pragma unroll
+  for (int h = 0; h < HPW; ++h) lt[h] = sum_halves(lsum[h]);
+  if constexpr (KSP > 1) {
+    float* mo = reinterpret_cast<float*>(lds);  // [wave][C tile handed over][register quad][lane] x 4
+    auto slot = [](int c, int from) { return NC < KSP ? c : c / KSP * (KSP - 1) + (c % KSP - from - 1 + KSP) % KSP; };
+    if (hf == 0) {
+#pragma unroll
+      for (int h = 0; h < HPW; ++h) {
+        ml[(wave * HPW + h) * 64 + r32] = m2[h];
+        ml[(wave * HPW + h) * 64 + 32 + r32] = lt[h];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      if (c % KSP == g) continue;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x16& x = acc[c / DB][c % DB];
+        *reinterpret_cast<f32x4*>(mo + (((wave * NM + slot(c, g)) * 4 + j) * 64 + lane) * 4) =
+            f32x4{x[4 * j], x[4 * j + 1], x[4 * j + 2], x[4 * j + 3]};
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < HPW; ++h) {
+      float mg[KSP], mt = kNegInf;
+#pragma unroll
+      for (int gg = 0; gg < KSP; ++gg) {
+        mg[gg] = ml[(((gg * wh + hi) * wq + qi) * HPW + h) * 64 + r32];
+        mt = fmaxf(mt, mg[gg]);
+      }
+      float sum = 0.f, own = 0.f, f[KSP];
+#pragma unroll
+      for (int gg = 0; gg < KSP; ++gg) {  // (a wave without an allowed key has maximum -inf and adds nothing)
+        f[gg] = mg[gg] == kNegInf ? 0.f : fast_exp2(mg[gg] - mt);
+        sum += ml[(((gg * wh + hi) * wq + qi) * HPW + h) * 64 + 32 + r32] * f[gg];
+        own = gg == g ? f[gg] : own;
+      }
+      m2[h] = mt;
+      lt[h] = sum;
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        const int c = h * DB + db;
+        if (c % KSP != g) continue;
+        acc[h][db] *= own;
+#pragma unroll
+        for (int gg = 0; gg < KSP; ++gg) {
+          if (gg == g) continue;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const f32x4 x = *reinterpret_cast<const f32x4*>(mo + (((((gg * wh + hi) * wq + qi) * NM + slot(c, gg)) * 4 + j) * 64 + lane) * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[h][db][4 * j + e] += x[e] * f[gg];
+          }
+        }
+      }
+    }
+  }
+  if (q >= L) return;
+#pragma unroll
+  for (int h = 0; h < HPW; ++h) {
+    float mt = m2[h], r = 1.f, l = lt[h];
+    if (a.sink_logits) {  // the learned sink joins the denominator (as in fwd_kernel)
+      const float sl = a.sink_logits[hw + h] * kLog2e;
+      const float mn = fmaxf(mt, sl);
+      r = fast_exp2(mt - mn);
+      l = l * r + fast_exp2(sl - mn);
+      mt = mn;
+    }
+    const float inv = l > 0.f ? r / l : 0.f;
+    char* op = reinterpret_cast<char*>(a.o_out) + 2 * slice_off(a.so_out, b, hw + h, sq.row + q);
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+      if ((h * DB + db) % KSP != g || (D == 16 && hf == 1)) continue;
+      float ov[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) ov[e] = acc[h][db][e] * inv;
+      const int d0 = 32 * db + (D >= 32 ? 16 * hf : 0);
+      st16(op + 2 * d0, pack8<E>(ov));
+      st16(op + 2 * (d0 + 8), pack8<E>(ov + 8));
+    }
+    if (hf == 0 && g == 0) a.lse_out[slice_off(a.slse, b, hw + h, sq.row + q)] = (mt + fast_log2(l)) * kLn2;
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 // Sliding forward, for the GPT-OSS sliding layers (16-bit, D = 64, KV groups of a multiple of 8
 // query heads, 1 <= W <= 129, S <= 32; the C ABI's plan_fwd_slide checks): the forward twin of
 // bwd_dq_slide_kernel (fa_bwd_slide.hip).  A workgroup is 4 waves x 2 heads -- the 8 query heads
@@ -948,35 +1139,64 @@ static int fwd_resident_per_cu() {
 template <typename E, int D, int HPW, int F8 = 0>
 static hipError_t launch_fwd_h(const Args& a, hipStream_t stream) {
   const int n_tiles = a.n_qtiles * (a.B * a.Hq / (HPW * a.wh));
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      cus < 1)
-    cus = 256;
   // one resident wave of workgroups, a multiple of the 8 XCDs
-  const int slots = fwd_resident_per_cu<fwd_kernel<E, D, HPW, F8>>() * cus;
+  const int slots = fwd_resident_per_cu<fwd_kernel<E, D, HPW, F8>>() * device_cus();
   const int wgs = 8 * ((min(n_tiles, slots) + 7) / 8);
   hipLaunchKernelGGL((fwd_kernel<E, D, HPW, F8>), dim3(wgs), dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 
-template <typename E, int D>
-static hipError_t launch_fwd_d(const Args& a, int hpw, hipStream_t stream) {
-  return hpw == 2 ? launch_fwd_h<E, D, 2>(a, stream) : launch_fwd_h<E, D, 1>(a, stream);
+template <typename E, int D, int HPW, int KSP>
+static hipError_t launch_fwd_split_k(const Args& a, hipStream_t stream) {
+  const dim3 grid(unsigned(a.n_qtiles * a.B * (a.Hq / (HPW * a.wh)))), block(256);
+  if constexpr (KSP < 4) {
+    if (a.wq > 1) {
+      hipLaunchKernelGGL((fwd_split_kernel<E, D, HPW, KSP, true>), grid, block, 0, stream, a);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((fwd_split_kernel<E, D, HPW, KSP, false>), grid, block, 0, stream, a);
+  return hipGetLastError();
+}
+
+template <typename E, int D, int HPW>
+static hipError_t launch_fwd_split_h(const Args& a, int ksp, hipStream_t stream) {
+  if (ksp == 1) return launch_fwd_split_k<E, D, HPW, 1>(a, stream);
+  if (ksp == 2) return launch_fwd_split_k<E, D, HPW, 2>(a, stream);
+  if constexpr (D < 128)  // (D = 128 would need 132 KB of LDS)
+    if (ksp == 4) return launch_fwd_split_k<E, D, HPW, 4>(a, stream);
+  return hipErrorInvalidValue;
 }
 
 template <typename E>
-static hipError_t launch_fwd_e(const Args& a, int D, int hpw, hipStream_t stream) {
+static hipError_t launch_fwd_split_e(const Args& a, int D, int hpw, int ksp, hipStream_t stream) {
   switch (D) {
-    case 16: return launch_fwd_d<E, 16>(a, hpw, stream);
-    case 32: return launch_fwd_d<E, 32>(a, hpw, stream);
-    case 64: return launch_fwd_d<E, 64>(a, hpw, stream);
-    case 128: return launch_fwd_d<E, 128>(a, hpw, stream);
+    case 16: return hpw == 2 ? launch_fwd_split_h<E, 16, 2>(a, ksp, stream) : launch_fwd_split_h<E, 16, 1>(a, ksp, stream);
+    case 32: return hpw == 2 ? launch_fwd_split_h<E, 32, 2>(a, ksp, stream) : launch_fwd_split_h<E, 32, 1>(a, ksp, stream);
+    case 64: return hpw == 2 ? launch_fwd_split_h<E, 64, 2>(a, ksp, stream) : launch_fwd_split_h<E, 64, 1>(a, ksp, stream);
+    case 128: return launch_fwd_split_h<E, 128, 1>(a, ksp, stream);
   }
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_fwd(const Args& a, int dtype, int D, int hpw, hipStream_t stream) {
-  return dtype == 1 ? launch_fwd_e<BF16>(a, D, hpw, stream) : launch_fwd_e<F16>(a, D, hpw, stream);
+hipError_t launch_fwd_split(const Args& a, int dtype, int D, int hpw, int ksp, hipStream_t stream) {
+  return dtype == 1 ? launch_fwd_split_e<BF16>(a, D, hpw, ksp, stream) : launch_fwd_split_e<F16>(a, D, hpw, ksp, stream);
+}
+
+// fwd_kernel on 16-bit inputs: the shapes that plan_fwd_split leaves to it (one head per wave; D = 64
+// never).
+template <typename E>
+static hipError_t launch_fwd_e(const Args& a, int D, hipStream_t stream) {
+  switch (D) {
+    case 16: return launch_fwd_h<E, 16, 1>(a, stream);
+    case 32: return launch_fwd_h<E, 32, 1>(a, stream);
+    case 128: return launch_fwd_h<E, 128, 1>(a, stream);
+  }
+  return hipErrorInvalidValue;
+}
+
+hipError_t launch_fwd(const Args& a, int dtype, int D, hipStream_t stream) {
+  return dtype == 1 ? launch_fwd_e<BF16>(a, D, stream) : launch_fwd_e<F16>(a, D, stream);
 }
 
 // e4m3 inputs, bf16 output: D = 64 shares K/V fragments between two heads per wave where the

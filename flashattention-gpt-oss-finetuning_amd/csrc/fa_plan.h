@@ -54,6 +54,24 @@ FA_HD QPlan qplan(int q0, int bm, int L, int W, int S) {
 
 FA_HD int qplan_block(const QPlan& p, int i) { return i < p.nsb ? i * kLdsKeys : p.ws + (i - p.nsb) * kLdsKeys; }
 
+// The same in tiles of 32 keys, for workgroups of rows [q0, q0 + bm) that visit 32-key tiles: the sink
+// tiles [0, nsink) (keys below S that lie before the window tiles), then the window tiles [ws, we).
+struct Plan32 {
+  int nsink, ws, we;
+};
+
+FA_HD Plan32 plan32(int q0, int bm, int L, int W, int S) {
+  Plan32 p;
+  const int q_end = imin(q0 + bm, L);
+  const int wlo = imax(0, q0 - W + 1);  // first key in any row's window
+  p.ws = wlo / 32;
+  p.we = q_end > wlo ? (q_end - 1) / 32 + 1 : p.ws;
+  p.nsink = (imin(S, 32 * p.ws) + 31) / 32;
+  return p;
+}
+
+FA_HD int plan32_tile(const Plan32& p, int i) { return i < p.nsink ? i : p.ws + (i - p.nsink); }
+
 // Does the wave owning rows [qw, qw + 32) need the 32 keys starting at ks0?  (Sinks, or an
 // overlap with its own window [qw - W + 1, qw + 31].)
 FA_HD bool wave_needs(int ks0, int qw, int L, int W, int S) {
