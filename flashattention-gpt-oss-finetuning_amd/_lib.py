@@ -45,6 +45,8 @@ EXPORTS = (
     "fa_bwd_sinks",
     "fa_fwd_varlen",
     "fa_bwd_varlen",
+    "fa_fwd_ranges",
+    "fa_bwd_ranges",
     "fa_fwd_fp8",
     "fa_fwd_fp8_pv",
     "fa_quantize_fp8",
@@ -151,6 +153,10 @@ def lib() -> ctypes.CDLL:
             L.fa_bwd_varlen.argtypes = [ctypes.POINTER(BwdParams), ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p,
                                         ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
             L.fa_bwd_varlen.restype = ctypes.c_int
+            L.fa_fwd_ranges.argtypes = ([ctypes.POINTER(FwdParams)] + [ctypes.c_void_p] * 2 + [ctypes.c_int32] * 2
+                                        + [ctypes.c_void_p] * 2)
+            L.fa_bwd_ranges.argtypes = ([ctypes.POINTER(BwdParams)] + [ctypes.c_void_p] * 2 + [ctypes.c_int32] * 2
+                                        + [ctypes.c_void_p] * 3 + [ctypes.c_size_t, ctypes.c_void_p])
             for fn in (L.fa_fwd_fp8, L.fa_fwd_fp8_pv):
                 fn.argtypes = [ctypes.POINTER(FwdParams), ctypes.c_float, ctypes.c_float, ctypes.c_float,
                                ctypes.c_void_p, ctypes.c_void_p]

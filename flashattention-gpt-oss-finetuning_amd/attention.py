@@ -100,9 +100,7 @@ class FlashSWDAWithSinkVarlen(torch.autograd.Function):
     def forward(ctx, q, k, v, cu_seqlens, max_seqlen, window_size, sink_size, softmax_scale=None, sinks=None):
         if softmax_scale is None:
             softmax_scale = 1.0 / math.sqrt(q.shape[-1])
-        if q.dim() != 3 or k.dim() != 3 or v.dim() != 3:
-            raise AssertionError("Packed inputs must be 3-D [total, H, D]")
-        _check_shapes(q.unsqueeze(0).transpose(1, 2), k.unsqueeze(0).transpose(1, 2), v.unsqueeze(0).transpose(1, 2))
+        _check_packed_shapes(q, k, v)
         cu, max_seqlen = _ops.cu_seqlens_ready(cu_seqlens, q.shape[0], q.device, max_seqlen)
         if window_size is None:
             window_size = max_seqlen
@@ -128,8 +126,32 @@ def flash_swda_with_sink_varlen(q, k, v, cu_seqlens, max_seqlen, window_size, si
                                 scale: Optional[float] = None, sinks=None):
     """Functional form of FlashSWDAWithSinkVarlen: packed q [total, Hq, D], k/v [total, Hkv, D],
     cu_seqlens [B + 1] (int32 or int64; on the host it is validated, on the GPU max_seqlen is
-    required), window_size None for full causal attention."""
-    return FlashSWDAWithSinkVarlen.apply(q, k, v, cu_seqlens, max_seqlen, window_size, sink_size, scale, sinks)
+    required), window_size None for full causal attention.  On GPU tensors its C++ twin (the
+    binding's swda_varlen: the same checks, kernels, saved tensors and gradients)."""
+    b = _ops.autograd_binding(q)
+    if b is None:
+        return FlashSWDAWithSinkVarlen.apply(q, k, v, cu_seqlens, max_seqlen, window_size, sink_size, scale, sinks)
+    if scale is None:
+        scale = 1.0 / math.sqrt(q.shape[-1])
+    _check_packed_shapes(q, k, v)
+    cu, max_seqlen = _ops.cu_seqlens_ready(cu_seqlens, q.shape[0], q.device, max_seqlen)
+    if window_size is None:
+        window_size = max_seqlen
+    return b.swda_varlen(q, k, v, cu, None, max_seqlen, 0, int(window_size), int(sink_size), float(scale), sinks)
+
+
+def _check_packed_shapes(q, k, v):
+    """The packed inputs' conditions: 3-D, then those of _check_shapes with the rows as the length."""
+    if q.dim() != 3 or k.dim() != 3 or v.dim() != 3:
+        raise AssertionError("Packed inputs must be 3-D [total, H, D]")
+    if not (q.shape[0] == v.shape[0] and q.shape[2] == v.shape[2]):
+        raise AssertionError("Query and Value shapes must be compatible except for num_heads")
+    if not k.shape == v.shape:
+        raise AssertionError("Key and Value shapes must be the same")
+    if not q.shape[2] <= 128:
+        raise AssertionError("Head dimension must be less than or equal to 128")
+    if not q.shape[1] % k.shape[1] == 0:
+        raise AssertionError("Number of query heads must be divisible by number of K/V heads")
 
 
 E4M3_MAX = 448.0  # largest finite float8 e4m3 (OCP) value

@@ -66,6 +66,10 @@ struct Args {
   // tensors of total_rows packed rows (L is then the longest sequence, batch strides are 0)
   const int* cu_seqlens;
   int total_rows;
+  // sequences with other rows between them: NULL, or [B] device lengths; sequence b is then rows
+  // [cu_seqlens[b], cu_seqlens[b] + seq_lens[b])
+  const int* seq_lens;
+  int token_rows;    // rows of all sequences together, at most total_rows (host-side planning)
   // Packed batches: the sliding kernels' units and the dK/dV kernel's 64-key workgroups are handed
   // out over the pieces the sequences hold (varlen_nth), so no workgroup is launched for a piece
   // past a short sequence's end.  vl_units units per (KV head, head group) and vl_kblocks key
@@ -91,8 +95,11 @@ struct Seq {
 template <typename A>
 __device__ __forceinline__ Seq seq_of(const A& a, int b) {
   if (!a.cu_seqlens) return Seq{a.L, 0};
-  int lo = a.cu_seqlens[b], hi = a.cu_seqlens[b + 1];
+  // (both loads first: their latency is paid once)
+  int lo = a.cu_seqlens[b];
+  const int e = *(a.seq_lens ? a.seq_lens + b : a.cu_seqlens + b + 1);
   lo = lo < 0 ? 0 : (lo > a.total_rows ? a.total_rows : lo);
+  int hi = !a.seq_lens ? e : e < a.total_rows - lo ? lo + e : a.total_rows;
   hi = hi < lo ? lo : (hi > a.total_rows ? a.total_rows : hi);
   const int n = hi - lo;
   return Seq{n < a.L ? n : a.L, lo};
@@ -196,12 +203,13 @@ using KArgs = const Args;
 __device__ KArgs& args_fresh();  // device code only
 #endif
 
-// Rows of a packed (variable-length) batch that belong to no sequence -- [0, cu_seqlens[0]) and
-// [cu_seqlens[B], total_rows) -- are written by no attention kernel.  varlen_tail_kernel fills
-// them in up to three outputs: every (row, head) of tensor i gets `cols[i]` elements of
-// `elem_bytes[i]` bytes (2 or 4) set to the bit pattern `fill[i]`.  Strides are in elements.
+// Rows of a packed (variable-length) batch that belong to no sequence -- before the first one, after the
+// last one and, with seq_lens, between them -- are written by no attention kernel.
+// varlen_tail_kernel fills them in up to three outputs: every (row, head) of tensor i gets `cols[i]`
+// elements of `elem_bytes[i]` bytes (2 or 4) set to the bit pattern `fill[i]`.  Strides are in elements.
 struct TailArgs {
   const int* cu_seqlens;
+  const int* seq_lens;  // NULL: as Args
   int batch, total_rows, n;
   void* ptr[3];
   int64_t head_stride[3], row_stride[3];

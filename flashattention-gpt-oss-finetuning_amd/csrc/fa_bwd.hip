@@ -1767,37 +1767,50 @@ __global__ __launch_bounds__(256) void bwd_sink_logit_kernel(const Args a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Packed rows outside every sequence (see TailArgs): one thread per (row, head) of each tensor, in
-// a grid-stride loop over the uncovered rows.  With cu_seqlens[0] = 0 and cu_seqlens[B] =
-// total_rows (the usual case) every workgroup reads two offsets and exits.
+// Packed rows outside every sequence (see TailArgs): blockIdx.y is a gap -- before the first sequence and
+// after the last one, or with seq_lens the rows before sequence y (after the last one for y = batch) --
+// and the workgroups of a gap stride over its (row, head, 16 bytes) pieces.  With cu_seqlens[0] = 0 and
+// cu_seqlens[B] = total_rows (the usual case without seq_lens) every workgroup reads two offsets and
+// exits.
 // ---------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void varlen_tail_kernel(const TailArgs t) {
-  const int total = t.total_rows;
-  int lo = t.cu_seqlens[0], hi = t.cu_seqlens[t.batch];
-  lo = lo < 0 ? 0 : (lo > total ? total : lo);
-  hi = hi < lo ? lo : (hi > total ? total : hi);
-  const int64_t n_rows = int64_t(lo) + (total - hi);  // uncovered rows, [0, lo) then [hi, total)
-  if (n_rows == 0) return;
+  const int total = t.total_rows, y = blockIdx.y;
+  auto row = [&](int x) { return x < 0 ? 0 : (x > total ? total : x); };
+  auto end_of = [&](int b) {  // of sequence b, as seq_of
+    const int lo = row(t.cu_seqlens[b]), n = t.seq_lens[b] < 0 ? 0 : t.seq_lens[b];
+    return n < total - lo ? lo + n : total;
+  };
+  int lo, hi;
+  if (t.seq_lens) {
+    lo = y == 0 ? 0 : end_of(y - 1);
+    hi = y == t.batch ? total : row(t.cu_seqlens[y]);
+  } else if (y == 0) {
+    lo = 0;
+    hi = row(t.cu_seqlens[0]);
+  } else {
+    lo = max(row(t.cu_seqlens[0]), row(t.cu_seqlens[t.batch]));
+    hi = total;
+  }
+  if (lo >= hi) return;
   const int64_t stride = int64_t(gridDim.x) * blockDim.x;
   for (int i = 0; i < t.n; ++i) {
-    const int64_t units = n_rows * t.heads[i];
+    const int eb = t.elem_bytes[i], heads = t.heads[i];
+    const int pieces = t.cols[i] * eb >= 16 ? t.cols[i] * eb / 16 : 1;  // (one column: a single 4-byte value)
+    const uint32_t f = eb == 4 ? t.fill[i] : (t.fill[i] & 0xffffu) * 0x10001u;
+    const int64_t units = int64_t(hi - lo) * heads * pieces;
     for (int64_t u = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; u < units; u += stride) {
-      const int64_t r = u / t.heads[i];
-      const int h = int(u % t.heads[i]);
-      const int64_t row = r < lo ? r : hi + (r - lo);
-      char* p = static_cast<char*>(t.ptr[i]) + (h * t.head_stride[i] + row * t.row_stride[i]) * t.elem_bytes[i];
-      if (t.elem_bytes[i] == 4) {
-        for (int c = 0; c < t.cols[i]; ++c) reinterpret_cast<uint32_t*>(p)[c] = t.fill[i];
-      } else {
-        const uint32_t f2 = (t.fill[i] & 0xffffu) * 0x10001u;
-        for (int c = 0; c < t.cols[i]; c += 8) st16(p + 2 * c, u32x4{f2, f2, f2, f2});  // rows 16-byte aligned
-      }
+      const int c = int(u % pieces), h = int(u / pieces % heads);
+      const int64_t r = lo + u / pieces / heads;
+      char* p = static_cast<char*>(t.ptr[i]) + (h * t.head_stride[i] + r * t.row_stride[i]) * eb;
+      if (t.cols[i] == 1) *reinterpret_cast<uint32_t*>(p) = f;
+      else st16(p + 16 * c, u32x4{f, f, f, f});  // (rows are 16-byte aligned)
     }
   }
 }
 
 hipError_t launch_varlen_tail(const TailArgs& t, hipStream_t stream) {
-  hipLaunchKernelGGL(varlen_tail_kernel, dim3(256), dim3(256), 0, stream, t);
+  const dim3 grid = t.seq_lens ? dim3(64, t.batch + 1) : dim3(128, 2);
+  hipLaunchKernelGGL(varlen_tail_kernel, grid, dim3(256), 0, stream, t);
   return hipGetLastError();
 }
 

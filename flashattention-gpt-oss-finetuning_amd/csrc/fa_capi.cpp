@@ -172,7 +172,7 @@ void copy3(int64_t dst[3], const int64_t src[3]) {
 
 // Tiles per unit (slide_ct) of the sliding kernels, for `slots` resident units.  A fixed-length
 // batch spreads its B Hkv (G / 8) n_qt tiles evenly over the slots.  A packed batch holds at most
-// T = ceil(total_rows / 32) + B tiles with rows (each sequence adds at most one partial tile),
+// T = ceil(token_rows / 32) + B tiles with rows (each sequence adds at most one partial tile),
 // however long its longest sequence (which sets n_qt); units past a short sequence's end exit at
 // once.  Its units cut every sequence separately, so a (KV head, head group of 8) needs about
 // T / ct + B / 2 units (half a unit lost per sequence on average), and ct is raised until those
@@ -181,7 +181,7 @@ int slide_units_ct(const fa::Args& a, int64_t slots) {
   const int64_t n_qt = (int64_t(a.L) + 31) / 32;
   const int64_t hg = int64_t(a.Hkv) * (a.G / 8);
   int64_t tiles = int64_t(a.B) * n_qt;
-  if (a.cu_seqlens) tiles = std::min(tiles, (int64_t(a.total_rows) + 31) / 32 + a.B);
+  if (a.cu_seqlens) tiles = std::min(tiles, (int64_t(a.token_rows) + 31) / 32 + a.B);
   int64_t ct = (hg * tiles + slots - 1) / slots;
   if (a.cu_seqlens) {
     const int64_t per_group = slots / hg - a.B / 2;
@@ -192,12 +192,12 @@ int slide_units_ct(const fa::Args& a, int64_t slots) {
 
 // Packed batches, the sliding kernels: units per (KV head, head group) that the sequences' rows can
 // fill -- sequence b needs ceil(ceil(L_b / 32) / ct) <= L_b / (32 ct) + 1 units, so at most
-// ceil(total_rows / (32 ct)) + B in all -- when fewer than B x slide_ncu (see fa::Args); 0 for a
+// ceil(token_rows / (32 ct)) + B in all -- when fewer than B x slide_ncu (see fa::Args); 0 for a
 // fixed-length batch.
 int vl_units(const fa::Args& a) {
   if (!a.cu_seqlens) return 0;
   const int64_t rows_ct = 32 * int64_t(a.slide_ct);
-  const int64_t bound = (int64_t(a.total_rows) + rows_ct - 1) / rows_ct + a.B;
+  const int64_t bound = (int64_t(a.token_rows) + rows_ct - 1) / rows_ct + a.B;
   return bound < int64_t(a.B) * a.slide_ncu ? int(bound) : 0;
 }
 
@@ -235,7 +235,7 @@ bool plan_fwd_slide(fa::Args& a, int D, int dtype) {
 // (each sequence adds at most one partial block), when fewer than B x n_kblocks (see fa::Args).
 int vl_kblocks(const fa::Args& a) {
   if (!a.cu_seqlens) return 0;
-  const int64_t bound = (int64_t(a.total_rows) + fa::kKvKeys - 1) / fa::kKvKeys + a.B;
+  const int64_t bound = (int64_t(a.token_rows) + fa::kKvKeys - 1) / fa::kKvKeys + a.B;
   return bound < int64_t(a.B) * a.n_kblocks ? int(bound) : 0;
 }
 
@@ -309,7 +309,7 @@ void plan_kv_split(fa::Args& a, int D, bool f32, char* ws, size_t spare) {
   a.kv_split = 1;
   const int cus = fa::device_cus();
   if (!f32 && fa::dkdv4_eligible(a, D, cus)) return;
-  const double rows = a.cu_seqlens ? std::min(double(a.L), std::max(1., double(a.total_rows) / a.B)) : double(a.L);
+  const double rows = a.cu_seqlens ? std::min(double(a.L), std::max(1., double(a.token_rows) / a.B)) : double(a.L);
   int ns = kv_split_pieces(f32, D, a.G, a.Hkv, a.B, rows, a.L, a.W, a.sink_dq != 0, cus);
   const int64_t blocks = kv_blocks(a);
   while (ns > 1 && (kv_part_bytes(D, blocks, ns) > spare || blocks * ns > (int64_t(1) << 24))) ns /= 2;
@@ -343,7 +343,7 @@ int plan_fwd_split(fa::Args& a, int D, int hpw) {
   const int di = D == 16 ? 0 : D == 32 ? 1 : D == 64 ? 2 : 3;
   if (D <= 32 && hpw == 1 && a.W <= 320) return 0;
   if (D == 128 && a.G % 2 != 0) return 0;
-  const double rows = a.cu_seqlens ? std::min(double(a.L), std::max(1., double(a.total_rows) / a.B)) : double(a.L);
+  const double rows = a.cu_seqlens ? std::min(double(a.L), std::max(1., double(a.token_rows) / a.B)) : double(a.L);
   const int cus = fa::device_cus();
   // steps of one head set's tiles over `n` rows in tiles of 32 wq, for `ksp` waves on a tile's halves
   auto steps = [&](double n, int wq, int ksp, double* longest) {
@@ -486,11 +486,18 @@ int fa_check_bwd(const fa_bwd_params* p) {
 
 namespace {
 
-// Variable-length batches: the sequences' rows are packed, so the batch strides are unused.
-int check_varlen(const int32_t* cu_seqlens, int32_t total_rows) {
-  if (!cu_seqlens) return FA_ERR_NULL;
-  if (!aligned4(cu_seqlens)) return FA_ERR_ALIGN;
-  if (total_rows < 0) return FA_ERR_SHAPE;
+// Variable-length batches: the sequences' rows lie in one row dimension, so the batch strides are unused.
+// Without `lens` sequence b is rows [cu[b], cu[b + 1]), with it [cu[b], cu[b] + lens[b]).
+struct Packed {
+  const int32_t* cu;
+  const int32_t* lens;
+  int32_t total_rows, token_rows;
+};
+
+int check_varlen(const Packed& v) {
+  if (!v.cu) return FA_ERR_NULL;
+  if (!aligned4(v.cu) || !aligned4(v.lens)) return FA_ERR_ALIGN;
+  if (v.total_rows < 0 || v.token_rows < 0 || v.token_rows > v.total_rows) return FA_ERR_SHAPE;
   return FA_OK;
 }
 
@@ -507,23 +514,25 @@ void tail_add(fa::TailArgs* t, void* ptr, const int64_t s[3], int heads, int col
   t->fill[i] = fill;
 }
 
-fa::TailArgs tail_args(const int32_t* cu_seqlens, int32_t batch, int32_t total_rows) {
+fa::TailArgs tail_args(const Packed& v, int32_t batch) {
   fa::TailArgs t;
   std::memset(&t, 0, sizeof(t));
-  t.cu_seqlens = cu_seqlens;
+  t.cu_seqlens = v.cu;
+  t.seq_lens = v.lens;
   t.batch = batch;
-  t.total_rows = total_rows;
+  t.total_rows = v.total_rows;
   return t;
 }
 
-void set_varlen(fa::Args* a, const int32_t* cu_seqlens, int32_t total_rows) {
-  a->cu_seqlens = cu_seqlens;
-  a->total_rows = total_rows;
+void set_varlen(fa::Args* a, const Packed& v) {
+  a->cu_seqlens = v.cu;
+  a->seq_lens = v.lens;
+  a->total_rows = v.total_rows;
+  a->token_rows = v.token_rows;
   for (int64_t* st : {a->sq, a->sk, a->sv, a->so, a->sdo, a->slse, a->sdq, a->sdk, a->sdv, a->so_out}) st[0] = 0;
 }
 
-int run_fwd(const fa_fwd_params* p, const float* sinks, void* stream, const int32_t* cu_seqlens = nullptr,
-            int32_t total_rows = 0) {
+int run_fwd(const fa_fwd_params* p, const float* sinks, void* stream, const Packed* packed = nullptr) {
   fa::Args a = base_args(p->batch, p->heads_q, p->heads_kv, p->seqlen, p->head_dim, p->window, p->sink,
                          p->softmax_scale);
   a.q = p->q;
@@ -537,7 +546,7 @@ int run_fwd(const fa_fwd_params* p, const float* sinks, void* stream, const int3
   copy3(a.sv, p->v_stride);
   copy3(a.so_out, p->o_stride);
   copy3(a.slse, p->lse_stride);
-  if (cu_seqlens) set_varlen(&a, cu_seqlens, total_rows);
+  if (packed) set_varlen(&a, *packed);
   if (plan_fwd_slide(a, p->head_dim, p->dtype))
     return fa::launch_fwd_slide(a, p->dtype, static_cast<hipStream_t>(stream)) == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
   const bool f32 = p->dtype == FA_DTYPE_F32;
@@ -556,6 +565,20 @@ int run_fwd(const fa_fwd_params* p, const float* sinks, void* stream, const int3
     e = fa::launch_fwd(a, p->dtype, p->head_dim, s);
   }
   return e == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
+}
+
+int fwd_packed(const fa_fwd_params* p, const Packed& v, const float* sinks, void* stream) {
+  int rc = fa_check_fwd(p);
+  if (rc == FA_OK) rc = check_varlen(v);
+  if (rc != FA_OK) return rc;
+  if (sinks && !aligned4(sinks)) return FA_ERR_ALIGN;
+  rc = run_fwd(p, sinks, stream, &v);
+  if (rc != FA_OK) return rc;
+  // rows outside every sequence: o = 0, lse = -inf (an empty row)
+  fa::TailArgs t = tail_args(v, p->batch);
+  tail_add(&t, p->o, p->o_stride, p->heads_q, p->head_dim, elem_bytes(p->dtype), 0u);
+  tail_add(&t, p->lse, p->lse_stride, p->heads_q, 1, 4, 0xff800000u);
+  return fa::launch_varlen_tail(t, static_cast<hipStream_t>(stream)) == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
 }
 
 // fa_fwd_fp8: e4m3 q, k, v (1-byte elements), bf16 o, D in {64, 128}, finite dequantisation factors.
@@ -619,17 +642,14 @@ int fa_fwd(const fa_fwd_params* p, void* stream) {
 
 int fa_fwd_varlen(const fa_fwd_params* p, const int32_t* cu_seqlens, int32_t total_rows, const float* sinks,
                   void* stream) {
-  int rc = fa_check_fwd(p);
-  if (rc == FA_OK) rc = check_varlen(cu_seqlens, total_rows);
+  return fwd_packed(p, Packed{cu_seqlens, nullptr, total_rows, total_rows}, sinks, stream);
+}
+
+int fa_fwd_ranges(const fa_fwd_params* p, const int32_t* starts, const int32_t* lens, int32_t total_rows,
+                  int32_t token_rows, const float* sinks, void* stream) {
+  const int rc = fa_check_fwd(p);
   if (rc != FA_OK) return rc;
-  if (sinks && !aligned4(sinks)) return FA_ERR_ALIGN;
-  rc = run_fwd(p, sinks, stream, cu_seqlens, total_rows);
-  if (rc != FA_OK) return rc;
-  // rows outside every sequence: o = 0, lse = -inf (an empty row)
-  fa::TailArgs t = tail_args(cu_seqlens, p->batch, total_rows);
-  tail_add(&t, p->o, p->o_stride, p->heads_q, p->head_dim, elem_bytes(p->dtype), 0u);
-  tail_add(&t, p->lse, p->lse_stride, p->heads_q, 1, 4, 0xff800000u);
-  return fa::launch_varlen_tail(t, static_cast<hipStream_t>(stream)) == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
+  return lens ? fwd_packed(p, Packed{starts, lens, total_rows, token_rows}, sinks, stream) : FA_ERR_NULL;
 }
 
 int fa_fwd_fp8(const fa_fwd_params* p, float q_descale, float k_descale, float v_descale, const float* sinks,
@@ -673,7 +693,7 @@ size_t fa_bwd_full_workspace_bytes(int32_t batch, int32_t heads_q, int32_t heads
   set_kv_plan(&a, f32);
   if (total_rows >= 0) {
     a.cu_seqlens = &total_rows;  // (only whether there are offsets matters to the plan)
-    a.total_rows = total_rows;
+    a.token_rows = total_rows;
     a.vl_kblocks = vl_kblocks(a);
   }
   plan_kv_split(a, head_dim, f32, nullptr, SIZE_MAX);
@@ -685,9 +705,9 @@ size_t fa_bwd_full_workspace_bytes(int32_t batch, int32_t heads_q, int32_t heads
 namespace {
 
 // Validates a backward call and fills the kernel arguments; returns FA_OK or an fa_status.
-// cu_seqlens: a packed batch (checked by the caller).
+// packed: a packed batch (checked by the caller).
 int prepare_bwd(const fa_bwd_params* p, void* workspace, size_t workspace_bytes, fa::Args* out, int* hpw,
-                const int32_t* cu_seqlens = nullptr, int32_t total_rows = 0) {
+                const Packed* packed = nullptr) {
   const int rc = fa_check_bwd(p);
   if (rc != FA_OK) return rc;
   const size_t need = fa_bwd_workspace_bytes(p->batch, p->heads_q, p->heads_kv, p->seqlen, p->head_dim,
@@ -731,8 +751,8 @@ int prepare_bwd(const fa_bwd_params* p, void* workspace, size_t workspace_bytes,
   set_kv_plan(&a, f32);
   if (a.sink_dq)
     a.dq_sink_part = a.partial + partial_bytes(a.B, a.Hkv, p->head_dim, sink_plan(a.L, a.W, a.S)) / sizeof(float);
-  if (cu_seqlens) {
-    set_varlen(&a, cu_seqlens, total_rows);
+  if (packed) {
+    set_varlen(&a, *packed);
     a.vl_kblocks = vl_kblocks(a);
   }
   if (!f32) plan_slide(a, p->head_dim);
@@ -752,6 +772,32 @@ int run_dkdv(const fa::Args& a, const fa_bwd_params* p, hipStream_t s) {
   const hipError_t e = p->dtype == FA_DTYPE_F32 ? fa::launch_bwd_dkdv_f32(a, p->head_dim, s)
                                                 : fa::launch_bwd_dkdv(a, p->dtype, p->head_dim, s);
   return e == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
+}
+
+int bwd_packed(const fa_bwd_params* p, const Packed& v, const float* sinks, float* dsinks, void* workspace,
+               size_t workspace_bytes, void* stream) {
+  fa::Args a;
+  int hpw = 1;
+  const int vrc = check_varlen(v);
+  int rc = prepare_bwd(p, workspace, workspace_bytes, &a, &hpw, vrc == FA_OK ? &v : nullptr);
+  if (rc == FA_OK) rc = vrc;
+  if (rc != FA_OK) return rc;
+  if (!sinks != !dsinks) return FA_ERR_NULL;
+  if ((sinks && !aligned4(sinks)) || (dsinks && !aligned4(dsinks))) return FA_ERR_ALIGN;
+  a.sink_logits = sinks;
+  a.dsink = dsinks;
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  int r = run_dq(a, p, hpw, s);
+  if (r == FA_OK && sinks) r = fa::launch_bwd_sink_logits(a, s) == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
+  if (r == FA_OK) r = run_dkdv(a, p, s);
+  if (r != FA_OK) return r;
+  // rows outside every sequence have zero gradients
+  fa::TailArgs t = tail_args(v, p->batch);
+  const int eb = elem_bytes(p->dtype);
+  tail_add(&t, p->dq, p->dq_stride, p->heads_q, p->head_dim, eb, 0u);
+  tail_add(&t, p->dk, p->dk_stride, p->heads_kv, p->head_dim, eb, 0u);
+  tail_add(&t, p->dv, p->dv_stride, p->heads_kv, p->head_dim, eb, 0u);
+  return fa::launch_varlen_tail(t, s) == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
 }
 
 }  // namespace
@@ -786,28 +832,17 @@ int fa_bwd_sinks(const fa_bwd_params* p, const float* sinks, float* dsinks, void
 
 int fa_bwd_varlen(const fa_bwd_params* p, const int32_t* cu_seqlens, int32_t total_rows, const float* sinks,
                   float* dsinks, void* workspace, size_t workspace_bytes, void* stream) {
-  fa::Args a;
-  int hpw = 1;
-  const int vrc = check_varlen(cu_seqlens, total_rows);
-  int rc = prepare_bwd(p, workspace, workspace_bytes, &a, &hpw, vrc == FA_OK ? cu_seqlens : nullptr, total_rows);
-  if (rc == FA_OK) rc = vrc;
+  return bwd_packed(p, Packed{cu_seqlens, nullptr, total_rows, total_rows}, sinks, dsinks, workspace, workspace_bytes,
+                    stream);
+}
+
+int fa_bwd_ranges(const fa_bwd_params* p, const int32_t* starts, const int32_t* lens, int32_t total_rows,
+                  int32_t token_rows, const float* sinks, float* dsinks, void* workspace, size_t workspace_bytes,
+                  void* stream) {
+  const int rc = fa_check_bwd(p);
   if (rc != FA_OK) return rc;
-  if (!sinks != !dsinks) return FA_ERR_NULL;
-  if ((sinks && !aligned4(sinks)) || (dsinks && !aligned4(dsinks))) return FA_ERR_ALIGN;
-  a.sink_logits = sinks;
-  a.dsink = dsinks;
-  const hipStream_t s = static_cast<hipStream_t>(stream);
-  int r = run_dq(a, p, hpw, s);
-  if (r == FA_OK && sinks) r = fa::launch_bwd_sink_logits(a, s) == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
-  if (r == FA_OK) r = run_dkdv(a, p, s);
-  if (r != FA_OK) return r;
-  // rows outside every sequence have zero gradients
-  fa::TailArgs t = tail_args(cu_seqlens, p->batch, total_rows);
-  const int eb = elem_bytes(p->dtype);
-  tail_add(&t, p->dq, p->dq_stride, p->heads_q, p->head_dim, eb, 0u);
-  tail_add(&t, p->dk, p->dk_stride, p->heads_kv, p->head_dim, eb, 0u);
-  tail_add(&t, p->dv, p->dv_stride, p->heads_kv, p->head_dim, eb, 0u);
-  return fa::launch_varlen_tail(t, s) == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
+  if (!lens) return FA_ERR_NULL;
+  return bwd_packed(p, Packed{starts, lens, total_rows, token_rows}, sinks, dsinks, workspace, workspace_bytes, stream);
 }
 
 int fa_bwd_dq(const fa_bwd_params* p, void* workspace, size_t workspace_bytes, void* stream) {

@@ -4,9 +4,8 @@
 // caching allocator), the current HIP stream, filling fa_fwd_params / fa_bwd_params and the
 // launch -- in C++, so a forward + backward costs a few microseconds of host time instead of
 // the tens that per-field ctypes marshalling takes.  Every FLOP still runs in libfa_gfx950.so;
-// this module only calls fa_fwd / fa_bwd / fa_fwd_sinks / fa_bwd_sinks / fa_bwd_full_workspace_bytes /
-// fa_strerror.  swda / swda_sinks are the autograd functions themselves in C++ (forward, saved
-// tensors, backward), which the functional forms of the Python package call.
+// this module only calls the C ABI.  swda / swda_sinks / swda_varlen are the autograd functions themselves
+// in C++ (forward, saved tensors, backward), which the functional forms of the Python package call.
 //
 // Error behaviour matches the ctypes path (_ops.py): tensors not on a GPU -> RuntimeError,
 // unsupported dtype or shape -> ValueError, a C ABI status -> ValueError (argument) or
@@ -31,14 +30,14 @@ int32_t dtype_code(const at::Tensor& t) {
                               "; supported dtypes are bfloat16, float16 and float32");
 }
 
-void check(const std::vector<std::pair<const at::Tensor*, const char*>>& ts) {
+void check(const std::vector<std::pair<const at::Tensor*, const char*>>& ts, bool dim4 = true) {
   const at::Tensor& first = *ts[0].first;
   if (!first.is_cuda())
     throw std::runtime_error(std::string(ts[0].second) + " is on " + first.device().str() +
                              ": the gfx950 attention kernels need GPU tensors (there is no CPU implementation)");
   dtype_code(first);
   for (const auto& [t, name] : ts) {
-    if (t->dim() != 4) throw std::invalid_argument(std::string(name) + " must be 4-D [B, H, L, D]");
+    if (dim4 && t->dim() != 4) throw std::invalid_argument(std::string(name) + " must be 4-D [B, H, L, D]");
     if (t->device() != first.device())
       throw std::runtime_error(std::string(name) + " is on " + t->device().str() + " but " + ts[0].second +
                                " is on " + first.device().str());
@@ -248,6 +247,189 @@ at::Tensor swda_sinks(const at::Tensor& q, const at::Tensor& k, const at::Tensor
   return SwdaSinksFunction::apply(q, k, v, sinks, window, sink, scale);
 }
 
+// ---- packed batches ---------------------------------------------------------------------------
+// [total, H, D] tensors on one GPU with one supported dtype, all with q's rows and head dim (the kernels
+// bound every row they touch by q's row count).
+void check_packed(const std::vector<std::pair<const at::Tensor*, const char*>>& ts) {
+  const at::Tensor& q = *ts[0].first;
+  const auto shape = [](const at::Tensor& t) {
+    std::string r = "(";
+    for (int64_t i = 0; i < t.dim(); ++i) r += (i ? ", " : "") + std::to_string(t.size(i));
+    return r + (t.dim() == 1 ? ",)" : ")");
+  };
+  for (const auto& [t, name] : ts)
+    if (t->dim() != 3)
+      throw std::invalid_argument(std::string(name) + " must be 3-D [total, H, D], got shape " + shape(*t));
+  check(ts, false);
+  for (const auto& [t, name] : ts)
+    if (t->size(0) != q.size(0) || t->size(2) != q.size(2))
+      throw std::invalid_argument(std::string(name) + " has shape " + shape(*t) + "; packed tensors need " +
+                                  std::to_string(q.size(0)) + " rows and head dim " + std::to_string(q.size(2)));
+}
+
+// A packed [total, H, D] tensor as the [1, H, total, D] view the C ABI describes (the batch stride is not
+// used there), copied where the kernels cannot read it.
+at::Tensor as_bhld(const at::Tensor& t) { return kernel_ready(t.permute({1, 0, 2}).unsqueeze(0)); }
+
+// The sequences of a packed batch: offsets [B + 1], or starts [B] with lengths.
+struct Sequences {
+  at::Tensor cu, lens;
+  int64_t max_seqlen, token_rows;
+  int64_t batch() const { return cu.size(0) - (lens.defined() ? 0 : 1); }
+  const int32_t* cu_ptr() const { return cu.data_ptr<int32_t>(); }
+  const int32_t* lens_ptr() const { return lens.defined() ? lens.data_ptr<int32_t>() : nullptr; }
+};
+
+Sequences sequences(const at::Tensor& q, const at::Tensor& cu, const at::Tensor& lens, int64_t max_seqlen,
+                    int64_t token_rows) {
+  for (const at::Tensor* t : {&cu, &lens})
+    if (t->defined() && (t->device() != q.device() || t->scalar_type() != at::kInt || t->dim() != 1 || !t->is_contiguous()))
+      throw std::invalid_argument("sequence offsets must be a contiguous 1-D int32 tensor on q's device");
+  if (cu.size(0) < (lens.defined() ? 1 : 2) || (lens.defined() && lens.size(0) != cu.size(0)))
+    throw std::invalid_argument("sequence offsets must hold at least one sequence, and as many lengths as starts");
+  return Sequences{cu, lens, max_seqlen, lens.defined() ? token_rows : q.size(0)};
+}
+
+// (o [total, Hq, D], lse float32 [Hq, total])
+std::vector<at::Tensor> fwd_packed(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const Sequences& sq,
+                                   int64_t window, int64_t sink, double scale, const at::Tensor& sinks_in) {
+  check_packed({{&q, "q"}, {&k, "k"}, {&v, "v"}});
+  const c10::DeviceGuard guard(q.device());
+  const int64_t total = q.size(0), Hq = q.size(1), D = q.size(2);
+  const at::Tensor qv = as_bhld(q), kv = as_bhld(k), vv = as_bhld(v);
+  const at::Tensor sinks = sinks_in.defined() ? sinks_ready(sinks_in, Hq, q) : at::Tensor();
+  at::Tensor o = at::empty({total, Hq, D}, q.options());
+  at::Tensor lse = at::empty({Hq, total}, q.options().dtype(at::kFloat));
+  const at::Tensor ov = o.permute({1, 0, 2}).unsqueeze(0);
+  fa_fwd_params p{};
+  p.q = qv.data_ptr();
+  p.k = kv.data_ptr();
+  p.v = vv.data_ptr();
+  p.o = o.data_ptr();
+  p.lse = lse.data_ptr<float>();
+  strides3(p.q_stride, qv);
+  strides3(p.k_stride, kv);
+  strides3(p.v_stride, vv);
+  strides3(p.o_stride, ov);
+  p.lse_stride[1] = lse.stride(0);
+  p.lse_stride[2] = lse.stride(1);
+  p.batch = clamp_i32(sq.batch());
+  p.heads_q = clamp_i32(Hq);
+  p.heads_kv = clamp_i32(k.size(1));
+  p.seqlen = clamp_i32(sq.max_seqlen);
+  p.head_dim = clamp_i32(D);
+  p.window = clamp_i32(window);
+  p.sink = clamp_i32(sink);
+  p.softmax_scale = float(scale);
+  p.dtype = dtype_code(q);
+  const float* sk = sinks.defined() ? sinks.data_ptr<float>() : nullptr;
+  if (sq.lens.defined())
+    raise_for_status(fa_fwd_ranges(&p, sq.cu_ptr(), sq.lens_ptr(), clamp_i32(total), clamp_i32(sq.token_rows), sk,
+                                   current_stream(q)),
+                     "fa_fwd_ranges");
+  else
+    raise_for_status(fa_fwd_varlen(&p, sq.cu_ptr(), clamp_i32(total), sk, current_stream(q)), "fa_fwd_varlen");
+  return {o, lse};
+}
+
+// (dq, dk, dv packed like q, k, v, and with sinks dsinks float32 [Hq])
+std::vector<at::Tensor> bwd_packed(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o,
+                                   const at::Tensor& lse, const at::Tensor& dout, const Sequences& sq, int64_t window,
+                                   int64_t sink, double scale, const at::Tensor& sinks_in) {
+  check_packed({{&q, "q"}, {&k, "k"}, {&v, "v"}, {&o, "o"}, {&dout, "do"}});
+  const c10::DeviceGuard guard(q.device());
+  const int64_t total = q.size(0), Hq = q.size(1), D = q.size(2), Hkv = k.size(1);
+  const at::Tensor qv = as_bhld(q), kv = as_bhld(k), vv = as_bhld(v), ov = as_bhld(o), dov = as_bhld(dout);
+  const at::Tensor sinks = sinks_in.defined() ? sinks_ready(sinks_in, Hq, q) : at::Tensor();
+  at::Tensor dq = at::empty({total, Hq, D}, q.options());
+  at::Tensor dk = at::empty({total, Hkv, D}, q.options());
+  at::Tensor dv = at::empty({total, Hkv, D}, q.options());
+  at::Tensor dsinks = sinks.defined() ? at::empty({Hq}, q.options().dtype(at::kFloat)) : at::Tensor();
+  fa_bwd_params p{};
+  p.q = qv.data_ptr();
+  p.k = kv.data_ptr();
+  p.v = vv.data_ptr();
+  p.o = ov.data_ptr();
+  p.dout = dov.data_ptr();
+  p.lse = lse.data_ptr<float>();
+  p.dq = dq.data_ptr();
+  p.dk = dk.data_ptr();
+  p.dv = dv.data_ptr();
+  strides3(p.q_stride, qv);
+  strides3(p.k_stride, kv);
+  strides3(p.v_stride, vv);
+  strides3(p.o_stride, ov);
+  strides3(p.do_stride, dov);
+  p.lse_stride[1] = lse.stride(0);
+  p.lse_stride[2] = lse.stride(1);
+  for (int64_t* st : {p.dq_stride, p.dk_stride, p.dv_stride}) {
+    st[1] = D;
+    st[2] = (st == p.dq_stride ? Hq : Hkv) * D;
+  }
+  p.batch = clamp_i32(sq.batch());
+  p.heads_q = clamp_i32(Hq);
+  p.heads_kv = clamp_i32(Hkv);
+  p.seqlen = clamp_i32(sq.max_seqlen);
+  p.head_dim = clamp_i32(D);
+  p.window = clamp_i32(window);
+  p.sink = clamp_i32(sink);
+  p.softmax_scale = float(scale);
+  p.dtype = dtype_code(q);
+  const size_t ws_bytes = fa_bwd_full_workspace_bytes(p.batch, p.heads_q, p.heads_kv, p.seqlen, p.head_dim, p.window,
+                                                      p.sink, p.dtype, clamp_i32(sq.token_rows));
+  at::Tensor ws = at::empty({int64_t(ws_bytes > 256 ? ws_bytes : 256)}, q.options().dtype(at::kByte));
+  const float* sk = sinks.defined() ? sinks.data_ptr<float>() : nullptr;
+  float* dsk = sinks.defined() ? dsinks.data_ptr<float>() : nullptr;
+  if (sq.lens.defined())
+    raise_for_status(fa_bwd_ranges(&p, sq.cu_ptr(), sq.lens_ptr(), clamp_i32(total), clamp_i32(sq.token_rows), sk, dsk,
+                                   ws.data_ptr(), size_t(ws.numel()), current_stream(q)),
+                     "fa_bwd_ranges");
+  else
+    raise_for_status(fa_bwd_varlen(&p, sq.cu_ptr(), clamp_i32(total), sk, dsk, ws.data_ptr(), size_t(ws.numel()),
+                                   current_stream(q)),
+                     "fa_bwd_varlen");
+  return {dq, dk, dv, dsinks};
+}
+
+// FlashSWDAWithSinkVarlen in C++: the forward saves (q, k, v, o, lse, offsets[, lengths][, sinks]), the
+// backward returns dq, dk, dv and, with sinks, d sinks in their dtype.
+struct SwdaVarlenFunction : public torch::autograd::Function<SwdaVarlenFunction> {
+  static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& q, const at::Tensor& k,
+                            const at::Tensor& v, const at::Tensor& cu, const c10::optional<at::Tensor>& lens_in,
+                            int64_t max_seqlen, int64_t token_rows, int64_t window, int64_t sink, double scale,
+                            const c10::optional<at::Tensor>& sinks_in) {
+    const at::Tensor lens = lens_in.has_value() ? *lens_in : at::Tensor();
+    const at::Tensor sinks = sinks_in.has_value() ? *sinks_in : at::Tensor();
+    std::vector<at::Tensor> r =
+        fwd_packed(q, k, v, sequences(q, cu, lens, max_seqlen, token_rows), window, sink, scale, sinks);
+    ctx->save_for_backward({q, k, v, r[0], r[1], cu, lens, sinks});
+    ctx->saved_data["max_seqlen"] = max_seqlen;
+    ctx->saved_data["token_rows"] = token_rows;
+    ctx->saved_data["window"] = window;
+    ctx->saved_data["sink"] = sink;
+    ctx->saved_data["scale"] = scale;
+    return r[0];
+  }
+
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const torch::autograd::variable_list s = ctx->get_saved_variables();
+    const Sequences sq = sequences(s[0], s[5], s[6], ctx->saved_data["max_seqlen"].toInt(),
+                                   ctx->saved_data["token_rows"].toInt());
+    std::vector<at::Tensor> g = bwd_packed(s[0], s[1], s[2], s[3], s[4], grads[0], sq, ctx->saved_data["window"].toInt(),
+                                           ctx->saved_data["sink"].toInt(), ctx->saved_data["scale"].toDouble(), s[7]);
+    const at::Tensor none;
+    return {g[0], g[1], g[2], none, none, none, none, none, none, none,
+            s[7].defined() ? g[3].to(s[7].scalar_type()) : none};
+  }
+};
+
+at::Tensor swda_varlen(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& cu,
+                       const c10::optional<at::Tensor>& lens, int64_t max_seqlen, int64_t token_rows, int64_t window,
+                       int64_t sink, double scale, const c10::optional<at::Tensor>& sinks) {
+  return SwdaVarlenFunction::apply(q, k, v, cu, lens, max_seqlen, token_rows, window, sink, scale, sinks);
+}
+
 // Per-tensor e4m3 quantisation of a GPU tensor (quantize_fp8 in attention.py): (x8, descale), x8 with x's
 // strides; without a given descale it is max |x| / 448.  The host waits for the maximum only: the codes
 // are written by a kernel behind it that reads the maximum on the device.  Returns None for tensors
@@ -289,6 +471,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("swda_sinks", &swda_sinks,
         "autograd forward with learned sink logits: (q, k, v, sinks, window, sink, scale) -> o", py::arg("q"),
         py::arg("k"), py::arg("v"), py::arg("sinks"), py::arg("window"), py::arg("sink"), py::arg("scale"));
+  m.def("swda_varlen", &swda_varlen,
+        "autograd forward of a packed batch: (q, k, v, cu_seqlens or starts, lens, max_seqlen, token_rows, window, sink, "
+        "scale, sinks=None) -> o",
+        py::arg("q"), py::arg("k"), py::arg("v"), py::arg("cu"), py::arg("lens"), py::arg("max_seqlen"),
+        py::arg("token_rows"), py::arg("window"), py::arg("sink"), py::arg("scale"), py::arg("sinks") = py::none());
   m.def("quantize_fp8", &quantize_fp8, "per-tensor e4m3 quantisation: (x, descale=None) -> (x8, descale) or None",
         py::arg("x"), py::arg("descale") = py::none());
   m.doc() = "PyTorch binding of libfa_gfx950.so (fa_fwd / fa_bwd)";

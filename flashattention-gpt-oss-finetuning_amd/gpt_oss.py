@@ -16,12 +16,14 @@ read in place, and outputs take the inputs' memory layout, so neither layout is 
 """
 from __future__ import annotations
 
+import math
 import weakref
 from typing import Optional
 
 import torch
 
-from .attention import _swda, flash_swda_with_sink_varlen
+from . import _ops
+from .attention import _check_packed_shapes, _swda, flash_swda_with_sink_varlen
 
 
 class _BatchFacts:
@@ -67,6 +69,30 @@ def _mask_facts(attention_mask: torch.Tensor):
     cu = torch.zeros(B + 1, dtype=torch.int32, device=m.device)
     cu[1:] = lens.cumsum(0)
     return False, idx, cu, int(lens.max()) if B else 0
+
+
+def _padding_facts(attention_mask: torch.Tensor):
+    """What padded_attention needs of a [B, L] padding mask: (all rows are tokens, starts, lens, longest
+    sequence, tokens, packed facts).  Where every row's tokens are contiguous (left or right padding),
+    starts and lens (int32 [B]) give their rows in the [B * L] flattening; a mask with gaps has the
+    packed facts of _mask_facts instead.  One host synchronisation, or two with gaps."""
+    m = attention_mask.to(dtype=torch.bool)
+    B, L = m.shape
+    if m.numel() == 0:
+        return True, None, None, L, 0, None
+    i = m.to(torch.int32)
+    lens = i.sum(1, dtype=torch.int32)
+    first = i.argmax(1)
+    last = L - 1 - i.flip(1).argmax(1)
+    whole = ((last - first + 1 == lens) | (lens == 0)).all()
+    full, whole, longest, tokens = torch.stack((m.all().to(torch.int64), whole.to(torch.int64), lens.max().to(torch.int64),
+                                                lens.sum())).tolist()
+    if full:
+        return True, None, None, L, tokens, None
+    if not whole:
+        return False, None, None, longest, tokens, _mask_facts(m)
+    starts = (first + L * torch.arange(B, device=m.device)).to(torch.int32)
+    return False, starts, lens, longest, tokens, None
 
 
 def _position_facts(position_ids: torch.Tensor):
@@ -123,7 +149,7 @@ def gpt_oss_attention_forward(module, query, key, value, attention_mask, dropout
         if attention_mask.dim() != 2:
             raise NotImplementedError("only the 2-D [batch, seq] padding mask of the flash-attention mask function "
                                       f"is supported, got a {attention_mask.dim()}-D mask")
-        facts = _MASK_FACTS.get(attention_mask, lambda m: _mask_facts(m.to(query.device)))
+        facts = _MASK_FACTS.get(attention_mask, lambda m: _padding_facts(m.to(query.device)))
         if not facts[0]:
             o = padded_attention(query, key, value, attention_mask, window_size=sliding_window, sinks=s_aux,
                                  scale=scaling, _facts=facts)
@@ -170,27 +196,37 @@ def _packed_row_attention(q, k, v, cu, max_len, window_size, sinks, scale):
 def padded_attention(q, k, v, attention_mask, window_size: Optional[int] = None, sinks: Optional[torch.Tensor] = None,
                      scale: Optional[float] = None, _facts=None):
     """Attention over a padded batch: q [B, Hq, L, D], k/v [B, Hkv, L, D], attention_mask [B, L]
-    (nonzero = token).  The tokens of each row are gathered, in order, into one packed batch with
-    cu_seqlens and run through flash_swda_with_sink_varlen, so causality, the window and the sinks
-    count positions from each sequence's first token (left and right padding alike; a row with
-    gaps is concatenated, as flash-attention's unpadding does).  Returns o [B, L, Hq, D] with
-    zeros at padded positions; gradients flow through the gather and scatter."""
+    (nonzero = token).  Causality, the window and the sinks count positions from each sequence's first
+    token (left and right padding alike).  Where every row's tokens are contiguous, the variable-length
+    kernels read them where they are in the [B * L] rows; a row with gaps is concatenated, as
+    flash-attention's unpadding does: the tokens are gathered, in order, into one packed batch and run
+    through flash_swda_with_sink_varlen.  Returns o [B, L, Hq, D] with zeros at padded positions, where the
+    gradients are zero too."""
     B, Hq, L, D = q.shape
     if tuple(attention_mask.shape) != (B, L):
         raise ValueError(f"attention_mask must be [B, L] = [{B}, {L}], got {tuple(attention_mask.shape)}")
     if _facts is None:
-        _facts = _mask_facts(attention_mask.to(device=q.device))
-    # token rows of the [B * L] flattening (in order), their offsets, the longest sequence
-    _, idx, cu, max_len = _facts
-    if idx is None:  # every row is a token
+        _facts = _padding_facts(attention_mask.to(device=q.device))
+    full, starts, lens, max_len, tokens, packed = _facts
+    if full:  # every row is a token
         return attention(q, k, v, window_size=window_size, sinks=sinks, scale=scale).transpose(1, 2)
     if max_len == 0:
         return q.new_zeros(B, L, Hq, D)
+    W = max_len if window_size is None else int(window_size)
+    b = _ops.autograd_binding(q)
+    if b is not None and starts is not None:
+        # contiguous tokens: the kernels read each sequence's rows where they are
+        rows = lambda x: x.transpose(1, 2).reshape(B * L, x.shape[1], D)
+        qr, kr, vr = rows(q), rows(k), rows(v)
+        _check_packed_shapes(qr, kr, vr)
+        sc = 1.0 / math.sqrt(D) if scale is None else float(scale)
+        return b.swda_varlen(qr, kr, vr, starts, lens, max_len, tokens, W, 0, sc, sinks).view(B, L, Hq, D)
+    # token rows of the [B * L] flattening (in order), their offsets
+    _, idx, cu, _ = packed if packed is not None else _mask_facts(attention_mask.to(device=q.device))
 
     def pack(x):  # [B, H, L, D] -> [tokens, H, D]
         return x.transpose(1, 2).reshape(B * L, x.shape[1], D).index_select(0, idx)
 
-    W = max_len if window_size is None else int(window_size)
     op = flash_swda_with_sink_varlen(pack(q), pack(k), pack(v), cu, max_len, W, 0, scale, sinks)
     return op.new_zeros(B * L, Hq, D).index_copy(0, idx, op).view(B, L, Hq, D)
 

@@ -212,6 +212,18 @@ int fa_fwd_varlen(const fa_fwd_params* p, const int32_t* cu_seqlens, int32_t tot
 int fa_bwd_varlen(const fa_bwd_params* p, const int32_t* cu_seqlens, int32_t total_rows, const float* sinks,
                   float* dsinks, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Variable-length batches whose sequences have other rows between them, as the padded rows of a
+ * [batch, L] batch taken as total_rows = batch * L rows: sequence b is rows [starts[b], starts[b] + lens[b])
+ * (int32 [batch] in device memory, in ascending order without overlap, no longer than p->seqlen each).
+ * token_rows is the sum of the lengths (the host plans with it; it bounds the work that is done).
+ * Everything else is as in fa_fwd_varlen / fa_bwd_varlen: rows of no sequence get o = 0, lse = -inf and
+ * zero gradients, and offsets and lengths that reach outside the tensors are cut off there. */
+int fa_fwd_ranges(const fa_fwd_params* p, const int32_t* starts, const int32_t* lens, int32_t total_rows,
+                  int32_t token_rows, const float* sinks, void* stream);
+int fa_bwd_ranges(const fa_bwd_params* p, const int32_t* starts, const int32_t* lens, int32_t total_rows,
+                  int32_t token_rows, const float* sinks, float* dsinks, void* workspace, size_t workspace_bytes,
+                  void* stream);
+
 /* Per-tensor e4m3 quantisation for the FP8 forward, over the n elements of a dense bf16, fp16 or fp32
  * tensor x: the codes of clamp(x / descale, -448, 448) to `out` (both 16-byte aligned), dividing as a
  * product with the reciprocal of descale rounded to float32.  fa_quantize_fp8_amax takes descale = max |x| / 448 (1 where
