@@ -228,6 +228,9 @@ hipError_t launch_fwd_fp8(const Args& a, int D, int hpw, bool fp8_pv, hipStream_
 // reads wq, wh (wq wh ksp = 4) and n_qtiles (tiles of 32 wq rows)
 hipError_t launch_fwd_split(const Args& a, int dtype, int D, int hpw, int ksp, hipStream_t stream);
 hipError_t launch_bwd_dq(const Args& a, int dtype, int D, int hpw, hipStream_t stream);
+// dQ with one tile per workgroup, whose keys are split over `ksp` waves: 1, 2 or 4 (D < 128); no sink rows
+// (sink_dq = 0); reads wq, wh (wq wh ksp = 4) and n_qtiles
+hipError_t launch_bwd_dq_split(const Args& a, int dtype, int D, int ksp, hipStream_t stream);
 // the sliding dQ kernel (D = 64, 16-bit, G a multiple of 8, 1 <= W <= 161, S <= 32)
 hipError_t launch_bwd_dq_slide(const Args& a, int dtype, hipStream_t stream);
 // the sliding forward (the same, W <= 129; reads slide_ct / slide_ncu)

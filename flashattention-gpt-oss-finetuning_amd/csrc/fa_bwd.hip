@@ -60,8 +60,6 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const Args a) {
   constexpr int DB = D >= 32 ? D / 32 : 1;
   constexpr int BUF = 2 * BN * D;          // K, then V, both swizzled row-major [key][d]
   constexpr int CPB = BN * D / 8;          // 16-byte chunks per 64-key block of K (or V)
-  constexpr int NK = (CPB + 255) / 256;    // chunks per thread
-  constexpr bool ALL_ON = CPB >= 256;      // every thread loads a chunk of every tile
   constexpr int NX = 8;                    // XCDs: workgroup i runs on XCD i % 8
   constexpr int TILE = 32 * D;             // one 32-row tile, swizzled row-major [row][d]
   constexpr int STASH = 3 * TILE;          // per wave: the next tile's Q, dO, O tiles
@@ -72,11 +70,11 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const Args a) {
   // Small head dims (D <= 32): a key block's compute is short next to the latency of fetching the
   // next one, so (as in the forward) every block of a tile, up to NBUF at a time, is fetched at
   // once by LDS DMA into a buffer of its own and the blocks are then computed back to back; the
-  // first tile's rows come in the same round trip.  Wider heads double-buffer (see KDMA).
+  // first tile's rows come in the same round trip.
   constexpr bool PRE = D <= 32;
-  // D >= 64: key blocks by DMA into two buffers, one block ahead (16 registers fewer than staging
-  // them through registers at D = 64, 32 at D = 128; c3 dQ 867 -> 839 us).
-  constexpr bool KDMA = D >= 64;
+  // D >= 64 (only with sink rows: see bwd_dq_split_kernel) double-buffers key blocks by DMA, one block
+  // ahead (16 registers fewer than staging them through registers at D = 64, 32 at D = 128).
+  static_assert(PRE || SINK, "without sink rows D >= 64 runs bwd_dq_split_kernel");
   // D = 128 with sink rows: the sink keys' accumulators are split over the 4 waves by head-dim
   // columns (16 registers a wave instead of 64), each wave taking every wave's rows for its 32
   // columns (sink_split below), which leaves the D = 128 key loop (see compute_block) the
@@ -164,17 +162,6 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const Args a) {
     return buf_ldf(rl, uint32_t(int64_t(t.qw + r32) * A.slse[2] * 4));
   };
 
-  // K/V staging offsets (the same for every tile)
-  uint32_t off_k[NK], off_v[NK];
-  int off_l[NK];
-#pragma unroll
-  for (int it = 0; it < NK; ++it) {
-    const int c = tid + 256 * it;
-    const int row = c / (D / 8), col = c % (D / 8);
-    off_k[it] = uint32_t((int64_t(row) * a.sk[2] + 8 * col) * 2);
-    off_v[it] = uint32_t((int64_t(row) * a.sv[2] + 8 * col) * 2);
-    off_l[it] = swz_off<D>(row, 8 * col);
-  }
   const uint32_t bk = uint32_t(2 * a.sk[2]), bv = uint32_t(2 * a.sv[2]);  // bytes per key row
 
   // sink accumulators: lane l holds key 4(l/16) + i, head-dim column 16 nb + l % 16 (SPLIT: column
@@ -215,13 +202,13 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const Args a) {
     KArgs& Akv = args_fresh();
     const rsrc_t rk = make_rsrc(reinterpret_cast<const char*>(Akv.k) + 2 * slice_off(Akv.sk, t.b, t.kvh, t.row), span_bytes(L, Akv.sk[2], D));
     const rsrc_t rv = make_rsrc(reinterpret_cast<const char*>(Akv.v) + 2 * slice_off(Akv.sv, t.b, t.kvh, t.row), span_bytes(L, Akv.sv[2], D));
-    // PRE: DMA of a 64-key block into buffer j -- the block's K and V tiles are CPB 16-byte chunks
+    // DMA of a 64-key block into buffer j -- the block's K and V tiles are CPB 16-byte chunks
     // each, 2 CPB / 64 instructions of 64 lanes; wave w issues instructions [w NIW, (w + 1) NIW),
     // and lane l of instruction p (of K or V) loads the chunk that the swizzle places at position
     // 64 p + l (as the forward's)
     constexpr int IPT = CPB / 64;
-    constexpr int NIW = (PRE || KDMA) ? 2 * IPT / 4 : 1;
-    static_assert(!(PRE || KDMA) || (NIW >= 1 && 2 * IPT == 4 * NIW), "whole DMA instructions per wave");
+    constexpr int NIW = 2 * IPT / 4;
+    static_assert((NIW >= 1 && 2 * IPT == 4 * NIW), "whole DMA instructions per wave");
     auto dma_block = [&](int kb, int j) {
 #pragma unroll
       for (int n = 0; n < NIW; ++n) {
@@ -287,27 +274,6 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const Args a) {
 #pragma unroll
     for (int db = 0; db < DB; ++db) acc[db] = f32x16{};
 
-    u32x4 kreg[NK], vreg[NK];
-    auto gload = [&](int kb) {
-#pragma unroll
-      for (int it = 0; it < NK; ++it) {
-        if (ALL_ON || tid + 256 * it < CPB) {
-          kreg[it] = buf_ld16(rk, off_k[it] + uint32_t(kb) * bk);
-          vreg[it] = buf_ld16(rv, off_v[it] + uint32_t(kb) * bv);
-        }
-      }
-    };
-    auto sstore = [&](int buf) {
-      uint16_t* Kl = lds + buf * BUF;
-      uint16_t* Vl = Kl + BN * D;
-#pragma unroll
-      for (int it = 0; it < NK; ++it) {
-        if (ALL_ON || tid + 256 * it < CPB) {
-          st16(Kl + off_l[it], kreg[it]);
-          st16(Vl + off_l[it], vreg[it]);
-        }
-      }
-    };
     // the next tile's rows into the stash, once this tile's have been read out of it (and, on
     // the sink path, after the transposed reads of its Q and dO tiles in key block 0)
     auto refill = [&]() {
@@ -518,45 +484,23 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const Args a) {
         }
         __syncthreads();  // before the buffers are refilled
       }
-    } else if constexpr (KDMA) {
+    } else {
       // block i in buffer i & 1; block i + 1's DMA is issued before block i computes (its buffer was
       // last read by block i - 1, behind the barrier that ended it) and waited for after it.  The
       // next tile's rows (refill, 3 KS + 1 loads) are issued after block 1's DMA and may stay in
       // flight past block 0's wait; later waits find them landed.
-      // D = 128 without sink rows issues the refill with block 0's DMA, one block earlier (c5
-      // without sink keys: dQ 325 -> 314 us; D = 64 measured 0.6% slower).
-      constexpr bool EARLY = !SINK && D == 128;
       if (plan.nb > 0) {
         dma_block(qplan_block(plan, 0), 0);
-        if (EARLY) refill();
-        if (EARLY && has_next) wait_vm_lgkm0_barrier<3 * KS + 1>();
-        else wait_vm_lgkm0_barrier<0>();
+        wait_vm_lgkm0_barrier<0>();
       }
       for (int i = 0; i < plan.nb; ++i) {
         const bool more = i + 1 < plan.nb;
         if (more) dma_block(qplan_block(plan, i + 1), (i + 1) & 1);
-        if (!SINK && !EARLY && i == 0) refill();
         compute_block(qplan_block(plan, i), lds + (i & 1) * BUF);
         if (SPLIT && i == 0 && tile_sink && qplan_block(plan, 0) == 0) sink_split();
-        if (SINK && i == 0) refill();
-        if (!EARLY && i == 0 && has_next) wait_vm_lgkm0_barrier<3 * KS + 1>();
+        if (i == 0) refill();
+        if (i == 0 && has_next) wait_vm_lgkm0_barrier<3 * KS + 1>();
         else wait_vm_lgkm0_barrier<0>();
-      }
-    } else {
-      if (plan.nb > 0) {  // (a tile past its sequence's end, in a variable-length batch, has none)
-        gload(qplan_block(plan, 0));
-        sstore(0);
-        __syncthreads();
-      }
-      for (int i = 0; i < plan.nb; ++i) {
-        const bool more = i + 1 < plan.nb;
-        if (more) gload(qplan_block(plan, i + 1));
-        if (!SINK && i == 0) refill();
-        compute_block(qplan_block(plan, i), lds + (i & 1) * BUF);
-        if (SPLIT && i == 0 && tile_sink && qplan_block(plan, 0) == 0) sink_split();
-        if (SINK && i == 0) refill();
-        if (more) sstore((i + 1) & 1);
-        __syncthreads();
       }
     }
     if (plan.nb == 0) refill();  // no key block (cannot happen for valid masks; kept for safety)
@@ -1727,16 +1671,11 @@ __global__ __launch_bounds__(256) void bwd_dkdv_fold_kernel(const Args a) {
   st16(dst + 2 * d0, pack8<E>(v));
 }
 
-// The D = 128 dQ and dK/dV kernels and the D = 64 dQ kernel without sink rows are instantiated in
-// fa_bwd_wide.hip, which includes this file
+// The D = 128 dQ and dK/dV kernels are instantiated in fa_bwd_wide.hip, which includes this file
 // with FA_BWD_WIDE_TU defined and is compiled with another machine scheduler; everything below
 // belongs to this translation unit only.
 #ifndef FA_BWD_WIDE_TU
-extern template __global__ void bwd_dq_kernel<BF16, 64, false>(const Args);
-extern template __global__ void bwd_dq_kernel<F16, 64, false>(const Args);
-extern template __global__ void bwd_dq_kernel<BF16, 128, false>(const Args);
 extern template __global__ void bwd_dq_kernel<BF16, 128, true>(const Args);
-extern template __global__ void bwd_dq_kernel<F16, 128, false>(const Args);
 extern template __global__ void bwd_dq_kernel<F16, 128, true>(const Args);
 extern template __global__ void bwd_dkdv_kernel<BF16, 128>(const Args);
 extern template __global__ void bwd_dkdv_kernel<F16, 128>(const Args);
@@ -1843,9 +1782,12 @@ static hipError_t launch_dq_s(const Args& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// (without sink rows, D >= 64 runs bwd_dq_split_kernel: plan_dq_split in fa_capi.cpp)
 template <typename E, int D>
 static hipError_t launch_dq_d(const Args& a, int, hipStream_t stream) {
-  return a.sink_dq ? launch_dq_s<E, D, true>(a, stream) : launch_dq_s<E, D, false>(a, stream);
+  if (a.sink_dq) return launch_dq_s<E, D, true>(a, stream);
+  if constexpr (D <= 32) return launch_dq_s<E, D, false>(a, stream);
+  return hipErrorInvalidValue;
 }
 
 // bwd_dkdv4_kernel serves 16-bit D <= 64 with KV groups of a multiple of 4 query heads, windows of

@@ -317,32 +317,15 @@ void plan_kv_split(fa::Args& a, int D, bool f32, char* ws, size_t spare) {
   a.kv_part = reinterpret_cast<float*>(ws);
 }
 
-// The 16-bit forward with one tile per workgroup (fwd_split_kernel): how many waves share a tile's keys
-// (1, 2 or 4; wq, wh and n_qtiles are set), or 0 for fwd_kernel.  The least estimated time over the
-// choices, as for the dK/dV split: the longest tile alone on its CU, or the average work of a resident
-// slot plus part of the longest tile's excess, and each workgroup's fixed time (its Q rows and first
-// keys, the merge).  In us per step of a workgroup, alone / with full slots; measured over Hq = 8 .. 64,
-// G = 1 .. 16, L = 257 .. 8192, W = 128 .. full (fwd_split_kernel's comment has the D = 64 figures; G = 1,
-// Hq = 16, L = 4096 full causal: D = 64 81 / 60 / 74 for 1 / 2 / 4 waves against 88 for fwd_kernel, D = 16
-// at L = 2048 34 / 20 / 14 against 27).
-// fwd_kernel keeps what it still does better: D <= 32 with one head per wave and short windows, whose
-// tiles' key blocks it fetches at once (the D = 16, W = 256 default case 10.9 against 12.2 us), and D = 128
-// with one head per KV group (B = 2, Hq = 32, L = 2048 full causal 81.5 against 85 us).
-int plan_fwd_split(fa::Args& a, int D, int hpw) {
-  struct Cost {
-    int per_cu;
-    double alone, full;
-  };
-  static const Cost costs[4][2][3] = {
-      // [D][heads per wave - 1][KSP = 1, 2, 4]
-      {{{7, 0.47, 1.5}, {7, 0.5, 1.5}, {7, 0.6, 1.55}}, {{4, 0.5, 1.3}, {4, 0.6, 1.4}, {4, 0.75, 1.5}}},
-      {{{5, 0.5, 1.6}, {5, 0.6, 1.6}, {4, 0.8, 1.4}}, {{4, 0.63, 1.6}, {4, 0.77, 1.6}, {4, 1.0, 1.8}}},
-      {{{4, 0.56, 1.34}, {4, 0.7, 1.38}, {2, 0.9, 1.15}}, {{3, 0.75, 1.57}, {3, 0.85, 1.72}, {2, 1.1, 1.43}}},
-      {{{2, 0.83, 1.04}, {2, 1.2, 1.3}, {0, 0, 0}}, {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}}};
-  const double fixed[3] = {3, D == 64 ? 4.5 : 3.5, 3};  // one launch's, merge included
-  const int di = D == 16 ? 0 : D == 32 ? 1 : D == 64 ? 2 : 3;
-  if (D <= 32 && hpw == 1 && a.W <= 320) return 0;
-  if (D == 128 && a.G % 2 != 0) return 0;
+// The query-major kernels with one tile per workgroup (fwd_split_kernel, bwd_dq_split_kernel): how many
+// waves share a tile's keys, KSP = 1, 2 or 4 (wq, wh and n_qtiles are set).  The least estimated time, as
+// for the dK/dV split: the longest tile alone on its CU, or the average work of a resident slot plus part
+// of the longest tile's excess, and each workgroup's fixed time (its rows, the first keys, the merge).
+struct SplitCost {
+  int per_cu;          // resident workgroups (0: not built)
+  double alone, full;  // us per step of a workgroup, alone on its CU and with full slots
+};
+int plan_split(fa::Args& a, int hpw, const SplitCost (&costs)[3], const double (&fixed)[3], double per_wg) {
   const double rows = a.cu_seqlens ? std::min(double(a.L), std::max(1., double(a.token_rows) / a.B)) : double(a.L);
   const int cus = fa::device_cus();
   // steps of one head set's tiles over `n` rows in tiles of 32 wq, for `ksp` waves on a tile's halves
@@ -356,7 +339,7 @@ int plan_fwd_split(fa::Args& a, int D, int hpw) {
   int best = 0, best_wh = 0;
   double best_t = 0;
   for (int k = 0; k < 3; ++k) {
-    const Cost& c = costs[di][hpw - 1][k];
+    const SplitCost& c = costs[k];
     if (!c.per_cu) continue;
     const int ksp = 1 << k;
     int wh = 4 / ksp;
@@ -367,8 +350,8 @@ int plan_fwd_split(fa::Args& a, int D, int hpw) {
     const double slot = c.full * streams * steps(rows, wq, ksp, &longest) / slots;
     steps(a.L, wq, ksp, &longest);  // (a packed batch's longest sequence)
     const double wgs = streams * std::ceil(rows / (32 * wq));
-    const double t = std::max(c.alone * longest, slot + 0.3 * std::max(0., c.full * longest - slot)) +
-                     fixed[k] + (hpw == 2 ? 4. : 3.) * wgs / slots;
+    const double t = std::max(c.alone * longest, slot + 0.3 * std::max(0., c.full * longest - slot)) + fixed[k] +
+                     per_wg * wgs / slots;
     if (!best || t < 0.97 * best_t) {
       best = ksp;
       best_wh = wh;
@@ -379,6 +362,39 @@ int plan_fwd_split(fa::Args& a, int D, int hpw) {
   a.wq = 4 / best / best_wh;
   a.n_qtiles = (a.L + 32 * a.wq - 1) / (32 * a.wq);
   return best;
+}
+
+// The 16-bit forward: KSP, or 0 for fwd_kernel.  The costs are measured over Hq = 8 .. 64, G = 1 .. 16,
+// L = 257 .. 8192, W = 128 .. full (fwd_split_kernel's comment has the D = 64 figures; G = 1, Hq = 16,
+// L = 4096 full causal: D = 64 81 / 60 / 74 for 1 / 2 / 4 waves against 88 for fwd_kernel, D = 16 at
+// L = 2048 34 / 20 / 14 against 27).
+// fwd_kernel keeps what it still does better: D <= 32 with one head per wave and short windows, whose
+// tiles' key blocks it fetches at once (the D = 16, W = 256 default case 10.9 against 12.2 us), and D = 128
+// with odd KV groups (one head per group, B = 2, Hq = 32, L = 2048 full causal 81.5 against 85 us).
+int plan_fwd_split(fa::Args& a, int D, int hpw) {
+  static const SplitCost costs[4][2][3] = {
+      // [D][heads per wave - 1][KSP = 1, 2, 4]
+      {{{7, 0.47, 1.5}, {7, 0.5, 1.5}, {7, 0.6, 1.55}}, {{4, 0.5, 1.3}, {4, 0.6, 1.4}, {4, 0.75, 1.5}}},
+      {{{5, 0.5, 1.6}, {5, 0.6, 1.6}, {4, 0.8, 1.4}}, {{4, 0.63, 1.6}, {4, 0.77, 1.6}, {4, 1.0, 1.8}}},
+      {{{4, 0.56, 1.34}, {4, 0.7, 1.38}, {2, 0.9, 1.15}}, {{3, 0.75, 1.57}, {3, 0.85, 1.72}, {2, 1.1, 1.43}}},
+      {{{2, 0.83, 1.04}, {2, 1.2, 1.3}, {0, 0, 0}}, {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}}};
+  const double fixed[3] = {3, D == 64 ? 4.5 : 3.5, 3};
+  if (D <= 32 && hpw == 1 && a.W <= 320) return 0;
+  if (D == 128 && a.G % 2 != 0) return 0;
+  return plan_split(a, hpw, costs[D == 16 ? 0 : D == 32 ? 1 : D == 64 ? 2 : 3][hpw - 1], fixed, hpw == 2 ? 4. : 3.);
+}
+
+// The 16-bit dQ: KSP, or 0 for the sliding kernel's shapes and for bwd_dq_kernel, which keeps the shapes
+// whose sink keys' gradients it adds up (sink_dq) and short windows at D <= 32 (D = 16, L = 4096, W = 256,
+// Hq = 16: 10.0 against 11.5 us).  Costs measured as the forward's; bwd_dq_split_kernel's comment has figures.
+int plan_dq_split(fa::Args& a, int D) {
+  static const SplitCost costs[4][3] = {{{5, 0.42, 0.98}, {5, 0.46, 1.0}, {5, 0.6, 1.05}},
+                                        {{4, 0.41, 0.93}, {4, 0.57, 1.0}, {4, 0.8, 1.15}},
+                                        {{3, 0.6, 1.115}, {3, 0.75, 1.25}, {2, 1.0, 1.06}},
+                                        {{2, 1.05, 1.42}, {2, 1.4, 1.56}, {0, 0, 0}}};
+  const double fixed[3] = {4, 4, 4};
+  if (a.sink_dq || a.dq_slide || (D <= 32 && a.W <= 320)) return 0;
+  return plan_split(a, 1, costs[D == 16 ? 0 : D == 32 ? 1 : D == 64 ? 2 : 3], fixed, D <= 32 ? 3. : 4.);
 }
 
 // The kernel arguments that describe the dK/dV kernel's key blocks and sink chunks.
@@ -762,7 +778,10 @@ int prepare_bwd(const fa_bwd_params* p, void* workspace, size_t workspace_bytes,
 }
 
 int run_dq(const fa::Args& a, const fa_bwd_params* p, int hpw, hipStream_t s) {
+  fa::Args d = a;  // (the tiles of fa_bwd_dq.hip are not those that the sink fold enumerates)
+  const int ksp = p->dtype == FA_DTYPE_F32 ? 0 : plan_dq_split(d, p->head_dim);
   const hipError_t e = p->dtype == FA_DTYPE_F32 ? fa::launch_bwd_dq_f32(a, p->head_dim, s)
+                       : ksp                ? fa::launch_bwd_dq_split(d, p->dtype, p->head_dim, ksp, s)
                        : a.dq_slide         ? fa::launch_bwd_dq_slide(a, p->dtype, s)
                                             : fa::launch_bwd_dq(a, p->dtype, p->head_dim, hpw, s);
   return e == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
