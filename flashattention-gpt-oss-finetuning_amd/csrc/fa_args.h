@@ -82,6 +82,9 @@ struct Args {
   // [64 D]; bwd_dkdv_fold_kernel adds the pieces in order.
   int kv_split;
   float* kv_part;
+  // a kernel's own workgroups are [0, main_wgs); the ones behind them do the work of fa_aux.h, tail_wgs of
+  // them on packed rows outside every sequence
+  int main_wgs, tail_wgs;
 };
 
 // Sequence b: its length and the row where it starts in the packed tensors (fixed-length
@@ -203,24 +206,11 @@ using KArgs = const Args;
 __device__ KArgs& args_fresh();  // device code only
 #endif
 
-// Rows of a packed (variable-length) batch that belong to no sequence -- before the first one, after the
-// last one and, with seq_lens, between them -- are written by no attention kernel.
-// varlen_tail_kernel fills them in up to three outputs: every (row, head) of tensor i gets `cols[i]`
-// elements of `elem_bytes[i]` bytes (2 or 4) set to the bit pattern `fill[i]`.  Strides are in elements.
-struct TailArgs {
-  const int* cu_seqlens;
-  const int* seq_lens;  // NULL: as Args
-  int batch, total_rows, n;
-  void* ptr[3];
-  int64_t head_stride[3], row_stride[3];
-  int heads[3], cols[3], elem_bytes[3];
-  uint32_t fill[3];
-};
-
 // Compute units of the current device (fa_capi.cpp).
 int device_cus();
 
-// Launchers (return the hipError_t of the launch; launch_bwd_dkdv also launches the sink fold).
+// Launchers (return the hipError_t of the launch; launch_bwd_dkdv also launches the sink fold).  The forward
+// and dK/dV launches add the workgroups of fa_aux.h.
 hipError_t launch_fwd(const Args& a, int dtype, int D, hipStream_t stream);
 // e4m3 q, k, v; bf16 o; fp8_pv: P V on the fp8 MFMA as well
 hipError_t launch_fwd_fp8(const Args& a, int D, int hpw, bool fp8_pv, hipStream_t stream);
@@ -238,8 +228,6 @@ hipError_t launch_fwd_slide(const Args& a, int dtype, hipStream_t stream);
 hipError_t launch_bwd_dkdv(const Args& a, int dtype, int D, hipStream_t stream);
 // does the 32-key dK/dV kernel serve this 16-bit backward on a device of `cus` compute units?
 bool dkdv4_eligible(const Args& a, int D, int cus);
-hipError_t launch_bwd_sink_logits(const Args& a, hipStream_t stream);  // after launch_bwd_dq
-hipError_t launch_varlen_tail(const TailArgs& t, hipStream_t stream);
 // float32 inputs (fa_f32.hip).  The dK/dV launch reads the same plan as launch_bwd_dkdv (key blocks,
 // pieces, sink blocks and their chunk workgroups) and launches the folds.
 hipError_t launch_fwd_f32(const Args& a, int D, hipStream_t stream);

@@ -23,11 +23,12 @@
 //     dQ kernel's partials to its own when its sink keys' columns fit one pass of 256 threads.
 //  3. bwd_sink_fold_kernel (when rows were chunked, or the in-kernel fold does not apply): adds
 //     the sink rows' partial sums.
-//  4. bwd_sink_logit_kernel (only with learned sink logits): adds the dQ kernel's per-row-block
-//     partials of the sink logits' gradient.
+// The gradient of learned sink logits (the sum of the dQ kernel's per-row-block partials) rides on the
+// dK/dV kernel's launch (fa_aux.h).
 #include <type_traits>
 
 #include "fa_args.h"
+#include "fa_aux.h"
 #include "fa_common.h"
 
 namespace fa {
@@ -259,7 +260,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const Args a) {
       }
       if (A.sink_logits && wave_active) {
         // learned sink: d sink = -sum over rows of P_sink * delta, P_sink = 2^(sink*log2e - lse2);
-        // one partial per 32-row block, summed in a fixed order by bwd_sink_logit_kernel
+        // one partial per 32-row block, summed in a fixed order by sum_sink_logits
         float v = q < L ? fast_exp2(A.sink_logits[t.hw] * kLog2e - lse2) * delta : 0.f;
 #pragma unroll
         for (int m = 16; m >= 1; m >>= 1) v += __shfl_xor(v, m);
@@ -718,7 +719,8 @@ __global__ __launch_bounds__(256, D == 16 ? 4 : KVL ? 3 : 1) void bwd_dkdv_kerne
   // chunks.  A group's workgroups land on one XCD (they share its L2), and the short chunk
   // workgroups run last, filling the slots that the regular ones leave.
   const int per_group = a.n_kblocks + a.nsp * a.n_chunks;
-  const int id = SPLIT ? int(blockIdx.x) : xcd_remap(blockIdx.x, gridDim.x);
+  if (int(blockIdx.x) >= a.main_wgs) return bwd_aux<D, 2>(a, reinterpret_cast<float*>(lds));
+  const int id = SPLIT ? int(blockIdx.x) : xcd_remap(blockIdx.x, a.main_wgs);
   // groups in (KV head, batch) order, the KV head outermost: the XCDs then split over KV heads
   // before sequences, which keeps their work even for sequences of different lengths.  A packed
   // batch hands out only the key blocks with keys: per KV head, each sequence's blocks
@@ -1156,7 +1158,8 @@ __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : D == 16 && NW == 4 ? 3 : 2)
 
   // workgroups grouped per (b, KV head), n_kblocks 32-key blocks each, groups in (KV head, batch)
   // order with the KV head outermost (as bwd_dkdv_kernel)
-  const int id = xcd_remap(blockIdx.x, gridDim.x);
+  if (int(blockIdx.x) >= a.main_wgs) return bwd_aux<D, 2>(a, reinterpret_cast<float*>(lds));
+  const int id = xcd_remap(blockIdx.x, a.main_wgs);
   const int grp = id / a.n_kblocks, kblk = id % a.n_kblocks;
   const int kvh = grp / a.B, b = grp % a.B;
   const Seq sq = seq_of(a, b);
@@ -1682,77 +1685,6 @@ extern template __global__ void bwd_dkdv_kernel<F16, 128>(const Args);
 extern template __global__ void bwd_dkdv_kernel<BF16, 128, false, true>(const Args);
 extern template __global__ void bwd_dkdv_kernel<F16, 128, false, true>(const Args);
 
-// ---------------------------------------------------------------------------------------------
-// Gradient of the learned sink logits: dsink[h] = sum over (b, 32-row block) of the dQ kernel's
-// partials, in a fixed order (each thread strides over the partials in order, then the waves'
-// sums are combined in wave order), so reruns are bitwise identical.  One workgroup per head.
-// ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void bwd_sink_logit_kernel(const Args a) {
-  __shared__ float wsum[4];
-  const int h = blockIdx.x, tid = threadIdx.x;
-  const int nb = a.Lp / 32;
-  const int64_t n = int64_t(a.B) * nb;
-  float acc = 0.f;
-  for (int64_t i = tid; i < n; i += 256) {
-    const int64_t b = i / nb, j = i % nb;
-    // row blocks past the end of a short sequence hold no partial
-    if (32 * j < seq_of(a, int(b)).L) acc += a.dsink_part[(b * a.Hq + h) * nb + j];
-  }
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) acc += __shfl_xor(acc, m);
-  if ((tid & 63) == 0) wsum[tid >> 6] = acc;
-  __syncthreads();
-  if (tid == 0) a.dsink[h] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
-}
-
-// ---------------------------------------------------------------------------------------------
-// Packed rows outside every sequence (see TailArgs): blockIdx.y is a gap -- before the first sequence and
-// after the last one, or with seq_lens the rows before sequence y (after the last one for y = batch) --
-// and the workgroups of a gap stride over its (row, head, 16 bytes) pieces.  With cu_seqlens[0] = 0 and
-// cu_seqlens[B] = total_rows (the usual case without seq_lens) every workgroup reads two offsets and
-// exits.
-// ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void varlen_tail_kernel(const TailArgs t) {
-  const int total = t.total_rows, y = blockIdx.y;
-  auto row = [&](int x) { return x < 0 ? 0 : (x > total ? total : x); };
-  auto end_of = [&](int b) {  // of sequence b, as seq_of
-    const int lo = row(t.cu_seqlens[b]), n = t.seq_lens[b] < 0 ? 0 : t.seq_lens[b];
-    return n < total - lo ? lo + n : total;
-  };
-  int lo, hi;
-  if (t.seq_lens) {
-    lo = y == 0 ? 0 : end_of(y - 1);
-    hi = y == t.batch ? total : row(t.cu_seqlens[y]);
-  } else if (y == 0) {
-    lo = 0;
-    hi = row(t.cu_seqlens[0]);
-  } else {
-    lo = max(row(t.cu_seqlens[0]), row(t.cu_seqlens[t.batch]));
-    hi = total;
-  }
-  if (lo >= hi) return;
-  const int64_t stride = int64_t(gridDim.x) * blockDim.x;
-  for (int i = 0; i < t.n; ++i) {
-    const int eb = t.elem_bytes[i], heads = t.heads[i];
-    const int pieces = t.cols[i] * eb >= 16 ? t.cols[i] * eb / 16 : 1;  // (one column: a single 4-byte value)
-    const uint32_t f = eb == 4 ? t.fill[i] : (t.fill[i] & 0xffffu) * 0x10001u;
-    const int64_t units = int64_t(hi - lo) * heads * pieces;
-    for (int64_t u = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; u < units; u += stride) {
-      const int c = int(u % pieces), h = int(u / pieces % heads);
-      const int64_t r = lo + u / pieces / heads;
-      char* p = static_cast<char*>(t.ptr[i]) + (h * t.head_stride[i] + r * t.row_stride[i]) * eb;
-      if (t.cols[i] == 1) *reinterpret_cast<uint32_t*>(p) = f;
-      else st16(p + 16 * c, u32x4{f, f, f, f});  // (rows are 16-byte aligned)
-    }
-  }
-}
-
-hipError_t launch_varlen_tail(const TailArgs& t, hipStream_t stream) {
-  const dim3 grid = t.seq_lens ? dim3(64, t.batch + 1) : dim3(128, 2);
-  hipLaunchKernelGGL(varlen_tail_kernel, grid, dim3(256), 0, stream, t);
-  return hipGetLastError();
-}
-
 // Resident workgroups per CU of a kernel (hipOccupancyMaxActiveBlocksPerMultiprocessor,
 // 256 threads), remembered per kernel (one cache per template argument, i.e. per kernel): it
 // depends only on the kernel's resources.
@@ -1833,7 +1765,7 @@ static hipError_t launch_dkdv_d(const Args& a, hipStream_t stream) {
   bool folded = false;
   if (a.kv_split > 1) {  // (kv_split_plan leaves dkdv4_eligible shapes alone)
     const int blocks = a.Hkv * (a.vl_kblocks ? a.vl_kblocks : a.B * a.n_kblocks);
-    hipLaunchKernelGGL((bwd_dkdv_kernel<E, D, false, true>), dim3(a.kv_split * blocks + a.n_chunk_wgs), dim3(256), 0, stream, ad);
+    hipLaunchKernelGGL((bwd_dkdv_kernel<E, D, false, true>), dim3(grid_with_aux(ad, int64_t(a.kv_split) * blocks + a.n_chunk_wgs, true)), dim3(256), 0, stream, ad);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     constexpr int kWgs = 2 * (D >= 32 ? D / 32 : 1);  // workgroups per key block
@@ -1844,35 +1776,37 @@ static hipError_t launch_dkdv_d(const Args& a, hipStream_t stream) {
       ad.n_kblocks = (a.L + 31) / 32;  // 32-key blocks
       const int grid = a.B * a.Hkv * ad.n_kblocks;
       const int nw = dkdv4_waves(a, D, grid);
+      const dim3 wgs(grid_with_aux(ad, grid, true));
       if constexpr (D == 16) {
         if (nw == 16) {
-          hipLaunchKernelGGL((bwd_dkdv4_kernel<E, D, 16>), dim3(grid), dim3(1024), 0, stream, ad);
+          hipLaunchKernelGGL((bwd_dkdv4_kernel<E, D, 16>), wgs, dim3(1024), 0, stream, ad);
           folded = dkdv4_folds_in_kernel(ad, D, dkdv4_lds_elems<D, 16>());
         }
       }
       if (nw == 8) {
-        hipLaunchKernelGGL((bwd_dkdv4_kernel<E, D, 8>), dim3(grid), dim3(512), 0, stream, ad);
+        hipLaunchKernelGGL((bwd_dkdv4_kernel<E, D, 8>), wgs, dim3(512), 0, stream, ad);
         folded = dkdv4_folds_in_kernel(ad, D, dkdv4_lds_elems<D, 8>());
       } else if (nw == 4) {
-        hipLaunchKernelGGL((bwd_dkdv4_kernel<E, D>), dim3(grid), dim3(256), 0, stream, ad);
+        hipLaunchKernelGGL((bwd_dkdv4_kernel<E, D>), wgs, dim3(256), 0, stream, ad);
         folded = dkdv4_folds_in_kernel(ad, D, dkdv4_lds_elems<D>());
       }
       e = hipGetLastError();
     } else {
       const int per_kv = a.vl_kblocks ? a.vl_kblocks : a.B * a.n_kblocks;  // regular workgroups per KV head
       const int grid = a.n_chunk_wgs + a.Hkv * per_kv;
+      const dim3 wgs(grid_with_aux(ad, grid, true));
       bool kvl = false;
       if constexpr (D == 64) kvl = dkdv_kvl_pays(a, grid);
       if constexpr (D == 64) {
-        if (kvl) hipLaunchKernelGGL((bwd_dkdv_kernel<E, D, true>), dim3(grid), dim3(256), 0, stream, ad);
+        if (kvl) hipLaunchKernelGGL((bwd_dkdv_kernel<E, D, true>), wgs, dim3(256), 0, stream, ad);
       }
-      if (!kvl) hipLaunchKernelGGL((bwd_dkdv_kernel<E, D>), dim3(grid), dim3(256), 0, stream, ad);
+      if (!kvl) hipLaunchKernelGGL((bwd_dkdv_kernel<E, D>), wgs, dim3(256), 0, stream, ad);
       e = hipGetLastError();
       folded = dkdv_folds_in_kernel(ad, D, kvl);
     }
   } else {
     const int per_kv = a.vl_kblocks ? a.vl_kblocks : a.B * a.n_kblocks;
-    hipLaunchKernelGGL((bwd_dkdv_kernel<E, D>), dim3(a.n_chunk_wgs + a.Hkv * per_kv), dim3(256), 0, stream, ad);
+    hipLaunchKernelGGL((bwd_dkdv_kernel<E, D>), dim3(grid_with_aux(ad, a.n_chunk_wgs + int64_t(a.Hkv) * per_kv, true)), dim3(256), 0, stream, ad);
     e = hipGetLastError();
     folded = dkdv_folds_in_kernel(ad, D, false);
   }
@@ -1902,10 +1836,6 @@ hipError_t launch_bwd_dq(const Args& a, int dtype, int D, int hpw, hipStream_t s
 }
 hipError_t launch_bwd_dkdv(const Args& a, int dtype, int D, hipStream_t s) {
   return dtype == 1 ? dkdv_e<BF16>(a, D, s) : dkdv_e<F16>(a, D, s);
-}
-hipError_t launch_bwd_sink_logits(const Args& a, hipStream_t s) {
-  hipLaunchKernelGGL(bwd_sink_logit_kernel, dim3(a.Hq), dim3(256), 0, s, a);
-  return hipGetLastError();
 }
 #endif  // FA_BWD_WIDE_TU
 

@@ -517,29 +517,6 @@ int check_varlen(const Packed& v) {
   return FA_OK;
 }
 
-// Adds tensor (ptr, strides s = batch/head/row, heads, cols, element bytes, fill bits) to the
-// outputs whose uncovered packed rows varlen_tail_kernel fills.
-void tail_add(fa::TailArgs* t, void* ptr, const int64_t s[3], int heads, int cols, int eb, uint32_t fill) {
-  const int i = t->n++;
-  t->ptr[i] = ptr;
-  t->head_stride[i] = s[1];
-  t->row_stride[i] = s[2];
-  t->heads[i] = heads;
-  t->cols[i] = cols;
-  t->elem_bytes[i] = eb;
-  t->fill[i] = fill;
-}
-
-fa::TailArgs tail_args(const Packed& v, int32_t batch) {
-  fa::TailArgs t;
-  std::memset(&t, 0, sizeof(t));
-  t.cu_seqlens = v.cu;
-  t.seq_lens = v.lens;
-  t.batch = batch;
-  t.total_rows = v.total_rows;
-  return t;
-}
-
 void set_varlen(fa::Args* a, const Packed& v) {
   a->cu_seqlens = v.cu;
   a->seq_lens = v.lens;
@@ -588,13 +565,7 @@ int fwd_packed(const fa_fwd_params* p, const Packed& v, const float* sinks, void
   if (rc == FA_OK) rc = check_varlen(v);
   if (rc != FA_OK) return rc;
   if (sinks && !aligned4(sinks)) return FA_ERR_ALIGN;
-  rc = run_fwd(p, sinks, stream, &v);
-  if (rc != FA_OK) return rc;
-  // rows outside every sequence: o = 0, lse = -inf (an empty row)
-  fa::TailArgs t = tail_args(v, p->batch);
-  tail_add(&t, p->o, p->o_stride, p->heads_q, p->head_dim, elem_bytes(p->dtype), 0u);
-  tail_add(&t, p->lse, p->lse_stride, p->heads_q, 1, 4, 0xff800000u);
-  return fa::launch_varlen_tail(t, static_cast<hipStream_t>(stream)) == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
+  return run_fwd(p, sinks, stream, &v);  // (rows outside every sequence: o = 0, lse = -inf, see fa_aux.h)
 }
 
 // fa_fwd_fp8: e4m3 q, k, v (1-byte elements), bf16 o, D in {64, 128}, finite dequantisation factors.
@@ -806,17 +777,8 @@ int bwd_packed(const fa_bwd_params* p, const Packed& v, const float* sinks, floa
   a.sink_logits = sinks;
   a.dsink = dsinks;
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  int r = run_dq(a, p, hpw, s);
-  if (r == FA_OK && sinks) r = fa::launch_bwd_sink_logits(a, s) == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
-  if (r == FA_OK) r = run_dkdv(a, p, s);
-  if (r != FA_OK) return r;
-  // rows outside every sequence have zero gradients
-  fa::TailArgs t = tail_args(v, p->batch);
-  const int eb = elem_bytes(p->dtype);
-  tail_add(&t, p->dq, p->dq_stride, p->heads_q, p->head_dim, eb, 0u);
-  tail_add(&t, p->dk, p->dk_stride, p->heads_kv, p->head_dim, eb, 0u);
-  tail_add(&t, p->dv, p->dv_stride, p->heads_kv, p->head_dim, eb, 0u);
-  return fa::launch_varlen_tail(t, s) == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
+  const int r = run_dq(a, p, hpw, s);
+  return r != FA_OK ? r : run_dkdv(a, p, s);  // (rows outside every sequence have zero gradients, see fa_aux.h)
 }
 
 }  // namespace
@@ -844,8 +806,7 @@ int fa_bwd_sinks(const fa_bwd_params* p, const float* sinks, float* dsinks, void
   a.sink_logits = sinks;
   a.dsink = dsinks;
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  int r = run_dq(a, p, hpw, s);
-  if (r == FA_OK) r = fa::launch_bwd_sink_logits(a, s) == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
+  const int r = run_dq(a, p, hpw, s);
   return r != FA_OK ? r : run_dkdv(a, p, s);
 }
 

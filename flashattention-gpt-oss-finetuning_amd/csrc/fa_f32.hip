@@ -31,6 +31,7 @@
 // operands of one tile row with one LDS read of DB consecutive floats, and holds 4 DB
 // consecutive outputs per four registers.
 #include "fa_args.h"
+#include "fa_aux.h"
 #include "fa_common.h"
 
 namespace fa {
@@ -171,6 +172,7 @@ __global__ __launch_bounds__(256, 2) void fwd32_kernel(const Args a) {
   constexpr int DB = kDB<D>;
   __shared__ __attribute__((aligned(16))) float lds[2 * KvTiles<D>::kBuf];
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  if (int(blockIdx.x) >= a.main_wgs) return fwd_aux<D, 4>(a);
   const QTile t = q_tile(a);
   const Seq sq = seq_of(a, t.b);
   const int L = sq.L, W = a.W, S = a.S, hq = t.hq, b = t.b, qw = t.qw;
@@ -379,6 +381,7 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void dkdv32_kernel(const Arg
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kh = wave & 1, hh = wave >> 1;
+  if (int(blockIdx.x) >= a.main_wgs) return bwd_aux<D, 4>(a, lds);
   const int W = a.W, S = a.S, G = a.G, ns = a.kv_split;
   const int per = a.vl_kblocks ? a.vl_kblocks : a.n_kblocks;
   const int streams = ns * a.Hkv * (a.vl_kblocks ? 1 : a.B);
@@ -685,7 +688,9 @@ __global__ __launch_bounds__(128) void fold32_kernel(const Args a) {
 
 template <int D>
 hipError_t fwd_d(const Args& a, hipStream_t s) {
-  hipLaunchKernelGGL(fwd32_kernel<D>, dim3(a.n_qtiles * a.B * (a.Hq / a.wh)), dim3(256), 0, s, a);
+  Args x = a;
+  const dim3 grid(grid_with_aux(x, int64_t(a.n_qtiles) * a.B * (a.Hq / a.wh), false));
+  hipLaunchKernelGGL(fwd32_kernel<D>, grid, dim3(256), 0, s, x);
   return hipGetLastError();
 }
 template <int D>
@@ -696,7 +701,9 @@ hipError_t dq_d(const Args& a, hipStream_t s) {
 template <int D>
 hipError_t dkdv_d(const Args& a, hipStream_t s) {
   const int blocks = a.Hkv * (a.vl_kblocks ? a.vl_kblocks : a.B * a.n_kblocks);
-  hipLaunchKernelGGL(dkdv32_kernel<D>, dim3(a.kv_split * blocks + a.n_chunk_wgs), dim3(256), 0, s, a);
+  Args x = a;
+  const dim3 grid(grid_with_aux(x, int64_t(a.kv_split) * blocks + a.n_chunk_wgs, true));
+  hipLaunchKernelGGL(dkdv32_kernel<D>, grid, dim3(256), 0, s, x);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && a.kv_split > 1) {
     hipLaunchKernelGGL(fold_pieces32_kernel<D>, dim3(4 * blocks), dim3(256), 0, s, a);

@@ -20,6 +20,7 @@
 //    each wave additionally skips 32-key halves outside its own rows' window.  Tiles that are
 //    fully inside the mask skip the per-element mask.
 #include "fa_args.h"
+#include "fa_aux.h"
 #include "fa_common.h"
 
 namespace fa {
@@ -400,7 +401,8 @@ __global__ __launch_bounds__(256) void fwd_kernel(const Args a) {
   // (with a fixed stride the last workgroup of an XCD got 1.66x the first's at full causal).
   const int hwg = HPW * a.wh;
   const int n_tiles = a.n_qtiles * a.B * (a.Hq / hwg);
-  const int xcd = blockIdx.x % NX, pos = blockIdx.x / NX, wgs_x = gridDim.x / NX;
+  if (int(blockIdx.x) >= a.main_wgs) return fwd_aux<D, 2>(a);
+  const int xcd = blockIdx.x % NX, pos = blockIdx.x / NX, wgs_x = a.main_wgs / NX;
   const int per = n_tiles / NX, rem = n_tiles % NX;
   const int t_lo = xcd * per + min(xcd, rem), t_hi = t_lo + per + (xcd < rem ? 1 : 0);
 
@@ -775,6 +777,7 @@ __global__ __launch_bounds__(256, D == 128 || KSP == 4 ? 2 : 3) void fwd_split_k
   const int qi = ROWS ? wave % wq : 0, hi = wave / wq % wh, g = KSP == 1 ? 0 : wave / (wq * wh);
   const int W = a.W, S = a.S;
 
+  if (int(blockIdx.x) >= a.main_wgs) return fwd_aux<D, 2>(a);
   // workgroup -> row tile, batch, head set (see q_stream)
   const int gpk = a.G / (HPW * wh);
   const QStream qs = q_stream(blockIdx.x, a.B * a.Hkv * gpk);
@@ -959,7 +962,8 @@ __global__ __launch_bounds__(256, 2) void fwd_slide_kernel(const Args a) {
   // unit -> (KV head, batch, head group, chunk), chunks fastest (as bwd_dq_slide_kernel); a packed
   // batch hands out only the chunks with rows: (KV head, head group), then each sequence's chunks
   const int hg_n = a.G / 8;
-  const int unit = xcd_remap(blockIdx.x, gridDim.x);
+  if (int(blockIdx.x) >= a.main_wgs) return fwd_aux<D, 2>(a);
+  const int unit = xcd_remap(blockIdx.x, a.main_wgs);
   int chunk, hg, b, kvh;
   if constexpr (VL) {
     const int grp = unit / a.vl_units;
@@ -1113,9 +1117,10 @@ __global__ __launch_bounds__(256, 2) void fwd_slide_kernel(const Args a) {
 template <typename E>
 static hipError_t launch_fwd_slide_e(const Args& a, hipStream_t stream) {
   const int per = a.vl_units ? a.vl_units : a.B * a.slide_ncu;  // units per (KV head, head group)
-  const dim3 grid(unsigned(a.Hkv * (a.G / 8) * per)), block(256);
-  if (a.vl_units) hipLaunchKernelGGL((fwd_slide_kernel<E, true>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((fwd_slide_kernel<E, false>), grid, block, 0, stream, a);
+  Args x = a;
+  const dim3 grid(grid_with_aux(x, int64_t(a.Hkv) * (a.G / 8) * per, false)), block(256);
+  if (a.vl_units) hipLaunchKernelGGL((fwd_slide_kernel<E, true>), grid, block, 0, stream, x);
+  else hipLaunchKernelGGL((fwd_slide_kernel<E, false>), grid, block, 0, stream, x);
   return hipGetLastError();
 }
 
@@ -1142,20 +1147,22 @@ static hipError_t launch_fwd_h(const Args& a, hipStream_t stream) {
   // one resident wave of workgroups, a multiple of the 8 XCDs
   const int slots = fwd_resident_per_cu<fwd_kernel<E, D, HPW, F8>>() * device_cus();
   const int wgs = 8 * ((min(n_tiles, slots) + 7) / 8);
-  hipLaunchKernelGGL((fwd_kernel<E, D, HPW, F8>), dim3(wgs), dim3(256), 0, stream, a);
+  Args x = a;
+  hipLaunchKernelGGL((fwd_kernel<E, D, HPW, F8>), dim3(grid_with_aux(x, wgs, false)), dim3(256), 0, stream, x);
   return hipGetLastError();
 }
 
 template <typename E, int D, int HPW, int KSP>
 static hipError_t launch_fwd_split_k(const Args& a, hipStream_t stream) {
-  const dim3 grid(unsigned(a.n_qtiles * a.B * (a.Hq / (HPW * a.wh)))), block(256);
+  Args x = a;
+  const dim3 grid(grid_with_aux(x, int64_t(a.n_qtiles) * a.B * (a.Hq / (HPW * a.wh)), false)), block(256);
   if constexpr (KSP < 4) {
     if (a.wq > 1) {
-      hipLaunchKernelGGL((fwd_split_kernel<E, D, HPW, KSP, true>), grid, block, 0, stream, a);
+      hipLaunchKernelGGL((fwd_split_kernel<E, D, HPW, KSP, true>), grid, block, 0, stream, x);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((fwd_split_kernel<E, D, HPW, KSP, false>), grid, block, 0, stream, a);
+  hipLaunchKernelGGL((fwd_split_kernel<E, D, HPW, KSP, false>), grid, block, 0, stream, x);
   return hipGetLastError();
 }
 
