@@ -1734,15 +1734,17 @@ bool dkdv4_eligible(const Args& a, int D, int cus) {
          int64_t(a.B) * a.Hkv * ((a.L + kKvKeys - 1) / kKvKeys) <= cus;
 }
 
-// The D = 64 dK/dV kernel with its K/V operands in LDS (three workgroups per CU instead of two)
-// pays on grids of many short workgroups: windows up to 512 keys and at least six workgroups per
-// CU.  Measured on MI355X (Hq = 64 or 32, D = 64): 4096 workgroups at W = 128 (L = 32768) 247
-// against 272 us, at W = 512 666 against 695 us; 2048 workgroups (B = 4, G = 4) 67 against 75 us.
-// With fewer workgroups the last, partly filled round of three per CU costs more than the extra
-// workgroup gains (1024 at W = 128: 69 against 64 us; 512: 37 against 35 us), and the long sweeps
-// of full causal attention are slower with the extra LDS reads (936 against 843 us at Hkv = 4).
+// Does the D = 64 dK/dV kernel with its K/V operands in LDS pay?  It fits three workgroups per CU instead
+// of two, each about 1.5 x 1.12 slower (it reads the operands every step), so with windows, whose
+// workgroups are equally long, it pays where it saves a round of workgroups.  dK/dV on MI355X, K/V in
+// registers / in LDS, Hq = 64, Hkv = 8, W = 128: 1024 workgroups (L = 8192) 62.6 / 66.3 us, 1256 80.7 /
+// 70.8, 1504 87.5 / 82.0, 1752 115 / 104, 2048 130 / 120, 4096 265 / 236; Hq = Hkv = 16, L = 8192, W = 256
+// (2048) 43 / 38; W = 1024, L = 16384 (2048) 590 / 587, L = 8192 (1024) 289 / 325.  The long, unequal
+// sweeps of full causal attention are slower with the extra LDS reads (936 against 843 us at Hkv = 4).
 static bool dkdv_kvl_pays(const Args& a, int grid) {
-  return a.W <= 512 && grid >= 6 * device_cus();
+  const int cus = device_cus();
+  const double in_lds = 1.12 * ((grid + 3 * cus - 1) / (3 * cus)), in_regs = (grid + 2 * cus - 1) / (2 * cus);
+  return a.W <= 1024 && a.W < a.L && in_lds < in_regs;
 }
 
 // Waves (query-head slots) per workgroup of bwd_dkdv4_kernel: its grid is at most two 32-key
