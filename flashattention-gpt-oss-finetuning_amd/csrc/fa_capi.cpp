@@ -397,8 +397,28 @@ int plan_dq_split(fa::Args& a, int D) {
   return plan_split(a, 1, costs[D == 16 ? 0 : D == 32 ? 1 : D == 64 ? 2 : 3], fixed, D <= 32 ? 3. : 4.);
 }
 
+// Where dq_sink_mode's shapes rather have the dK/dV kernel's chunk workgroups add up the sink keys'
+// gradients: rows per chunk, or 0 for the dQ kernel.  A row outside key block 0's window then costs the
+// dK/dV grid one short step per head, but the dQ kernel is bwd_dq_split_kernel, which holds no sink sums
+// and is faster per window step -- the more so the longer the window.  Whole backward in us, dQ kernel ->
+// chunks: D = 128, B = 8, Hq = 32, Hkv = 4, L = 2048, S = 16: W = 512 707 -> 649, W = 256 504 -> 456;
+// B = 1, Hq = 32, Hkv = 8, L = 4096, S = 4: W = 1024 294 -> 276, W = 256 127 -> 126, but W = 128
+// 102 -> 106.  D = 64, Hq = 64, Hkv = 8, L = 4096, S = 4: W = 1024 265 -> 254, but W = 512 157 -> 158.
+// With few heads per group a chunk has too little work (D = 64, Hq = 16, L = 4096, W = 1024: G = 1 80 -> 88,
+// G = 2 with B = 2 156.8 -> 157.7), and D <= 32 does not gain below W = 2048.  The chunks' sums lie in the room that the dQ kernel's slots have
+// (a slot per 32 rows and head set: more than a chunk's, checked all the same).
+int sinks_by_chunks(const fa::Args& a, int D, const SinkPlan& sp) {
+  if (!sp.dq || a.G < 2) return 0;
+  const int rows = D == 128 && a.W >= 256 ? 128 : D == 64 && a.W >= 1024 && a.G >= 4 ? 64 : 0;
+  if (!rows) return 0;
+  SinkPlan c = sp;
+  c.n_chunks = fa::kv_n_chunks(a.L, a.W, a.S, rows);
+  const size_t room = partial_bytes(a.B, a.Hkv, D, sp) + dq_sink_slot_bytes(a.B, a.Hq, a.Hkv, a.L, D, sp);
+  return partial_bytes(a.B, a.Hkv, D, c) <= room ? rows : 0;
+}
+
 // The kernel arguments that describe the dK/dV kernel's key blocks and sink chunks.
-void set_kv_plan(fa::Args* a, bool f32) {
+void set_kv_plan(fa::Args* a, int D, bool f32) {
   a->n_kblocks = (a->L + fa::kKvKeys - 1) / fa::kKvKeys;
   const SinkPlan sp = sink_plan(a->L, a->W, a->S);
   a->nsp = sp.nsp;
@@ -406,9 +426,10 @@ void set_kv_plan(fa::Args* a, bool f32) {
     a->chunk_rows = f32_chunk_rows(a->L, a->W, a->S);
     a->n_chunks = fa::kv_n_chunks(a->L, a->W, a->S, a->chunk_rows);
   } else {
-    a->sink_dq = sp.dq;
-    a->n_chunks = sp.n_chunks;
-    a->chunk_rows = kChunkRows;
+    const int rows = sinks_by_chunks(*a, D, sp);
+    a->sink_dq = sp.dq && !rows;
+    a->chunk_rows = rows ? rows : kChunkRows;
+    a->n_chunks = a->sink_dq ? 0 : fa::kv_n_chunks(a->L, a->W, a->S, a->chunk_rows);
     a->srows = sp.srows;
   }
   a->n_chunk_wgs = a->B * a->Hkv * a->nsp * a->n_chunks;
@@ -677,7 +698,7 @@ size_t fa_bwd_full_workspace_bytes(int32_t batch, int32_t heads_q, int32_t heads
   if (need == 0) return 0;
   const bool f32 = dtype == FA_DTYPE_F32;
   fa::Args a = base_args(batch, heads_q, heads_kv, seqlen, head_dim, window, sink, 1.f);
-  set_kv_plan(&a, f32);
+  set_kv_plan(&a, head_dim, f32);
   if (total_rows >= 0) {
     a.cu_seqlens = &total_rows;  // (only whether there are offsets matters to the plan)
     a.token_rows = total_rows;
@@ -735,7 +756,7 @@ int prepare_bwd(const fa_bwd_params* p, void* workspace, size_t workspace_bytes,
   a.dsink_part = reinterpret_cast<float*>(ws + off_dsink);
   a.partial = reinterpret_cast<float*>(ws + off_dsink + dsink_part_bytes(a.B, a.Hq, a.L));
   const bool f32 = p->dtype == FA_DTYPE_F32;
-  set_kv_plan(&a, f32);
+  set_kv_plan(&a, p->head_dim, f32);
   if (a.sink_dq)
     a.dq_sink_part = a.partial + partial_bytes(a.B, a.Hkv, p->head_dim, sink_plan(a.L, a.W, a.S)) / sizeof(float);
   if (packed) {

@@ -32,6 +32,11 @@ CASES = [
     pytest.param(1, 3, 3, 257, 128, 60, 0, FP, id="2w-D128-G1"),
     pytest.param(8, 32, 4, 700, 128, 200, 0, FP, id="1w-D128-G8"),
     pytest.param(8, 16, 16, 400, 128, 400, 0, BF, id="1w-D128-G1-row-tiles"),
+    # few sink keys whose gradients the dK/dV kernel's chunks take at these windows
+    pytest.param(1, 8, 2, 385, 128, 256, 16, BF, id="D128-sinks-in-chunks"),
+    pytest.param(2, 6, 2, 1153, 128, 300, 3, FP, id="D128-G3-sinks-in-chunks"),
+    pytest.param(1, 4, 1, 1090, 64, 1024, 1, BF, id="D64-G4-one-ragged-chunk"),
+    pytest.param(1, 16, 2, 2500, 64, 1100, 16, FP, id="D64-G8-sinks-in-chunks"),
     pytest.param(1, 6, 6, 511, 16, 511, 0, FP, id="4w-D16"),
     pytest.param(4, 16, 16, 3001, 16, 3001, 0, FP, id="D16-row-tiles"),
     pytest.param(1, 16, 1, 900, 32, 900, 0, BF, id="4w-D32"),
