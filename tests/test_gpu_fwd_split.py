@@ -41,8 +41,11 @@ CASES = [
     pytest.param(2, 64, 8, 1500, 64, 300, 4, BF, id="1w-D64-G8-window"),
     pytest.param(8, 16, 16, 1100, 64, 256, 20, BF, id="1w-D64-G1-four-row-tiles"),
     pytest.param(4, 32, 8, 1111, 64, 200, 0, FP, id="1w-D64-G4-two-row-tiles"),
-    pytest.param(8, 32, 4, 700, 128, 200, 16, FP, id="1w-D128-G8"),
-    pytest.param(8, 32, 16, 650, 128, 650, 0, BF, id="1w-D128-G2-two-row-tiles"),
+    pytest.param(8, 32, 4, 700, 128, 190, 16, FP, id="1w-D128-G8"),
+    pytest.param(8, 32, 16, 650, 128, 190, 0, BF, id="1w-D128-G2-two-row-tiles"),
+    # long windows in two rounds and more: fwd_kernel
+    pytest.param(8, 32, 4, 700, 128, 200, 16, FP, id="rounds-D128-G8"),
+    pytest.param(8, 32, 16, 650, 128, 650, 0, BF, id="rounds-D128-G2"),
     pytest.param(8, 16, 1, 1500, 32, 1500, 0, FP, id="1w-D32-G16"),
 ]
 
