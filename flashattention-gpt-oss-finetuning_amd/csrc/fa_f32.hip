@@ -23,8 +23,8 @@
 // LDS DMA, one tile ahead, and every operand is read from LDS, where it costs a small share of
 // the matrix time; the waves' own rows stay in registers.  Against one wave per workgroup with
 // operands straight from memory, in us (B = 1, Hq = 64, Hkv = 8, D = 64): L = 4096, W = 128, S = 4
-// forward 240 -> 133, dQ 338 -> 205, dK/dV 1119 -> 299; L = 2048 full causal 1007 -> 334,
-// 1390 -> 489, 4862 -> 620 (105 TFLOP/s of allowed pairs).
+// forward 240 -> 133, dQ 338 -> 205, dK/dV 1119 -> 253; L = 2048 full causal 1007 -> 334,
+// 1390 -> 489, 4862 -> 633 (109 TFLOP/s of allowed pairs).
 //
 // The head-dim order of a product whose A rows are head-dim indices (O^T, dQ^T, dV^T, dK^T) is free:
 // A row m of its C tile db (DB = D / 32 of them) stands for index DB m + db, so a lane reads the DB
@@ -40,6 +40,9 @@ namespace {
 
 __device__ __forceinline__ f32x16 mfma32(float a, float b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mfma16(float x, float y, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0);
 }
 __device__ __forceinline__ int crow(int i, int h) { return 8 * (i >> 2) + 4 * h + (i & 3); }
 __device__ __forceinline__ f32x4 ld4f(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
@@ -365,11 +368,185 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void dq32_kernel(const Args 
 // sink keys (block < nsp) go to chunk workgroups of chunk_rows rows; those and the block's own
 // workgroup write fp32 sums of its sink rows, [slot][dK, dV][S][D] per (batch, KV head), slot c for
 // chunk c and n_chunks for the block's own rows, and fold32_kernel adds them.
-// A chunk workgroup whose sink keys all lie in half 0 has its two waves of an item both take half 0
-// and half of the head-dim columns each (kh is then the column half).
+// With at most 32 sink keys the chunk workgroups are sink_chunk32's.
 // ---------------------------------------------------------------------------------------------
 template <int D>
 constexpr int kDkdv32Slot = 2 * 32 * D + 64;  // floats of an item: Q tile, dO tile, lse2[32], -delta[32]
+
+// Staging of the dK/dV kernel: wave w loads tile w of a step (item slot w / 2, Q or dO) and slot w % 2's
+// statistics (waves w and w + 2 the same bytes to the same place).
+template <int D>
+struct ItemStage {
+  static constexpr int SLOT = kDkdv32Slot<D>;
+  const float *tensor, *stats;
+  int64_t t_rs, t_hs;
+  float* lds;
+  int L, nblk, qb_lo, n_qb, n_items;
+  __device__ __forceinline__ ItemStage(const Args& a, const Seq& sq, int b, int kvh, int qb_lo, int n_qb, int n_items, float* lds)
+      : lds(lds), L(sq.L), nblk(a.Lp / 32), qb_lo(qb_lo), n_qb(n_qb), n_items(n_items) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t_do = wave & 1;
+    t_rs = t_do ? a.sdo[2] : a.sq[2];
+    t_hs = t_do ? a.sdo[1] : a.sq[1];
+    tensor = t_do ? static_cast<const float*>(a.dout) + slice_off(a.sdo, b, kvh * a.G, sq.row)
+                  : static_cast<const float*>(a.q) + slice_off(a.sq, b, kvh * a.G, sq.row);
+    stats = a.delta + (int64_t(b) * a.Hq + int64_t(kvh) * a.G) * nblk * 64;
+  }
+  __device__ __forceinline__ void operator()(int step) const {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t_slot = wave >> 1, t_do = wave & 1;
+    float* st = lds + (step & 1) * 2 * SLOT;
+    const int i = min(2 * step + t_slot, n_items - 1);  // (past the last item: loaded, not used)
+    const int g = i / n_qb, row0 = 32 * (qb_lo + i % n_qb);
+    const rsrc_t rs = slice_rsrc(tensor + g * t_hs, L, t_rs, D);
+#pragma unroll
+    for (int p = 0; p < D / 8; ++p) dma_tile<D>(rs, st + t_slot * SLOT + t_do * 32 * D, row0, t_rs, p);
+    const int i2 = min(2 * step + (wave & 1), n_items - 1);
+    const int blk = i2 / n_qb * nblk + qb_lo + i2 % n_qb;
+    buf_dma4(make_rsrc(stats + int64_t(blk) * 64, 256), reinterpret_cast<uint16_t*>(st + (wave & 1) * SLOT + 64 * D),
+             4u * (threadIdx.x & 63));
+  }
+};
+
+// A chunk's rows against all of at most 16 KB sink keys (KB = 1, 2), by 16x16x4 products: the wave's
+// matrix time is that of the keys there are, and no product is computed twice, where the 32x32x2 products
+// below work for 64 keys.  Wave (kh, hh) takes rows 16 kh .. + 15 of item hh; lane (m, g) = (lane % 16,
+// lane / 16) supplies row or key m and the head dims of 16-byte chunk 2 u + g % 2 of half row g / 2
+// to the S and dP products, holds P and dS of keys 16 x + m at rows 4 g + e, and supplies columns NT m + t
+// of those rows to dV^T += dO^T P, dK^T += Q^T dS.  Whole dK/dV, before (32x32x2 products of one 32-key
+// half, S and dP computed by two waves) -> now, us: Hq = 64, Hkv = 8, L = 4096, D = 64, W = 128: S = 4
+// 303 -> 253, S = 20 418 -> 327; D = 128, Hq = 32, L = 2048, W = 256, S = 4 259 -> 212 (part of it from the
+// registers that the regular workgroups no longer share with that path: without sinks 224 -> 216, 214 -> 195).
+// What is left of the S = 4 case's chunks, 37 us, is mostly their Q and dO (134 MB, 27 us at the rate of a copy).
+// `c` is the workgroup's place among the chunk workgroups (all of block 0).
+template <int D, int KB>
+__device__ __forceinline__ void sink_chunk32(const Args& a, int c, float* lds) {
+  constexpr int SLOT = kDkdv32Slot<D>, STAGE = 2 * SLOT, NT = D / 16;
+  static_assert(4 * 8 * NT * 64 <= 2 * STAGE, "the waves' sums of 16 keys fit the stages");
+  const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kh = wave & 1, hh = wave >> 1, S = a.S;
+  const int kvh = c / (a.B * a.n_chunks), b = c / a.n_chunks % a.B, chunk = c % a.n_chunks;
+  const Seq sq = seq_of(a, b);
+  const int lo = kv_chunk_lo(0, chunk, a.chunk_rows, sq.L, a.W), hi = kv_chunk_hi(0, chunk, a.chunk_rows, sq.L, a.W);
+  if (lo >= hi) return;  // (the fold reads no slot of it)
+  const int qb_lo = lo / 32, n_qb = (hi + 31) / 32 - qb_lo, n_items = a.G * n_qb;
+  const ItemStage<D> issue(a, sq, b, kvh, qb_lo, n_qb, n_items, lds);
+  issue(0);
+  const float c2 = a.scale * kLog2e;
+  float kf[KB][D / 4], vf[KB][D / 4];
+  f32x4 dk[KB][NT], dv[KB][NT];
+#pragma unroll
+  for (int x = 0; x < KB; ++x) {
+    const int key = 16 * x + m, d0 = (g >> 1) * (D / 2) + 4 * (g & 1);
+    const float* K = static_cast<const float*>(a.k) + slice_off(a.sk, b, kvh, sq.row) + int64_t(key) * a.sk[2] + d0;
+    const float* V = static_cast<const float*>(a.v) + slice_off(a.sv, b, kvh, sq.row) + int64_t(key) * a.sv[2] + d0;
+#pragma unroll
+    for (int u = 0; u < D / 16; ++u) {
+      const f32x4 kx = key < S ? ld4f(K + 8 * u) : f32x4{}, vx = key < S ? ld4f(V + 8 * u) : f32x4{};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        kf[x][4 * u + j] = kx[j] * c2;
+        vf[x][4 * u + j] = vx[j];
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      dk[x][t] = f32x4{};
+      dv[x][t] = f32x4{};
+    }
+  }
+  auto cols16 = [&](const float* t, int row, float (&out)[NT]) {  // columns NT m .. NT m + NT - 1
+    if constexpr (NT >= 4) {
+#pragma unroll
+      for (int i = 0; i < NT / 4; ++i) {
+        const f32x4 x = ld4f(t + row * D + 4 * ((NT / 4 * m + i) ^ swz32<D>(row)));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[4 * i + e] = x[e];
+      }
+    } else {
+      const float* p = t + row * D + 4 * ((NT * m >> 2) ^ swz32<D>(row)) + (NT * m & 3);
+#pragma unroll
+      for (int e = 0; e < NT; ++e) out[e] = p[e];
+    }
+  };
+  const int steps = (n_items + 1) / 2;
+  for (int s = 0; s < steps; ++s) {
+    wait_vm_lgkm0_barrier<0>();  // step s has landed, and nobody reads the other stage any more
+    if (s + 1 < steps) issue(s + 1);
+    const int i = 2 * s + hh;
+    const int r0 = 32 * (qb_lo + i % n_qb) + 16 * kh;  // this wave's first row
+    if (!(i < n_items && r0 + 16 > lo && r0 < hi)) continue;
+    const float* Qt = lds + (s & 1) * STAGE + hh * SLOT;
+    const float* Dt = Qt + 32 * D;
+    const float* st = Qt + 64 * D + 16 * kh + 4 * g;
+    f32x4 sc[KB], dp[KB];
+#pragma unroll
+    for (int x = 0; x < KB; ++x) {
+      sc[x] = f32x4{};
+      dp[x] = ld4f(st + 32);
+    }
+#pragma unroll
+    for (int u = 0; u < D / 16; ++u) {
+      const f32x4 qa = tile_half<D>(Qt, 16 * kh + m, g >> 1, 2 * u + (g & 1));
+      const f32x4 da = tile_half<D>(Dt, 16 * kh + m, g >> 1, 2 * u + (g & 1));
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int x = 0; x < KB; ++x) {
+          sc[x] = mfma16(qa[j], kf[x][4 * u + j], sc[x]);
+          dp[x] = mfma16(da[j], vf[x][4 * u + j], dp[x]);
+        }
+    }
+    const f32x4 l4 = ld4f(st);
+    float p[KB][4], ds[KB][4];
+#pragma unroll
+    for (int x = 0; x < KB; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool on = 16 * x + m < S && unsigned(r0 + 4 * g + e - lo) < unsigned(hi - lo);
+        p[x][e] = on ? exp2f(sc[x][e] - l4[e]) : 0.f;
+        ds[x][e] = p[x][e] * dp[x][e];
+      }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float oa[NT], qa[NT];
+      cols16(Dt, 16 * kh + 4 * g + e, oa);
+      cols16(Qt, 16 * kh + 4 * g + e, qa);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int x = 0; x < KB; ++x) {
+          dv[x][t] = mfma16(oa[t], p[x][e], dv[x][t]);
+          dk[x][t] = mfma16(qa[t], ds[x][e], dk[x][t]);
+        }
+    }
+  }
+  // the four waves' sums, 16 keys at a time, in order; wave w adds and stores rows [2 NT w, 2 NT (w + 1))
+  // of the 8 NT [dK, dV][t][e]
+#pragma unroll
+  for (int x = 0; x < KB; ++x) {
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        lds[((wave * 2 * NT + t) * 4 + e) * 64 + lane] = dk[x][t][e];
+        lds[((wave * 2 * NT + NT + t) * 4 + e) * 64 + lane] = dv[x][t][e];
+      }
+    __syncthreads();
+    if (16 * x + m < S) {
+      float* out = a.partial + ((int64_t(b) * a.Hkv + kvh) * (a.n_chunks + 1) + chunk) * 2 * S * D + (16 * x + m) * D;
+#pragma unroll
+      for (int y = 0; y < 2 * NT; ++y) {
+        const int row = 2 * NT * wave + y, t = row / 4 % NT, e = row % 4;
+        float v = lds[row * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) v += lds[(w * 8 * NT + row) * 64 + lane];
+        out[(row / (4 * NT)) * S * D + NT * (4 * g + e) + t] = v;
+      }
+    }
+  }
+}
 
 template <int D>
 __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void dkdv32_kernel(const Args a) {
@@ -402,6 +579,8 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void dkdv32_kernel(const Arg
     }
   } else {
     const int n_cw = a.nsp * a.n_chunks, c = id - streams * per;
+    if (S <= 16) return sink_chunk32<D, 1>(a, c, lds);
+    if (S <= 32) return sink_chunk32<D, 2>(a, c, lds);
     kvh = c / (a.B * n_cw);
     b = c / n_cw % a.B;
     kblk = c % n_cw % a.nsp;
@@ -420,8 +599,7 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void dkdv32_kernel(const Arg
     lo = kKvKeys * kblk;
     hi = kv_window_end(kblk, L, W);  // > lo
   }
-  const bool col_split = DB >= 2 && is_chunk && S <= kKvKeys * kblk + 32;
-  const int ks0 = kKvKeys * kblk + (col_split ? 0 : 32 * kh);  // this wave's keys
+  const int ks0 = kKvKeys * kblk + 32 * kh;  // this wave's keys
   const int key = ks0 + r;
   const bool wave_on = ks0 < L && (!is_chunk || ks0 < S);
   const int wlo = is_chunk ? lo : max(lo, ks0);
@@ -435,25 +613,7 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void dkdv32_kernel(const Arg
     s_hi = int(int64_t(all_steps) * (piece + 1) / ns);
   }
 
-  // staging: wave w loads tile w of a step (item slot w / 2, Q or dO) and slot w % 2's statistics (waves
-  // w and w + 2 the same bytes to the same place)
-  const int t_slot = wave >> 1, t_do = wave & 1;
-  const int64_t t_rs = t_do ? a.sdo[2] : a.sq[2], t_hs = t_do ? a.sdo[1] : a.sq[1];
-  const float* tensor = t_do ? static_cast<const float*>(a.dout) + slice_off(a.sdo, b, kvh * G, sq.row)
-                             : static_cast<const float*>(a.q) + slice_off(a.sq, b, kvh * G, sq.row);
-  const int nblk = a.Lp / 32;
-  const float* stats = a.delta + (int64_t(b) * a.Hq + int64_t(kvh) * G) * nblk * 64;
-  auto issue = [&](int step) {
-    float* st = lds + (step & 1) * STAGE;
-    const int i = min(2 * step + t_slot, n_items - 1);  // (past the last item: loaded, not used)
-    const int g = i / n_qb, row0 = 32 * (qb_lo + i % n_qb);
-    const rsrc_t rs = slice_rsrc(tensor + g * t_hs, L, t_rs, D);
-#pragma unroll
-    for (int p = 0; p < D / 8; ++p) dma_tile<D>(rs, st + t_slot * SLOT + t_do * 32 * D, row0, t_rs, p);
-    const int i2 = min(2 * step + (wave & 1), n_items - 1);
-    const int blk = i2 / n_qb * nblk + qb_lo + i2 % n_qb;
-    buf_dma4(make_rsrc(stats + int64_t(blk) * 64, 256), reinterpret_cast<uint16_t*>(st + (wave & 1) * SLOT + 64 * D), 4u * lane);
-  };
+  const ItemStage<D> issue(a, sq, b, kvh, qb_lo, n_qb, n_items, lds);
   if (s_lo < s_hi) issue(s_lo);
 
   const float c2 = a.scale * kLog2e;
@@ -516,30 +676,15 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void dkdv32_kernel(const Arg
       }
     }
     // dV^T += dO^T P and dK^T += Q^T dS: lane (r, h) supplies dO / Q[qr0 + crow(t, h)][DB r + db]
-    if (col_split) {
 #pragma unroll
-      for (int x = 0; x < 16; ++x) {
-        float oa[DB], qa[DB];
-        tile_cols<D>(Dt, crow(x, h), r, oa);
-        tile_cols<D>(Qt, crow(x, h), r, qa);
-        // this wave's half of the column tiles, in the accumulators of the first half
+    for (int x = 0; x < 16; ++x) {
+      float oa[DB], qa[DB];
+      tile_cols<D>(Dt, crow(x, h), r, oa);
+      tile_cols<D>(Qt, crow(x, h), r, qa);
 #pragma unroll
-        for (int db = 0; db < DB / 2; ++db) {
-          dv[db] = mfma32(kh ? oa[DB / 2 + db] : oa[db], p[x], dv[db]);
-          dk[db] = mfma32(kh ? qa[DB / 2 + db] : qa[db], ds[x], dk[db]);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int x = 0; x < 16; ++x) {
-        float oa[DB], qa[DB];
-        tile_cols<D>(Dt, crow(x, h), r, oa);
-        tile_cols<D>(Qt, crow(x, h), r, qa);
-#pragma unroll
-        for (int db = 0; db < DB; ++db) {
-          dv[db] = mfma32(oa[db], p[x], dv[db]);
-          dk[db] = mfma32(qa[db], ds[x], dk[db]);
-        }
+      for (int db = 0; db < DB; ++db) {
+        dv[db] = mfma32(oa[db], p[x], dv[db]);
+        dk[db] = mfma32(qa[db], ds[x], dk[db]);
       }
     }
   }
@@ -583,17 +728,6 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void dkdv32_kernel(const Arg
   if (partial_block && key < S) {
     float* pk = a.partial + ((int64_t(b) * a.Hkv + kvh) * (a.n_chunks + 1) + (is_chunk ? chunk : a.n_chunks)) * 2 * S * D + key * D;
     float* pv = pk + S * D;
-    if (col_split) {
-#pragma unroll
-      for (int db = 0; db < DB / 2; ++db)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int d = DB * crow(e, h) + kh * (DB / 2) + db;
-          pk[d] = dk[db][e];
-          pv[d] = dv[db][e];
-        }
-      return;
-    }
     store_cols<D>(pk, dk, h, 1.f);
     store_cols<D>(pv, dv, h, 1.f);
     return;

@@ -26,6 +26,13 @@ pytestmark = pytest.mark.gpu
     pytest.param(1, 2, 1, 900, 32, 64, 96, id="two-sink-blocks"),
     pytest.param(1, 2, 2, 700, 128, 1, 16, id="W1-sinks-D128"),
     pytest.param(1, 2, 1, 450, 16, 0, 20, id="sinks-only-D16"),
+    # chunks of at most 16 sink keys: ragged ends, odd numbers of items, every head dim
+    pytest.param(1, 3, 1, 369, 64, 77, 1, id="one-sink-G3"),
+    pytest.param(2, 8, 1, 500, 64, 128, 16, id="16-sinks-G8"),
+    pytest.param(1, 4, 1, 513, 64, 33, 17, id="17-sinks"),
+    pytest.param(1, 2, 1, 600, 128, 90, 31, id="31-sinks-D128"),
+    pytest.param(1, 3, 3, 333, 16, 40, 15, id="sinks-D16"),
+    pytest.param(1, 4, 2, 129, 32, 64, 9, id="one-chunk-D32"),
 ])
 def test_fp32_tiles(gpu, B, Hq, Hkv, L, D, W, S):
     run(B, Hq, Hkv, L, D, W, S, seed=5)
