@@ -9,17 +9,20 @@
 // dK/dV summed over the query heads that share a KV head.
 //
 // Launches:
-//  1. bwd_dq_kernel (query-major, same tiling as the forward): computes delta for its rows
-//     (stored in the workspace) and dQ over the sink + window key blocks.  With at most 16 sink
-//     keys in key block 0 (dq_sink_mode) it also accumulates those keys' dK/dV for the rows past
-//     block 0's window, flushing fp32 partials to the workspace.
+//  1. dQ (query-major): computes delta for its rows (stored in the workspace) and dQ over the sink +
+//     window key blocks.  bwd_dq_split_kernel (fa_bwd_dq.hip), one tile per workgroup;
+//     bwd_dq_slide_kernel (fa_bwd_slide.hip) for the GPT-OSS sliding layers; or bwd_dq_kernel, which with
+//     at most 16 sink keys in key block 0 (dq_sink_mode) also accumulates those keys' dK/dV for the
+//     rows past block 0's window (as the sliding kernel does), flushing fp32 partials to the workspace,
+//     and keeps short windows at D <= 32 (plan_dq_split in fa_capi.cpp).
 //  2. bwd_dkdv_kernel (key-major): a workgroup owns 64 keys of one KV head and sweeps the
 //     (query head, 32-row query block) pairs that can see those keys, bounded by the window:
 //     rows [k0, k0 + 63 + W).  Every sum is formed in a fixed order, so results are
 //     deterministic.  Sink keys are also seen by every later row; outside dq_sink_mode those
 //     rows are split into chunks of `chunk_rows` handled by extra workgroups of the same kernel
 //     (the reference instead loops one program over all of L for a sink block,
-//     benchmark_backward_speed.py:432-438).  In dq_sink_mode key block 0's workgroup adds the
+//     benchmark_backward_speed.py:432-438).  A key block's steps can be cut into pieces
+//     (kv_split), whose fp32 sums bwd_dkdv_fold_kernel adds.  In dq_sink_mode key block 0's workgroup adds the
 //     dQ kernel's partials to its own when its sink keys' columns fit one pass of 256 threads.
 //  3. bwd_sink_fold_kernel (when rows were chunked, or the in-kernel fold does not apply): adds
 //     the sink rows' partial sums.

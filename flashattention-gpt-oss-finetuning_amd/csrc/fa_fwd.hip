@@ -5,10 +5,12 @@
 // online softmax in the log2 domain), a different decomposition:
 //
 //  * A tile is 32*wq query rows of HPW*wh query heads of ONE KV group, so every K/V block
-//    staged in LDS serves all of those heads.  The grid is one resident wave of 4-wave
-//    workgroups; every XCD owns a contiguous range of tiles (neighbouring tiles share K/V rows in
-//    its L2) and its workgroups walk it, each loading its next tile's Q rows by LDS DMA while the
-//    current tile computes.
+//    staged in LDS serves all of those heads.  fwd_split_kernel takes one tile per workgroup, its keys
+//    shared by up to four waves.  fwd_kernel (plan_fwd_split in fa_capi.cpp says for which shapes) is
+//    one resident wave of 4-wave workgroups; every XCD owns a contiguous range of tiles
+//    (neighbouring tiles share K/V rows in its L2) and its workgroups walk it, each loading its next
+//    tile's Q rows by LDS DMA while the current tile computes.  fwd_slide_kernel walks the GPT-OSS
+//    sliding layers' tiles with the window's keys in an LDS ring.
 //  * Each wave owns 32 query rows x HPW heads and computes the transposed score tile
 //    S^T = K Q^T (keys x queries) on v_mfma_f32_32x32x16: the lane that holds column q of S^T
 //    owns query row q, so the row max / row sum / rescale of the online softmax are per-lane

@@ -156,9 +156,9 @@ FA_HD int kv_n_chunks(int L, int W, int S, int chunk_rows) {
 
 // ---- sink rows in the dQ kernel ------------------------------------------------------------------
 // With at most kDqSinkKeys sink keys (all in key block 0) and rows past block 0's window, the dQ
-// kernel -- which visits keys [0, 32) for every query tile -- also accumulates the sink keys' dK/dV
-// contributions of those rows, [dq_sink_row0, L); the key-major kernel then runs no chunk
-// workgroups and covers only rows [0, dq_sink_row0) of block 0.
+// kernel -- which visits keys [0, 32) for every query tile -- can also accumulate the sink keys' dK/dV
+// contributions of those rows, [dq_sink_row0, L) (not with long windows at D >= 64, see sinks_by_chunks in
+// fa_capi.cpp); the key-major kernel then runs no chunk workgroups and covers only rows [0, dq_sink_row0) of block 0.
 constexpr int kDqSinkKeys = 16;
 
 FA_HD bool dq_sink_mode(int L, int W, int S) { return S >= 1 && S <= kDqSinkKeys && kv_sink_blocks(L, W, S) == 1; }
