@@ -41,7 +41,7 @@ __global__ __launch_bounds__(256, D == 128 || KSP == 4 ? 2 : 3) void bwd_dq_spli
   const int W = a.W, S = a.S;
 
   const int gpk = a.G / wh;
-  const QStream qs = q_stream(blockIdx.x, a.B * a.Hkv * gpk);
+  const QStream qs = q_stream(blockIdx.x, a.B * a.Hkv * gpk, a.cu_seqlens != nullptr);
   const int kvh = qs.stream / gpk / a.B, b = qs.stream / gpk % a.B;
   const int hw = kvh * a.G + qs.stream % gpk * wh + hi;
   const Seq sq = seq_of(a, b);

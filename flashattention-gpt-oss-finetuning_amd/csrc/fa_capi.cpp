@@ -371,10 +371,10 @@ int plan_split(fa::Args& a, int hpw, const SplitCost (&costs)[3], const double (
 // fwd_kernel keeps what it still does better: D <= 32 with one head per wave and short windows, whose
 // tiles' key blocks it fetches at once (the D = 16, W = 256 default case 10.9 against 12.2 us), and D = 128
 // with odd KV groups (one head per group, B = 2, Hq = 32, L = 2048 full causal 81.5 against 85 us) or with
-// two rounds and more of workgroups that keep one wave per tile over long rows (B = 2, Hq = 64, Hkv = 8,
+// two rounds and more of workgroups that keep one wave per tile over long rows of equal length (B = 2, Hq = 64, Hkv = 8,
 // L = 16384: W = 1024 1335 against 1376, full causal 9003 against 9309; Hq = 32, L = 4096, W = 400 46.7
 // against 48.4; but W = 64 366 against 349 and 28.4 against 27.3, and one round, Hq = 64, L = 1024 full
-// causal 38 against 32).
+// causal 38 against 32; sequences of 1536, 1187, 640 and 933 rows, Hq = 32, Hkv = 8, full causal 100 against 60).
 int plan_fwd_split(fa::Args& a, int D, int hpw) {
   static const SplitCost costs[4][2][3] = {
       // [D][heads per wave - 1][KSP = 1, 2, 4]
@@ -387,9 +387,8 @@ int plan_fwd_split(fa::Args& a, int D, int hpw) {
   if (D == 128 && a.G % 2 != 0) return 0;
   const fa::Args given = a;
   const int ksp = plan_split(a, hpw, costs[D == 16 ? 0 : D == 32 ? 1 : D == 64 ? 2 : 3][hpw - 1], fixed, hpw == 2 ? 4. : 3.);
-  if (D == 128 && ksp == 1 && a.W >= 192) {
-    const int64_t rows = a.cu_seqlens ? std::min(int64_t(a.B) * a.L, int64_t(a.token_rows)) : int64_t(a.B) * a.L;
-    if (rows * (a.Hq / a.wh) >= int64_t(32) * a.wq * 2 * 2 * fa::device_cus()) {  // (two fit a CU)
+  if (D == 128 && ksp == 1 && a.W >= 192 && !a.cu_seqlens) {
+    if (int64_t(a.B) * a.L * (a.Hq / a.wh) >= int64_t(32) * a.wq * 2 * 2 * fa::device_cus()) {  // (two fit a CU)
       a = given;
       return 0;
     }

@@ -136,7 +136,7 @@ struct QTile {
 __device__ __forceinline__ QTile q_tile(const Args& a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int gpk = a.G / a.wh;  // head groups per KV head
-  const QStream s = q_stream(blockIdx.x, a.B * a.Hkv * gpk);
+  const QStream s = q_stream(blockIdx.x, a.B * a.Hkv * gpk, a.cu_seqlens != nullptr);
   QTile t;
   t.kvh = s.stream / gpk / a.B;
   t.b = s.stream / gpk % a.B;

@@ -782,7 +782,7 @@ __global__ __launch_bounds__(256, D == 128 || KSP == 4 ? 2 : 3) void fwd_split_k
   if (int(blockIdx.x) >= a.main_wgs) return fwd_aux<D, 2>(a);
   // workgroup -> row tile, batch, head set (see q_stream)
   const int gpk = a.G / (HPW * wh);
-  const QStream qs = q_stream(blockIdx.x, a.B * a.Hkv * gpk);
+  const QStream qs = q_stream(blockIdx.x, a.B * a.Hkv * gpk, a.cu_seqlens != nullptr);
   const int kvh = qs.stream / gpk / a.B, b = qs.stream / gpk % a.B;
   const int hw = kvh * a.G + (qs.stream % gpk * wh + hi) * HPW;
   const Seq sq = seq_of(a, b);
