@@ -55,7 +55,9 @@ FA_HD QPlan qplan(int q0, int bm, int L, int W, int S) {
 FA_HD int qplan_block(const QPlan& p, int i) { return i < p.nsb ? i * kLdsKeys : p.ws + (i - p.nsb) * kLdsKeys; }
 
 // The same in tiles of 32 keys, for workgroups of rows [q0, q0 + bm) that visit 32-key tiles: the sink
-// tiles [0, nsink) (keys below S that lie before the window tiles), then the window tiles [ws, we).
+// tiles [0, nsink) (keys below S that lie before the window tiles), then the window tiles [ws, we).  A
+// window of no keys counts as one of one key here, so that a row's own key, which may be a sink, is always in a
+// tile (a last tile of one row, q0 = L - 1, has no other).
 struct Plan32 {
   int nsink, ws, we;
 };
@@ -63,7 +65,7 @@ struct Plan32 {
 FA_HD Plan32 plan32(int q0, int bm, int L, int W, int S) {
   Plan32 p;
   const int q_end = imin(q0 + bm, L);
-  const int wlo = imax(0, q0 - W + 1);  // first key in any row's window
+  const int wlo = imax(0, q0 - imax(W, 1) + 1);  // first key in any row's window
   p.ws = wlo / 32;
   p.we = q_end > wlo ? (q_end - 1) / 32 + 1 : p.ws;
   p.nsink = (imin(S, 32 * p.ws) + 31) / 32;

@@ -1,7 +1,8 @@
 // plan_check.cpp - host check of the kernels' visit plan (csrc/fa_plan.h compiled with g++).
 //
-// Walks the loops of the query-major kernels (fa_fwd.hip fwd_kernel, fa_bwd.hip bwd_dq_kernel,
-// fa_bwd_slide.hip bwd_dq_slide_kernel) and of the key-major kernels (bwd_dkdv_kernel,
+// Walks the loops of the query-major kernels (fa_fwd.hip fwd_kernel, fa_bwd.hip bwd_dq_kernel by
+// 64-key blocks; fwd_split_kernel, fa_bwd_dq.hip bwd_dq_split_kernel and the float32 kernels by 32-key
+// tiles; fa_bwd_slide.hip bwd_dq_slide_kernel) and of the key-major kernels (bwd_dkdv_kernel,
 // bwd_dkdv4_kernel) over many (L, W, S, rows-per-workgroup, chunk size) cases and checks that
 //   * every allowed (q, k) pair is visited exactly once and no other pair is counted,
 //   * a tile reported "full" (mask skipped) holds only allowed pairs,
@@ -57,6 +58,38 @@ static int check_qmajor(int L, int W, int S, int wq) {
     for (int k = 0; k < L; ++k) {
       const int want = ref_allowed(q, k, W, S) ? 1 : 0;
       if (cnt[size_t(q) * L + k] != want) return fail("q-major visit count", L, W, S, wq, q, k, cnt[size_t(q) * L + k]);
+    }
+  return 0;
+}
+
+// Query-major in 32-key tiles (plan32): workgroups of bm = 32*wq rows, whose waves of 32 rows skip
+// tiles that wave_needs rules out when there are several (one wave takes every tile), tile i going to
+// one of the waves that share a tile's keys.
+static int check_plan32(int L, int W, int S, int wq) {
+  const int bm = 32 * wq;
+  std::vector<int> cnt(size_t(L) * L, 0);
+  for (int q0 = 0; q0 < L; q0 += bm) {
+    const Plan32 p = plan32(q0, bm, L, W, S);
+    for (int i = 0; i < p.nsink + (p.we - p.ws); ++i) {
+      const int ks0 = 32 * plan32_tile(p, i);
+      if (ks0 < 0 || ks0 >= L) return fail("32-key tile out of range", L, W, S, wq, q0, ks0, 0);
+      for (int qw = q0; qw < q0 + bm && qw < L; qw += 32) {
+        if (wq > 1 && !wave_needs(ks0, qw, L, W, S)) continue;
+        const bool full = tile_full(ks0, qw, W, S);
+        for (int q = qw; q < qw + 32 && q < L; ++q)  // rows >= L are never stored
+          for (int k = ks0; k < ks0 + 32; ++k) {
+            if (full && !(k < L && ref_allowed(q, k, W, S))) return fail("full 32-key tile has a masked pair", L, W, S, wq, q, k, 0);
+            if (!full && !allowed(q - k, k, W, S)) continue;
+            if (k >= L) return fail("key beyond L passes the mask", L, W, S, wq, q, k, 0);
+            ++cnt[size_t(q) * L + k];
+          }
+      }
+    }
+  }
+  for (int q = 0; q < L; ++q)
+    for (int k = 0; k < L; ++k) {
+      const int want = ref_allowed(q, k, W, S) ? 1 : 0;
+      if (cnt[size_t(q) * L + k] != want) return fail("32-key tile visit count", L, W, S, wq, q, k, cnt[size_t(q) * L + k]);
     }
   return 0;
 }
@@ -230,10 +263,10 @@ int main() {
         if (Wr < 1 && Sr < 1) continue;  // rejected by the C ABI
         const int W = Wr > L ? L : Wr, S = Sr > L ? L : Sr;  // clamped as in fa_capi.cpp
         for (int wq : {1, 2, 4}) {
-          if (check_qmajor(L, W, S, wq)) return 1;
-          ++cases;
+          if (check_qmajor(L, W, S, wq) || check_plan32(L, W, S, wq)) return 1;
+          cases += 2;
         }
-        for (int cr : {32, 64, 256}) {
+        for (int cr : {32, 64, 128, 256}) {
           if (check_kvmajor(L, W, S, cr)) return 1;
           ++cases;
         }
@@ -243,6 +276,16 @@ int main() {
         }
         if (W >= 1 && W <= kSlideMaxW && S <= 32) {
           if (check_slide(L, W, S)) return 1;
+          ++cases;
+        }
+      }
+  // every small length with windows and sinks around it
+  for (int L = 1; L <= 140; ++L)
+    for (int W : {0, 1, 31, 32, 33, 64, 65, L - 1, L})
+      for (int S : {0, 1, 32, 33, 65, L - 1, L}) {
+        if (W > L || S > L || (W < 1 && S < 1)) continue;
+        for (int wq : {1, 2, 4}) {
+          if (check_plan32(L, W, S, wq)) return 1;
           ++cases;
         }
       }
