@@ -10,7 +10,7 @@
 //
 // The codes are those of (x / descale).clamp(-448, 448).to(float8_e4m3fn) on float32 values, where
 // PyTorch divides a GPU tensor by a host number (a double) as a product with that number's reciprocal rounded
-// to float32; NaNs stay NaNs (this file is compiled with NaNs honoured).
+// to float32; NaNs stay NaNs of their sign (this file is compiled with NaNs honoured).
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -124,11 +124,10 @@ __global__ __launch_bounds__(kThreads) void quantize_kernel(const void* x, int64
     const float amax = __builtin_bit_cast(float, m);
     inv = amax > 0.f ? float(1.0 / (double(amax) / 448.0)) : 1.f;
   }
+  auto clamp = [](float a) { return a < -kE4m3Max ? -kE4m3Max : a > kE4m3Max ? kE4m3Max : a; };
   auto code2 = [&](float a, float b, int old, bool hi) {
-    a *= inv;
-    b *= inv;
-    a = a < -kE4m3Max ? -kE4m3Max : a > kE4m3Max ? kE4m3Max : a;
-    b = b < -kE4m3Max ? -kE4m3Max : b > kE4m3Max ? kE4m3Max : b;
+    a = clamp(a);
+    b = clamp(b);
     return hi ? __builtin_amdgcn_cvt_pk_fp8_f32(a, b, old, true) : __builtin_amdgcn_cvt_pk_fp8_f32(a, b, old, false);
   };
   // a unit is 16 codes
@@ -137,16 +136,25 @@ __global__ __launch_bounds__(kThreads) void quantize_kernel(const void* x, int64
   const int64_t units = n / 16, step = int64_t(gridDim.x) * kThreads;
   auto encode = [&](const u32x4 (&v)[PIECES]) {
     float f[16];
+    bool nan = false;
 #pragma unroll
     for (int j = 0; j < PIECES; ++j) {
       float g[T::N];
       T::get(v[j], g);
 #pragma unroll
-      for (int e = 0; e < T::N; ++e) f[T::N * j + e] = g[e];
+      for (int e = 0; e < T::N; ++e) {
+        f[T::N * j + e] = g[e] * inv;
+        nan |= f[T::N * j + e] != f[T::N * j + e];
+      }
     }
     u32x4 o;
 #pragma unroll
     for (int w = 0; w < 4; ++w) o[w] = uint32_t(code2(f[4 * w + 2], f[4 * w + 3], code2(f[4 * w], f[4 * w + 1], 0, false), true));
+    if (nan) {  // the conversion gives every NaN the code 0xff; a NaN keeps its sign (of two, the scale's counts)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (f[i] != f[i]) o[i / 4] ^= (~__builtin_bit_cast(uint32_t, inv != inv ? inv : f[i]) >> 31) << (8 * (i % 4) + 7);
+    }
     return o;
   };
   for (int64_t u = int64_t(blockIdx.x) * kThreads + threadIdx.x; u < units; u += step) {

@@ -61,3 +61,18 @@ def test_layouts_and_special_tensors(gpu):
     check(torch.full((33,), float("inf"), device=gpu))
     check(torch.full((33,), 1e-44, device=gpu))
     check(torch.tensor([0.0, -0.0, 1e-30, -3e38], device=gpu))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_nan_codes(gpu, dtype):
+    """A NaN's code is 0x7f or 0xff by its sign, as PyTorch's; also NaNs that the scaling makes."""
+    bits = torch.int16 if dtype != torch.float32 else torch.int32
+    x = torch.randn(8 * 37 + 3, device=gpu).to(dtype)
+    quiet = torch.full((), float("nan"), dtype=dtype).view(bits).item() & torch.iinfo(bits).max
+    x.view(bits)[5::7] = quiet
+    x.view(bits)[3::11] = quiet | torch.iinfo(bits).min
+    x[40] = float("inf")
+    x[41] = -float("inf")
+    for descale in (None, 0.5, float("inf"), float("nan")):
+        got, ref = load_pkg().quantize_fp8(x, descale)[0], reference(x, descale)[0]
+        assert torch.equal(got.view(torch.uint8), ref.view(torch.uint8)), descale
