@@ -161,9 +161,11 @@ def quantize_fp8(x: torch.Tensor, descale: Optional[float] = None):
     """Per-tensor e4m3 quantisation for flash_swda_with_sink_fp8: returns (x8, descale) with
     x ~= descale * x8 (x8 in torch.float8_e4m3fn, round to nearest even); descale defaults to
     amax(|x|) / 448, so the largest magnitude maps to the largest finite e4m3 value."""
-    b = _ops.autograd_binding(x)
+    plain = not (torch.compiler.is_compiling() or torch.overrides.has_torch_function_unary(x))
+    b = _ops.autograd_binding(x) if plain else None
     if b is not None and (descale is None or isinstance(descale, (int, float))):
-        # two passes over a dense 16- or 32-bit GPU tensor (fa_quantize_fp8*); None for other tensors
+        # two passes over a dense 16- or 32-bit GPU tensor (fa_quantize_fp8*); None for other tensors, and
+        # where the call is traced or transformed, which only PyTorch's own operations allow
         r = b.quantize_fp8(x, descale)
         if r is not None:
             return r

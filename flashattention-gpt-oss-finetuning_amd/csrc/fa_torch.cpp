@@ -13,7 +13,10 @@
 #include <torch/extension.h>
 
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <stdexcept>
 #include <string>
@@ -79,6 +82,18 @@ void raise_for_status(int rc, const char* what) {
 
 void* current_stream(const at::Tensor& t) {
   return c10::hip::getCurrentHIPStream(t.device().index()).stream();
+}
+
+// Is the call recorded or transformed instead of computed on plain tensors (torch.jit tracing, dispatch modes as
+// make_fx's and FakeTensorMode, functorch's transforms, forward-mode AD)?  What a C ABI call writes is
+// invisible to all of them: a trace would keep the allocation of its outputs only.
+bool transformed(std::initializer_list<const at::Tensor*> ts) {
+  if (torch::jit::tracer::isTracing() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+      c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
+    return true;
+  for (const at::Tensor* t : ts)
+    if (t->key_set().has(c10::DispatchKey::Python) || t->_fw_grad(0).defined()) return true;
+  return false;
 }
 
 // Learned sink logits as the C ABI takes them: float32 [Hq], contiguous, on q's device.
@@ -433,8 +448,9 @@ at::Tensor swda_varlen(const at::Tensor& q, const at::Tensor& k, const at::Tenso
 // Per-tensor e4m3 quantisation of a GPU tensor (quantize_fp8 in attention.py): (x8, descale), x8 with x's
 // strides; without a given descale it is max |x| / 448.  The host waits for the maximum only: the codes
 // are written by a kernel behind it that reads the maximum on the device.  Returns None for tensors
-// the kernels do not take (other dtypes, strides with gaps, unaligned or empty).
+// the kernels do not take (other dtypes, strides with gaps, unaligned or empty) and in transformed calls.
 py::object quantize_fp8(const at::Tensor& x_in, c10::optional<double> descale) {
+  if (transformed({&x_in})) return py::none();
   const at::Tensor x = x_in.detach();
   const auto st = x.scalar_type();
   const int dtype = st == at::kBFloat16 ? FA_DTYPE_BF16 : st == at::kHalf ? FA_DTYPE_F16 : st == at::kFloat ? FA_DTYPE_F32 : 0;

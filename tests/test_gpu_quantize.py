@@ -76,3 +76,33 @@ def test_nan_codes(gpu, dtype):
     for descale in (None, 0.5, float("inf"), float("nan")):
         got, ref = load_pkg().quantize_fp8(x, descale)[0], reference(x, descale)[0]
         assert torch.equal(got.view(torch.uint8), ref.view(torch.uint8)), descale
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+def test_traced_and_transformed_calls(gpu):
+    """Calls that are recorded or transformed run the PyTorch expression: traces compute, on other
+    inputs too, and vmap, functorch, fake tensors, subclasses and compilation work as with it."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    fa = load_pkg()
+    f = lambda t: fa.quantize_fp8(t, 0.5)[0]
+    x, y = torch.randn(4, 64, device=gpu), torch.randn(4, 64, device=gpu)
+    same = lambda a, t: torch.equal(a.view(torch.uint8), reference(t, 0.5)[0].view(torch.uint8))
+    for traced in (torch.jit.trace(f, (x,), check_trace=False), make_fx(f)(x),
+                   torch.compile(f, backend="eager", fullgraph=True)):
+        stale = torch.full((4, 64), 7, dtype=torch.uint8, device=gpu)
+        del stale  # (what uninitialised outputs would hold)
+        assert same(traced(y), y)
+    assert same(torch.vmap(f)(x), x)
+    assert same(torch.func.functionalize(f)(x), x)
+    assert not torch.func.grad(lambda t: f(t).float().sum())(x).any()
+    mode = FakeTensorMode()
+    fake = mode.from_tensor(x)
+    with mode:
+        assert f(fake).shape == (4, 64)
+    assert f(fake).dtype == torch.float8_e4m3fn
+    assert type(f(x.as_subclass(_Sub))) is _Sub and same(f(x.as_subclass(_Sub)).as_subclass(torch.Tensor), x)
