@@ -129,15 +129,15 @@ def flash_swda_with_sink_varlen(q, k, v, cu_seqlens, max_seqlen, window_size, si
     required), window_size None for full causal attention.  On GPU tensors its C++ twin (the
     binding's swda_varlen: the same checks, kernels, saved tensors and gradients)."""
     b = _ops.autograd_binding(q)
-    if b is None:
-        return FlashSWDAWithSinkVarlen.apply(q, k, v, cu_seqlens, max_seqlen, window_size, sink_size, scale, sinks)
-    if scale is None:
-        scale = 1.0 / math.sqrt(q.shape[-1])
-    _check_packed_shapes(q, k, v)
-    cu, max_seqlen = _ops.cu_seqlens_ready(cu_seqlens, q.shape[0], q.device, max_seqlen)
-    if window_size is None:
-        window_size = max_seqlen
-    return b.swda_varlen(q, k, v, cu, None, max_seqlen, 0, int(window_size), int(sink_size), float(scale), sinks)
+    if b is not None:
+        sc = 1.0 / math.sqrt(q.shape[-1]) if scale is None else scale
+        _check_packed_shapes(q, k, v)
+        cu, longest = _ops.cu_seqlens_ready(cu_seqlens, q.shape[0], q.device, max_seqlen)
+        W = longest if window_size is None else int(window_size)
+        o = b.swda_varlen(q, k, v, cu, None, longest, 0, W, int(sink_size), float(sc), sinks)
+        if o is not None:  # (None where the call is traced or transformed)
+            return o
+    return FlashSWDAWithSinkVarlen.apply(q, k, v, cu_seqlens, max_seqlen, window_size, sink_size, scale, sinks)
 
 
 def _check_packed_shapes(q, k, v):
@@ -213,22 +213,24 @@ def _swda(q, k, v, window_size, sink_size, is_causal=True, scale=None, sinks=Non
     """FlashSWDAWithSink (or, with `sinks`, FlashSWDAWithLearnedSinks) applied to GPU tensors
     through the binding's autograd functions in C++ (fa_torch.swda / swda_sinks): the same checks
     and messages, the same kernels, saved tensors and gradients, without Python in the backward.
-    Without the binding, or for tensors that are not on a GPU, the Python autograd functions."""
+    Without the binding, for tensors that are not on a GPU and where the call is traced or
+    transformed (the binding then returns None), the Python autograd functions."""
     b = _ops.autograd_binding(q)
-    if b is None:
+    if b is not None:
+        if not is_causal:
+            raise AssertionError("Currently, only causal attention is supported")
+        sc = 1.0 / math.sqrt(q.shape[-1]) if scale is None else scale
+        _check_shapes(q, k, v)
         if sinks is None:
-            return FlashSWDAWithSink.apply(q, k, v, window_size, sink_size, is_causal, scale)
-        return FlashSWDAWithLearnedSinks.apply(q, k, v, sinks, window_size, sink_size, scale)
-    if not is_causal:
-        raise AssertionError("Currently, only causal attention is supported")
-    if scale is None:
-        scale = 1.0 / math.sqrt(q.shape[-1])
-    _check_shapes(q, k, v)
+            o = b.swda(q, k, v, int(window_size), int(sink_size), float(sc))
+        else:
+            W = q.shape[2] if window_size is None else int(window_size)
+            o = b.swda_sinks(q, k, v, sinks, W, int(sink_size), float(sc))
+        if o is not None:
+            return o
     if sinks is None:
-        return b.swda(q, k, v, int(window_size), int(sink_size), float(scale))
-    if window_size is None:
-        window_size = q.shape[2]
-    return b.swda_sinks(q, k, v, sinks, int(window_size), int(sink_size), float(scale))
+        return FlashSWDAWithSink.apply(q, k, v, window_size, sink_size, is_causal, scale)
+    return FlashSWDAWithLearnedSinks.apply(q, k, v, sinks, window_size, sink_size, scale)
 
 
 def flash_swda_with_sink(q, k, v, window_size: int, sink_size: int = 0, is_causal: bool = True,

@@ -252,13 +252,17 @@ struct SwdaSinksFunction : public torch::autograd::Function<SwdaSinksFunction> {
   }
 };
 
-at::Tensor swda(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, int64_t window, int64_t sink,
-                double scale) {
+// The autograd functions' forwards; None for a transformed call, which the Python functions take (torch.jit traces
+// those as a call, forward-mode AD and functorch refuse them by name).
+c10::optional<at::Tensor> swda(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, int64_t window,
+                               int64_t sink, double scale) {
+  if (transformed({&q, &k, &v})) return c10::nullopt;
   return SwdaFunction::apply(q, k, v, window, sink, scale);
 }
 
-at::Tensor swda_sinks(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& sinks,
-                      int64_t window, int64_t sink, double scale) {
+c10::optional<at::Tensor> swda_sinks(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                                     const at::Tensor& sinks, int64_t window, int64_t sink, double scale) {
+  if (transformed({&q, &k, &v, &sinks})) return c10::nullopt;
   return SwdaSinksFunction::apply(q, k, v, sinks, window, sink, scale);
 }
 
@@ -439,9 +443,11 @@ struct SwdaVarlenFunction : public torch::autograd::Function<SwdaVarlenFunction>
   }
 };
 
-at::Tensor swda_varlen(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& cu,
-                       const c10::optional<at::Tensor>& lens, int64_t max_seqlen, int64_t token_rows, int64_t window,
-                       int64_t sink, double scale, const c10::optional<at::Tensor>& sinks) {
+c10::optional<at::Tensor> swda_varlen(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                                      const at::Tensor& cu, const c10::optional<at::Tensor>& lens, int64_t max_seqlen,
+                                      int64_t token_rows, int64_t window, int64_t sink, double scale,
+                                      const c10::optional<at::Tensor>& sinks) {
+  if (transformed({&q, &k, &v, sinks.has_value() ? &*sinks : &q})) return c10::nullopt;
   return SwdaVarlenFunction::apply(q, k, v, cu, lens, max_seqlen, token_rows, window, sink, scale, sinks);
 }
 
@@ -482,14 +488,14 @@ py::object quantize_fp8(const at::Tensor& x_in, c10::optional<double> descale) {
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("swda", &swda,
-        "autograd forward of causal sliding-window + sink attention: (q, k, v, window, sink, scale) -> o",
+        "autograd forward of causal sliding-window + sink attention: (q, k, v, window, sink, scale) -> o or None",
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("window"), py::arg("sink"), py::arg("scale"));
   m.def("swda_sinks", &swda_sinks,
-        "autograd forward with learned sink logits: (q, k, v, sinks, window, sink, scale) -> o", py::arg("q"),
+        "autograd forward with learned sink logits: (q, k, v, sinks, window, sink, scale) -> o or None", py::arg("q"),
         py::arg("k"), py::arg("v"), py::arg("sinks"), py::arg("window"), py::arg("sink"), py::arg("scale"));
   m.def("swda_varlen", &swda_varlen,
         "autograd forward of a packed batch: (q, k, v, cu_seqlens or starts, lens, max_seqlen, token_rows, window, sink, "
-        "scale, sinks=None) -> o",
+        "scale, sinks=None) -> o or None",
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("cu"), py::arg("lens"), py::arg("max_seqlen"),
         py::arg("token_rows"), py::arg("window"), py::arg("sink"), py::arg("scale"), py::arg("sinks") = py::none());
   m.def("quantize_fp8", &quantize_fp8, "per-tensor e4m3 quantisation: (x, descale=None) -> (x8, descale) or None",

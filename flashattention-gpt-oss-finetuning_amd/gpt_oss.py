@@ -220,7 +220,9 @@ def padded_attention(q, k, v, attention_mask, window_size: Optional[int] = None,
         qr, kr, vr = rows(q), rows(k), rows(v)
         _check_packed_shapes(qr, kr, vr)
         sc = 1.0 / math.sqrt(D) if scale is None else float(scale)
-        return b.swda_varlen(qr, kr, vr, starts, lens, max_len, tokens, W, 0, sc, sinks).view(B, L, Hq, D)
+        o = b.swda_varlen(qr, kr, vr, starts, lens, max_len, tokens, W, 0, sc, sinks)
+        if o is not None:  # (None where the call is traced or transformed)
+            return o.view(B, L, Hq, D)
     # token rows of the [B * L] flattening (in order), their offsets
     _, idx, cu, _ = packed if packed is not None else _mask_facts(attention_mask.to(device=q.device))
 
