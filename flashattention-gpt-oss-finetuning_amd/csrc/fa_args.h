@@ -84,8 +84,28 @@ struct Args {
   float* kv_part;
   // a kernel's own workgroups are [0, main_wgs); the ones behind them do the work of fa_aux.h, tail_wgs of
   // them on packed rows outside every sequence
-  int main_wgs, tail_wgs;
+  unsigned main_wgs;
+  int tail_wgs;
+  // kernels with a workgroup per tile of a B x longest sequence grid: the first workgroup of this launch
+  // (launch_in_ranges)
+  unsigned wg_base;
 };
+
+// A grid holds fewer than 2^32 threads; a larger one is not refused, but not all of it runs (measured).
+// Launches of 256-thread workgroups whose number follows B times the longest sequence (most of them empty in a
+// packed batch with short ones) are cut into ranges of kRangeWgs, whole rounds of the 8 XCDs; `launch` gets a
+// range's grid, with args.wg_base set.
+constexpr int64_t kRangeWgs = int64_t(1) << 23;
+template <typename F>
+inline hipError_t launch_in_ranges(Args& args, int64_t wgs, F&& launch) {
+  for (int64_t lo = 0; lo < wgs; lo += kRangeWgs) {
+    args.wg_base = unsigned(lo);
+    launch(dim3(unsigned(wgs - lo < kRangeWgs ? wgs - lo : kRangeWgs)));
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
 
 // Sequence b: its length and the row where it starts in the packed tensors (fixed-length
 // batches: L rows from row 0 of batch b's slice).  Offsets are clamped to the tensors' rows and

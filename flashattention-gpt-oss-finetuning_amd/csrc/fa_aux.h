@@ -72,10 +72,10 @@ __device__ inline void zero_rows(void* ptr, const int64_t (&st)[3], int heads, i
   }
 }
 
-// The forward's extra workgroups; EB bytes per element of o.
+// The forward's extra workgroups (`wg`: the workgroup's id); EB bytes per element of o.
 template <int D, int EB>
-__device__ inline void fwd_aux(const Args& a) {
-  for_gaps(a, int(blockIdx.x) - a.main_wgs, [&](int lo, int hi, int64_t first, int64_t step) {
+__device__ inline void fwd_aux(const Args& a, unsigned wg) {
+  for_gaps(a, int(wg - a.main_wgs), [&](int lo, int hi, int64_t first, int64_t step) {
     if (lo >= hi) return;
     zero_rows(a.o_out, a.so_out, a.Hq, D * EB, EB, lo, hi, first, step);
     for (int64_t u = first; u < int64_t(hi - lo) * a.Hq; u += step)
@@ -85,8 +85,8 @@ __device__ inline void fwd_aux(const Args& a) {
 
 // The dK/dV kernel's: a workgroup per head for the learned sinks (when a.dsink), then a.tail_wgs.
 template <int D, int EB>
-__device__ inline void bwd_aux(const Args& a, float* smem) {
-  int x = int(blockIdx.x) - a.main_wgs;
+__device__ inline void bwd_aux(const Args& a, unsigned wg, float* smem) {
+  int x = int(wg - a.main_wgs);
   if (a.dsink) {
     if (x < a.Hq) return sum_sink_logits(a, x, smem);
     x -= a.Hq;
@@ -99,12 +99,13 @@ __device__ inline void bwd_aux(const Args& a, float* smem) {
   });
 }
 
-// Host: workgroups behind a kernel's own `main` (a.main_wgs and a.tail_wgs are set): the whole grid.
+// Host: workgroups behind a kernel's own `main` (a.main_wgs and a.tail_wgs are set): all of the launch's.
 // Without seq_lens a packed batch usually covers every row, and its workgroups only read two offsets.
-inline unsigned grid_with_aux(Args& a, int64_t main, bool bwd) {
-  a.main_wgs = int(main);
+inline int64_t wgs_with_aux(Args& a, int64_t main, bool bwd) {
+  a.main_wgs = unsigned(main);
   a.tail_wgs = !a.cu_seqlens ? 0 : a.seq_lens ? 256 : 64;
-  return unsigned(main + a.tail_wgs + (bwd && a.dsink ? a.Hq : 0));
+  return main + a.tail_wgs + (bwd && a.dsink ? a.Hq : 0);
 }
+inline unsigned grid_with_aux(Args& a, int64_t main, bool bwd) { return unsigned(wgs_with_aux(a, main, bwd)); }
 
 }  // namespace fa

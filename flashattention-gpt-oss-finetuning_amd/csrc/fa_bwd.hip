@@ -722,8 +722,8 @@ __global__ __launch_bounds__(256, D == 16 ? 4 : KVL ? 3 : 1) void bwd_dkdv_kerne
   // chunks.  A group's workgroups land on one XCD (they share its L2), and the short chunk
   // workgroups run last, filling the slots that the regular ones leave.
   const int per_group = a.n_kblocks + a.nsp * a.n_chunks;
-  if (int(blockIdx.x) >= a.main_wgs) return bwd_aux<D, 2>(a, reinterpret_cast<float*>(lds));
-  const int id = SPLIT ? int(blockIdx.x) : xcd_remap(blockIdx.x, a.main_wgs);
+  if (blockIdx.x >= a.main_wgs) return bwd_aux<D, 2>(a, blockIdx.x, reinterpret_cast<float*>(lds));
+  const int id = SPLIT ? int(blockIdx.x) : xcd_remap(blockIdx.x, int(a.main_wgs));
   // groups in (KV head, batch) order, the KV head outermost: the XCDs then split over KV heads
   // before sequences, which keeps their work even for sequences of different lengths.  A packed
   // batch hands out only the key blocks with keys: per KV head, each sequence's blocks
@@ -1161,8 +1161,8 @@ __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : D == 16 && NW == 4 ? 3 : 2)
 
   // workgroups grouped per (b, KV head), n_kblocks 32-key blocks each, groups in (KV head, batch)
   // order with the KV head outermost (as bwd_dkdv_kernel)
-  if (int(blockIdx.x) >= a.main_wgs) return bwd_aux<D, 2>(a, reinterpret_cast<float*>(lds));
-  const int id = xcd_remap(blockIdx.x, a.main_wgs);
+  if (blockIdx.x >= a.main_wgs) return bwd_aux<D, 2>(a, blockIdx.x, reinterpret_cast<float*>(lds));
+  const int id = xcd_remap(blockIdx.x, int(a.main_wgs));
   const int grp = id / a.n_kblocks, kblk = id % a.n_kblocks;
   const int kvh = grp / a.B, b = grp % a.B;
   const Seq sq = seq_of(a, b);

@@ -41,7 +41,7 @@ __global__ __launch_bounds__(256, D == 128 || KSP == 4 ? 2 : 3) void bwd_dq_spli
   const int W = a.W, S = a.S;
 
   const int gpk = a.G / wh;
-  const QStream qs = q_stream(blockIdx.x, a.B * a.Hkv * gpk, a.cu_seqlens != nullptr);
+  const QStream qs = q_stream(int(a.wg_base + blockIdx.x), a.B * a.Hkv * gpk, a.cu_seqlens != nullptr);
   const int kvh = qs.stream / gpk / a.B, b = qs.stream / gpk % a.B;
   const int hw = kvh * a.G + qs.stream % gpk * wh + hi;
   const Seq sq = seq_of(a, b);
@@ -205,15 +205,16 @@ __global__ __launch_bounds__(256, D == 128 || KSP == 4 ? 2 : 3) void bwd_dq_spli
 
 template <typename E, int D, int KSP>
 static hipError_t dq_split_k(const Args& a, hipStream_t stream) {
-  const dim3 grid(unsigned(a.n_qtiles * a.B * (a.Hq / a.wh))), block(256);
-  if constexpr (KSP < 4) {
-    if (a.wq > 1) {
-      hipLaunchKernelGGL((bwd_dq_split_kernel<E, D, KSP, true>), grid, block, 0, stream, a);
-      return hipGetLastError();
+  Args x = a;
+  return launch_in_ranges(x, int64_t(a.n_qtiles) * a.B * (a.Hq / a.wh), [&](dim3 grid) {
+    if constexpr (KSP < 4) {
+      if (a.wq > 1) {
+        hipLaunchKernelGGL((bwd_dq_split_kernel<E, D, KSP, true>), grid, dim3(256), 0, stream, x);
+        return;
+      }
     }
-  }
-  hipLaunchKernelGGL((bwd_dq_split_kernel<E, D, KSP, false>), grid, block, 0, stream, a);
-  return hipGetLastError();
+    hipLaunchKernelGGL((bwd_dq_split_kernel<E, D, KSP, false>), grid, dim3(256), 0, stream, x);
+  });
 }
 
 template <typename E, int D>

@@ -425,6 +425,8 @@ int sinks_by_chunks(const fa::Args& a, int D, const SinkPlan& sp) {
   if (!rows) return 0;
   SinkPlan c = sp;
   c.n_chunks = fa::kv_n_chunks(a.L, a.W, a.S, rows);
+  // (the dQ kernel's grid is bounded; a dK/dV launch with a chunk per B x longest sequence need not fit one grid)
+  if (int64_t(a.B) * a.Hkv * c.n_chunks >= fa::kRangeWgs) return 0;
   const size_t room = partial_bytes(a.B, a.Hkv, D, sp) + dq_sink_slot_bytes(a.B, a.Hq, a.Hkv, a.L, D, sp);
   return partial_bytes(a.B, a.Hkv, D, c) <= room ? rows : 0;
 }

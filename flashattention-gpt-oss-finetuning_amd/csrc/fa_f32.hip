@@ -133,10 +133,10 @@ __device__ __forceinline__ void store_cols(float* row, const f32x16 (&acc)[kDB<D
 struct QTile {
   int b, kvh, hq, q0, qw;
 };
-__device__ __forceinline__ QTile q_tile(const Args& a) {
+__device__ __forceinline__ QTile q_tile(const Args& a, unsigned wg) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int gpk = a.G / a.wh;  // head groups per KV head
-  const QStream s = q_stream(blockIdx.x, a.B * a.Hkv * gpk, a.cu_seqlens != nullptr);
+  const QStream s = q_stream(int(wg), a.B * a.Hkv * gpk, a.cu_seqlens != nullptr);
   QTile t;
   t.kvh = s.stream / gpk / a.B;
   t.b = s.stream / gpk % a.B;
@@ -175,8 +175,9 @@ __global__ __launch_bounds__(256, 2) void fwd32_kernel(const Args a) {
   constexpr int DB = kDB<D>;
   __shared__ __attribute__((aligned(16))) float lds[2 * KvTiles<D>::kBuf];
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
-  if (int(blockIdx.x) >= a.main_wgs) return fwd_aux<D, 4>(a);
-  const QTile t = q_tile(a);
+  const unsigned wg = a.wg_base + blockIdx.x;
+  if (wg >= a.main_wgs) return fwd_aux<D, 4>(a, wg);
+  const QTile t = q_tile(a, wg);
   const Seq sq = seq_of(a, t.b);
   const int L = sq.L, W = a.W, S = a.S, hq = t.hq, b = t.b, qw = t.qw;
   if (t.q0 >= L) return;
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void dq32_kernel(const Args 
   constexpr int DB = kDB<D>;
   __shared__ __attribute__((aligned(16))) float lds[2 * KvTiles<D>::kBuf];
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
-  const QTile t = q_tile(a);
+  const QTile t = q_tile(a, a.wg_base + blockIdx.x);
   const Seq sq = seq_of(a, t.b);
   const int L = sq.L, W = a.W, S = a.S, hq = t.hq, b = t.b, qw = t.qw;
   if (t.q0 >= L) return;
@@ -558,11 +559,12 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void dkdv32_kernel(const Arg
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kh = wave & 1, hh = wave >> 1;
-  if (int(blockIdx.x) >= a.main_wgs) return bwd_aux<D, 4>(a, lds);
+  const unsigned wg = a.wg_base + blockIdx.x;
+  if (wg >= a.main_wgs) return bwd_aux<D, 4>(a, wg, lds);
   const int W = a.W, S = a.S, G = a.G, ns = a.kv_split;
   const int per = a.vl_kblocks ? a.vl_kblocks : a.n_kblocks;
   const int streams = ns * a.Hkv * (a.vl_kblocks ? 1 : a.B);
-  const int id = blockIdx.x;
+  const int id = int(wg);
   int kvh, b, kblk, piece = 0, chunk = -1;
   int64_t part_slot = 0;
   if (id < streams * per) {
@@ -823,22 +825,21 @@ __global__ __launch_bounds__(128) void fold32_kernel(const Args a) {
 template <int D>
 hipError_t fwd_d(const Args& a, hipStream_t s) {
   Args x = a;
-  const dim3 grid(grid_with_aux(x, int64_t(a.n_qtiles) * a.B * (a.Hq / a.wh), false));
-  hipLaunchKernelGGL(fwd32_kernel<D>, grid, dim3(256), 0, s, x);
-  return hipGetLastError();
+  return launch_in_ranges(x, wgs_with_aux(x, int64_t(a.n_qtiles) * a.B * (a.Hq / a.wh), false),
+                          [&](dim3 grid) { hipLaunchKernelGGL(fwd32_kernel<D>, grid, dim3(256), 0, s, x); });
 }
 template <int D>
 hipError_t dq_d(const Args& a, hipStream_t s) {
-  hipLaunchKernelGGL(dq32_kernel<D>, dim3(a.n_qtiles * a.B * (a.Hq / a.wh)), dim3(256), 0, s, a);
-  return hipGetLastError();
+  Args x = a;
+  return launch_in_ranges(x, int64_t(a.n_qtiles) * a.B * (a.Hq / a.wh),
+                          [&](dim3 grid) { hipLaunchKernelGGL(dq32_kernel<D>, grid, dim3(256), 0, s, x); });
 }
 template <int D>
 hipError_t dkdv_d(const Args& a, hipStream_t s) {
   const int blocks = a.Hkv * (a.vl_kblocks ? a.vl_kblocks : a.B * a.n_kblocks);
   Args x = a;
-  const dim3 grid(grid_with_aux(x, int64_t(a.kv_split) * blocks + a.n_chunk_wgs, true));
-  hipLaunchKernelGGL(dkdv32_kernel<D>, grid, dim3(256), 0, s, x);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_in_ranges(x, wgs_with_aux(x, int64_t(a.kv_split) * blocks + a.n_chunk_wgs, true),
+                                  [&](dim3 grid) { hipLaunchKernelGGL(dkdv32_kernel<D>, grid, dim3(256), 0, s, x); });
   if (e == hipSuccess && a.kv_split > 1) {
     hipLaunchKernelGGL(fold_pieces32_kernel<D>, dim3(4 * blocks), dim3(256), 0, s, a);
     e = hipGetLastError();

@@ -403,8 +403,8 @@ __global__ __launch_bounds__(256) void fwd_kernel(const Args a) {
   // (with a fixed stride the last workgroup of an XCD got 1.66x the first's at full causal).
   const int hwg = HPW * a.wh;
   const int n_tiles = a.n_qtiles * a.B * (a.Hq / hwg);
-  if (int(blockIdx.x) >= a.main_wgs) return fwd_aux<D, 2>(a);
-  const int xcd = blockIdx.x % NX, pos = blockIdx.x / NX, wgs_x = a.main_wgs / NX;
+  if (blockIdx.x >= a.main_wgs) return fwd_aux<D, 2>(a, blockIdx.x);
+  const int xcd = blockIdx.x % NX, pos = blockIdx.x / NX, wgs_x = int(a.main_wgs) / NX;
   const int per = n_tiles / NX, rem = n_tiles % NX;
   const int t_lo = xcd * per + min(xcd, rem), t_hi = t_lo + per + (xcd < rem ? 1 : 0);
 
@@ -779,10 +779,11 @@ __global__ __launch_bounds__(256, D == 128 || KSP == 4 ? 2 : 3) void fwd_split_k
   const int qi = ROWS ? wave % wq : 0, hi = wave / wq % wh, g = KSP == 1 ? 0 : wave / (wq * wh);
   const int W = a.W, S = a.S;
 
-  if (int(blockIdx.x) >= a.main_wgs) return fwd_aux<D, 2>(a);
+  const unsigned wg = a.wg_base + blockIdx.x;
+  if (wg >= a.main_wgs) return fwd_aux<D, 2>(a, wg);
   // workgroup -> row tile, batch, head set (see q_stream)
   const int gpk = a.G / (HPW * wh);
-  const QStream qs = q_stream(blockIdx.x, a.B * a.Hkv * gpk, a.cu_seqlens != nullptr);
+  const QStream qs = q_stream(int(wg), a.B * a.Hkv * gpk, a.cu_seqlens != nullptr);
   const int kvh = qs.stream / gpk / a.B, b = qs.stream / gpk % a.B;
   const int hw = kvh * a.G + (qs.stream % gpk * wh + hi) * HPW;
   const Seq sq = seq_of(a, b);
@@ -964,8 +965,8 @@ __global__ __launch_bounds__(256, 2) void fwd_slide_kernel(const Args a) {
   // unit -> (KV head, batch, head group, chunk), chunks fastest (as bwd_dq_slide_kernel); a packed
   // batch hands out only the chunks with rows: (KV head, head group), then each sequence's chunks
   const int hg_n = a.G / 8;
-  if (int(blockIdx.x) >= a.main_wgs) return fwd_aux<D, 2>(a);
-  const int unit = xcd_remap(blockIdx.x, a.main_wgs);
+  if (blockIdx.x >= a.main_wgs) return fwd_aux<D, 2>(a, blockIdx.x);
+  const int unit = xcd_remap(blockIdx.x, int(a.main_wgs));
   int chunk, hg, b, kvh;
   if constexpr (VL) {
     const int grp = unit / a.vl_units;
@@ -1157,15 +1158,15 @@ static hipError_t launch_fwd_h(const Args& a, hipStream_t stream) {
 template <typename E, int D, int HPW, int KSP>
 static hipError_t launch_fwd_split_k(const Args& a, hipStream_t stream) {
   Args x = a;
-  const dim3 grid(grid_with_aux(x, int64_t(a.n_qtiles) * a.B * (a.Hq / (HPW * a.wh)), false)), block(256);
-  if constexpr (KSP < 4) {
-    if (a.wq > 1) {
-      hipLaunchKernelGGL((fwd_split_kernel<E, D, HPW, KSP, true>), grid, block, 0, stream, x);
-      return hipGetLastError();
+  return launch_in_ranges(x, wgs_with_aux(x, int64_t(a.n_qtiles) * a.B * (a.Hq / (HPW * a.wh)), false), [&](dim3 grid) {
+    if constexpr (KSP < 4) {
+      if (a.wq > 1) {
+        hipLaunchKernelGGL((fwd_split_kernel<E, D, HPW, KSP, true>), grid, dim3(256), 0, stream, x);
+        return;
+      }
     }
-  }
-  hipLaunchKernelGGL((fwd_split_kernel<E, D, HPW, KSP, false>), grid, block, 0, stream, x);
-  return hipGetLastError();
+    hipLaunchKernelGGL((fwd_split_kernel<E, D, HPW, KSP, false>), grid, dim3(256), 0, stream, x);
+  });
 }
 
 template <typename E, int D, int HPW>
