@@ -96,6 +96,8 @@ struct Args {
 // packed batch with short ones) are cut into ranges of kRangeWgs, whole rounds of the 8 XCDs; `launch` gets a
 // range's grid, with args.wg_base set.
 constexpr int64_t kRangeWgs = int64_t(1) << 23;
+// The other launches are refused instead.
+inline bool grid_fits(int64_t wgs, int threads = 256) { return wgs * threads < int64_t(1) << 32; }
 template <typename F>
 inline hipError_t launch_in_ranges(Args& args, int64_t wgs, F&& launch) {
   for (int64_t lo = 0; lo < wgs; lo += kRangeWgs) {

@@ -1768,13 +1768,16 @@ static hipError_t launch_dkdv_d(const Args& a, hipStream_t stream) {
   if (a.sink_dq) ad.dq_wgs = a.dq_slide ? (a.G / 8) * a.slide_ncu : dq_grid<E, D, true>(a);
   hipError_t e;
   bool folded = false;
-  if (a.kv_split > 1) {  // (kv_split_plan leaves dkdv4_eligible shapes alone)
-    const int blocks = a.Hkv * (a.vl_kblocks ? a.vl_kblocks : a.B * a.n_kblocks);
-    hipLaunchKernelGGL((bwd_dkdv_kernel<E, D, false, true>), dim3(grid_with_aux(ad, int64_t(a.kv_split) * blocks + a.n_chunk_wgs, true)), dim3(256), 0, stream, ad);
+  // key blocks' workgroups and their sink-chunk ones
+  const int64_t blocks = int64_t(a.Hkv) * (a.vl_kblocks ? a.vl_kblocks : int64_t(a.B) * a.n_kblocks);
+  const int64_t all = wgs_with_aux(ad, a.kv_split * blocks + a.n_chunk_wgs, true);
+  if (!grid_fits(all)) return hipErrorInvalidConfiguration;
+  if (a.kv_split > 1) {  // (plan_kv_split leaves dkdv4_eligible shapes alone)
+    hipLaunchKernelGGL((bwd_dkdv_kernel<E, D, false, true>), dim3(unsigned(all)), dim3(256), 0, stream, ad);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     constexpr int kWgs = 2 * (D >= 32 ? D / 32 : 1);  // workgroups per key block
-    hipLaunchKernelGGL((bwd_dkdv_fold_kernel<E, D>), dim3(kWgs * blocks), dim3(256), 0, stream, ad);
+    hipLaunchKernelGGL((bwd_dkdv_fold_kernel<E, D>), dim3(unsigned(kWgs * blocks)), dim3(256), 0, stream, ad);
     e = hipGetLastError();
   } else if constexpr (D <= 64) {
     if (dkdv4_eligible(a, D, device_cus())) {
@@ -1797,11 +1800,9 @@ static hipError_t launch_dkdv_d(const Args& a, hipStream_t stream) {
       }
       e = hipGetLastError();
     } else {
-      const int per_kv = a.vl_kblocks ? a.vl_kblocks : a.B * a.n_kblocks;  // regular workgroups per KV head
-      const int grid = a.n_chunk_wgs + a.Hkv * per_kv;
-      const dim3 wgs(grid_with_aux(ad, grid, true));
+      const dim3 wgs = dim3(unsigned(all));
       bool kvl = false;
-      if constexpr (D == 64) kvl = dkdv_kvl_pays(a, grid);
+      if constexpr (D == 64) kvl = dkdv_kvl_pays(a, int(ad.main_wgs));
       if constexpr (D == 64) {
         if (kvl) hipLaunchKernelGGL((bwd_dkdv_kernel<E, D, true>), wgs, dim3(256), 0, stream, ad);
       }
@@ -1810,14 +1811,14 @@ static hipError_t launch_dkdv_d(const Args& a, hipStream_t stream) {
       folded = dkdv_folds_in_kernel(ad, D, kvl);
     }
   } else {
-    const int per_kv = a.vl_kblocks ? a.vl_kblocks : a.B * a.n_kblocks;
-    hipLaunchKernelGGL((bwd_dkdv_kernel<E, D>), dim3(grid_with_aux(ad, a.n_chunk_wgs + int64_t(a.Hkv) * per_kv, true)), dim3(256), 0, stream, ad);
+    hipLaunchKernelGGL((bwd_dkdv_kernel<E, D>), dim3(unsigned(all)), dim3(256), 0, stream, ad);
     e = hipGetLastError();
     folded = dkdv_folds_in_kernel(ad, D, false);
   }
   // the sink keys are folded inside the dK/dV kernel or by a launch of their own
   if (e != hipSuccess || a.nsp == 0 || folded) return e;
   const int64_t n = int64_t(a.B) * a.Hkv * min(a.S, kKvKeys * a.nsp);  // one workgroup per sink key
+  if (!grid_fits(n)) return hipErrorInvalidConfiguration;
   hipLaunchKernelGGL((bwd_sink_fold_kernel<E, D>), dim3(unsigned(n)), dim3(256), 0, stream, ad);
   return hipGetLastError();
 }

@@ -425,7 +425,9 @@ __global__ __launch_bounds__(512, 1) void bwd_dq_slide_kernel(const Args a) {
 template <typename E>
 static hipError_t launch_slide_e(const Args& a, hipStream_t stream) {
   const int per = a.vl_units ? a.vl_units : a.B * a.slide_ncu;  // units per (KV head, head group)
-  const dim3 grid(unsigned(a.Hkv * (a.G / kSlideWaves) * per)), block(512);
+  const int64_t units = int64_t(a.Hkv) * (a.G / kSlideWaves) * per;
+  if (!grid_fits(units, 512)) return hipErrorInvalidConfiguration;
+  const dim3 grid = dim3(unsigned(units)), block(512);
   if (a.vl_units) {
     if (a.sink_dq) hipLaunchKernelGGL((bwd_dq_slide_kernel<E, true, true>), grid, block, 0, stream, a);
     else hipLaunchKernelGGL((bwd_dq_slide_kernel<E, false, true>), grid, block, 0, stream, a);

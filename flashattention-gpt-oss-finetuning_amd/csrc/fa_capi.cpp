@@ -312,7 +312,8 @@ void plan_kv_split(fa::Args& a, int D, bool f32, char* ws, size_t spare) {
   const double rows = a.cu_seqlens ? std::min(double(a.L), std::max(1., double(a.token_rows) / a.B)) : double(a.L);
   int ns = kv_split_pieces(f32, D, a.G, a.Hkv, a.B, rows, a.L, a.W, a.sink_dq != 0, cus);
   const int64_t blocks = kv_blocks(a);
-  while (ns > 1 && (kv_part_bytes(D, blocks, ns) > spare || blocks * ns > (int64_t(1) << 24))) ns /= 2;
+  // (the fold has up to 8 workgroups per block)
+  while (ns > 1 && (kv_part_bytes(D, blocks, ns) > spare || blocks * std::max(ns, 8) > fa::kRangeWgs)) ns /= 2;
   a.kv_split = ns;
   a.kv_part = reinterpret_cast<float*>(ws);
 }

@@ -1121,7 +1121,9 @@ template <typename E>
 static hipError_t launch_fwd_slide_e(const Args& a, hipStream_t stream) {
   const int per = a.vl_units ? a.vl_units : a.B * a.slide_ncu;  // units per (KV head, head group)
   Args x = a;
-  const dim3 grid(grid_with_aux(x, int64_t(a.Hkv) * (a.G / 8) * per, false)), block(256);
+  const int64_t wgs = wgs_with_aux(x, int64_t(a.Hkv) * (a.G / 8) * per, false);
+  if (!grid_fits(wgs)) return hipErrorInvalidConfiguration;
+  const dim3 grid = dim3(unsigned(wgs)), block(256);
   if (a.vl_units) hipLaunchKernelGGL((fwd_slide_kernel<E, true>), grid, block, 0, stream, x);
   else hipLaunchKernelGGL((fwd_slide_kernel<E, false>), grid, block, 0, stream, x);
   return hipGetLastError();

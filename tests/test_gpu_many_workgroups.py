@@ -45,3 +45,17 @@ def test_grids_past_one_launch(gpu, longest, Hq, Hkv, D, W, S, dtype):
         err = float((a.float() - b.float()).norm() / b.float().norm())
         print(f"  {name}: {err:.2e}")
         assert err <= tol, (name, err)
+
+
+def test_a_grid_that_does_not_fit_is_refused(gpu):
+    """The sliding forward has at least one workgroup per sequence, KV head and 8 query heads: 2^21 sequences
+    of 8 KV heads are 2^24 of them, one too many for a launch."""
+    ops = load_mod("_ops")
+    B = 1 << 21
+    cu = torch.zeros(B + 1, dtype=torch.int32, device="cuda")
+    cu[-10:] = 4
+    q, k, v = (torch.randn(4, H, 64, device="cuda").to(BF) for H in (64, 8, 8))
+    with pytest.raises(RuntimeError, match="launch failed"):
+        ops.forward_varlen(q, k, v, cu, 8, 8, 0, 0.125)
+    o, _ = ops.forward_varlen(q, k, v, cu[-100:].contiguous(), 8, 8, 0, 0.125)
+    assert bool(torch.isfinite(o).all())
