@@ -35,51 +35,76 @@ __device__ inline void sum_sink_logits(const Args& a, int h, float* smem) {
   if (tid == 0) a.dsink[h] = (smem[0] + smem[1]) + (smem[2] + smem[3]);
 }
 
-// Workgroup `wg` of a.tail_wgs: calls fill(lo, hi, first, step) for every gap's rows [lo, hi), where this
-// thread takes the pieces first, first + step, ... of the gap.
+// Calls fill(lo, hi) for every gap's rows [lo, hi) that is not empty.
 template <typename F>
-__device__ inline void for_gaps(const Args& a, int wg, F&& fill) {
-  const int64_t first = int64_t(wg) * blockDim.x + threadIdx.x, step = int64_t(a.tail_wgs) * blockDim.x;
+__device__ inline void for_gaps(const Args& a, F&& fill) {
   const int total = a.total_rows;
+  auto gap = [&](int lo, int hi) {
+    if (lo < hi) fill(lo, hi);
+  };
   if (!a.seq_lens) {
     auto row = [&](int x) { return x < 0 ? 0 : (x > total ? total : x); };
     const int lo = row(a.cu_seqlens[0]);
-    fill(0, lo, first, step);
-    fill(max(lo, row(a.cu_seqlens[a.B])), total, first, step);
+    gap(0, lo);
+    gap(max(lo, row(a.cu_seqlens[a.B])), total);
     return;
   }
   int end = 0;  // of the sequences so far
   for (int b = 0; b < a.B; ++b) {
     const int lo = a.cu_seqlens[b];
-    fill(end, lo < total ? lo : total, first, step);
+    gap(end, lo < total ? lo : total);
     const int s = lo < 0 ? 0 : (lo > total ? total : lo), n = a.seq_lens[b];
     const int e = n < total - s ? s + (n < 0 ? 0 : n) : total;
     end = e > end ? e : end;
   }
-  fill(end, total, first, step);
+  gap(end, total);
 }
 
-// Rows [lo, hi) of a tensor of `heads` heads whose rows are `bytes` bytes (a multiple of 16): zeros.
-__device__ inline void zero_rows(void* ptr, const int64_t (&st)[3], int heads, int bytes, int eb, int lo, int hi,
-                                 int64_t first, int64_t step) {
-  const int pieces = bytes / 16;
-  const int64_t n = int64_t(hi - lo) * heads * pieces;
-  for (int64_t u = first; u < n; u += step) {
-    const int c = int(u % pieces), h = int(u / pieces % heads);
-    const int64_t r = lo + u / pieces / heads;
-    char* p = static_cast<char*>(ptr) + (h * st[1] + r * st[2]) * eb + 16 * c;
-    *reinterpret_cast<uint4*>(p) = uint4{0u, 0u, 0u, 0u};
+// One thread's share of the (row, head, 16-byte piece) units of a gap in a tensor of `heads` heads of BYTES
+// bytes: piece `c` of rows of a head, the head fastest.  Set up once per tensor; the loop over the units
+// then divides nothing, and is bound by the stores.  4 x 4096 rows in a buffer of 65536 (Hq = 64, Hkv = 8, D = 64,
+// window 128), in us, with a division and a modulo per store and 64 workgroups / with those and a launch of its own /
+// now: forward 358 / 273 / 167 (96 without the unused rows, whose 403 MB take 71 at 5.7 TB/s), backward 527 / 462
+// ... 502 / 354 ... 381 (264).
+template <int BYTES>
+struct GapUnits {
+  static constexpr int P = BYTES / 16;
+  int heads, c, row0, head0, drow, dhead;
+  __device__ __forceinline__ GapUnits(const Args& a, int wg, int heads) : heads(heads) {
+    const int t = wg * int(blockDim.x) + int(threadIdx.x), u = t / P, du = a.tail_wgs * int(blockDim.x) / P;
+    c = t % P;
+    row0 = u / heads;
+    head0 = u % heads;
+    drow = du / heads;
+    dhead = du % heads;
   }
-}
+  // zeros in rows [lo, hi) of the tensor at `ptr` with strides `st` in elements of EB bytes
+  template <int EB>
+  __device__ __forceinline__ void zero(void* ptr, const int64_t (&st)[3], int lo, int hi) const {
+    char* p = static_cast<char*>(ptr) + 16 * c;
+    int h = head0;
+    for (int64_t r = int64_t(lo) + row0; r < hi;) {
+      *reinterpret_cast<uint4*>(p + (h * st[1] + r * st[2]) * EB) = uint4{0u, 0u, 0u, 0u};
+      r += drow;
+      h += dhead;
+      if (h >= heads) {
+        h -= heads;
+        ++r;
+      }
+    }
+  }
+};
 
 // The forward's extra workgroups (`wg`: the workgroup's id); EB bytes per element of o.
 template <int D, int EB>
 __device__ inline void fwd_aux(const Args& a, unsigned wg) {
-  for_gaps(a, int(wg - a.main_wgs), [&](int lo, int hi, int64_t first, int64_t step) {
-    if (lo >= hi) return;
-    zero_rows(a.o_out, a.so_out, a.Hq, D * EB, EB, lo, hi, first, step);
-    for (int64_t u = first; u < int64_t(hi - lo) * a.Hq; u += step)
-      a.lse_out[int64_t(u % a.Hq) * a.slse[1] + (lo + u / a.Hq) * a.slse[2]] = -__builtin_inff();
+  const int x = int(wg - a.main_wgs);
+  const GapUnits<D * EB> o(a, x, a.Hq);
+  const int first = x * int(blockDim.x) + int(threadIdx.x), step = a.tail_wgs * int(blockDim.x);
+  for_gaps(a, [&](int lo, int hi) {
+    o.template zero<EB>(a.o_out, a.so_out, lo, hi);
+    for (int64_t r = lo + int64_t(first); r < hi; r += step)  // (rows fastest: lse is [head][row])
+      for (int h = 0; h < a.Hq; ++h) a.lse_out[h * a.slse[1] + r * a.slse[2]] = -__builtin_inff();
   });
 }
 
@@ -91,19 +116,20 @@ __device__ inline void bwd_aux(const Args& a, unsigned wg, float* smem) {
     if (x < a.Hq) return sum_sink_logits(a, x, smem);
     x -= a.Hq;
   }
-  for_gaps(a, x, [&](int lo, int hi, int64_t first, int64_t step) {
-    if (lo >= hi) return;
-    zero_rows(a.dq, a.sdq, a.Hq, D * EB, EB, lo, hi, first, step);
-    zero_rows(a.dk, a.sdk, a.Hkv, D * EB, EB, lo, hi, first, step);
-    zero_rows(a.dv, a.sdv, a.Hkv, D * EB, EB, lo, hi, first, step);
+  const GapUnits<D * EB> q(a, x, a.Hq), kv(a, x, a.Hkv);
+  for_gaps(a, [&](int lo, int hi) {
+    q.template zero<EB>(a.dq, a.sdq, lo, hi);
+    kv.template zero<EB>(a.dk, a.sdk, lo, hi);
+    kv.template zero<EB>(a.dv, a.sdv, lo, hi);
   });
 }
 
-// Host: workgroups behind a kernel's own `main` (a.main_wgs and a.tail_wgs are set): all of the launch's.
-// Without seq_lens a packed batch usually covers every row, and its workgroups only read two offsets.
+// Host: workgroups behind a kernel's own `main`, 256 for the rows of no sequence: with 64 the case above takes
+// 199 and 388 us, and a batch that covers every row, where they only read two offsets, is no faster (0.3%, less
+// than two runs differ).  (a.main_wgs and a.tail_wgs are set): all of the launch's.
 inline int64_t wgs_with_aux(Args& a, int64_t main, bool bwd) {
   a.main_wgs = unsigned(main);
-  a.tail_wgs = !a.cu_seqlens ? 0 : a.seq_lens ? 256 : 64;
+  a.tail_wgs = a.cu_seqlens ? 256 : 0;
   return main + a.tail_wgs + (bwd && a.dsink ? a.Hq : 0);
 }
 inline unsigned grid_with_aux(Args& a, int64_t main, bool bwd) { return unsigned(wgs_with_aux(a, main, bwd)); }

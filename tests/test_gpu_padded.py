@@ -89,6 +89,37 @@ def test_bad_ranges_stay_inside_the_tensors(gpu):
     assert torch.equal(o, ref) and bool((o[20:60] == 0).all())
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,dtype", [(64, 8, 64, BF), (6, 3, 128, FP), (5, 1, 16, BF), (7, 7, 32, F32)])
+def test_rows_of_no_sequence(gpu, Hq, Hkv, D, dtype):
+    """A packed buffer with long unused stretches before, between and after its sequences: o, dq, dk and dv are
+    0 and lse is -inf on every row outside them, and only there."""
+    ops = load_mod("_ops")
+    total, starts, lens = 9000, (2500, 2533, 6000), (33, 0, 700)
+    rows = torch.zeros(total, dtype=torch.bool)
+    for s, n in zip(starts, lens):
+        rows[s:s + n] = True
+    q, k, v, do = (torch.randn(total, H, D, device="cuda").to(dtype) for H in (Hq, Hkv, Hkv, Hq))
+    b = ops.autograd_binding(q)
+    leaves = [t.requires_grad_() for t in (q, k, v)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    forms = [(lambda: b.swda_varlen(*leaves, i32(starts), i32(lens), 700, sum(lens), 128, 0, 0.125), rows)]
+    cu = i32((2500, 2533, 3000))  # (the first and last rows of the buffer are unused)
+    covered = torch.zeros(total, dtype=torch.bool)
+    covered[2500:3000] = True
+    forms.append((lambda: b.swda_varlen(*leaves, cu, None, 467, 0, 128, 0, 0.125), covered))
+    for f, on in forms:
+        junk = [torch.full_like(t, 7.0) for t in (q, q, k, v)]
+        del junk  # (what unwritten outputs would hold)
+        o = f()
+        grads = torch.autograd.grad(o, leaves, do)
+        for t in (o, *grads):
+            assert bool((t[~on] == 0).all()) and bool(torch.isfinite(t).all())
+        for t in (o, grads[2]):  # (a first row's dq is 0: it sees one key)
+            assert bool((t[on] != 0).any(-1).all())
+    _, lse = ops.forward_varlen(q, k, v, cu, 467, 128, 0, 0.125)
+    assert torch.equal(torch.isinf(lse), (~covered).cuda().expand_as(lse)) and bool((lse[:, ~covered] < 0).all())
+
+
 @pytest.mark.parametrize("D,window,sinks", [(64, 128, True), (64, None, False), (128, 200, True)])
 def test_packed_function_equals_the_python_one(gpu, D, window, sinks):
     fa = load_pkg()
