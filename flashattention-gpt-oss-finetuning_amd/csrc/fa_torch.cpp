@@ -287,8 +287,14 @@ void check_packed(const std::vector<std::pair<const at::Tensor*, const char*>>& 
 }
 
 // A packed [total, H, D] tensor as the [1, H, total, D] view the C ABI describes (the batch stride is not
-// used there), copied where the kernels cannot read it.
-at::Tensor as_bhld(const at::Tensor& t) { return kernel_ready(t.permute({1, 0, 2}).unsqueeze(0)); }
+// used there), copied where the kernels cannot read it.  `in_place`: the caller leaves its rows where they are,
+// at strides that it did not choose, so they are also copied where a sequence of that many rows spans more
+// than the kernels' 32-bit offsets.
+at::Tensor as_bhld(const at::Tensor& t, int64_t in_place = 0) {
+  const int64_t span = ((in_place - 1) * t.stride(0) + t.size(2)) * int64_t(t.element_size());
+  const at::Tensor x = in_place > 0 && span >= (int64_t(1) << 31) ? t.contiguous() : t;
+  return kernel_ready(x.permute({1, 0, 2}).unsqueeze(0));
+}
 
 // The sequences of a packed batch: offsets [B + 1], or starts [B] with lengths.
 struct Sequences {
@@ -296,6 +302,7 @@ struct Sequences {
   int64_t max_seqlen, token_rows;
   int64_t batch() const { return cu.size(0) - (lens.defined() ? 0 : 1); }
   const int32_t* cu_ptr() const { return cu.data_ptr<int32_t>(); }
+  int64_t in_place() const { return lens.defined() ? max_seqlen : 0; }
   const int32_t* lens_ptr() const { return lens.defined() ? lens.data_ptr<int32_t>() : nullptr; }
 };
 
@@ -315,7 +322,8 @@ std::vector<at::Tensor> fwd_packed(const at::Tensor& q, const at::Tensor& k, con
   check_packed({{&q, "q"}, {&k, "k"}, {&v, "v"}});
   const c10::DeviceGuard guard(q.device());
   const int64_t total = q.size(0), Hq = q.size(1), D = q.size(2);
-  const at::Tensor qv = as_bhld(q), kv = as_bhld(k), vv = as_bhld(v);
+  const int64_t ip = sq.in_place();
+  const at::Tensor qv = as_bhld(q, ip), kv = as_bhld(k, ip), vv = as_bhld(v, ip);
   const at::Tensor sinks = sinks_in.defined() ? sinks_ready(sinks_in, Hq, q) : at::Tensor();
   at::Tensor o = at::empty({total, Hq, D}, q.options());
   at::Tensor lse = at::empty({Hq, total}, q.options().dtype(at::kFloat));
@@ -358,7 +366,8 @@ std::vector<at::Tensor> bwd_packed(const at::Tensor& q, const at::Tensor& k, con
   check_packed({{&q, "q"}, {&k, "k"}, {&v, "v"}, {&o, "o"}, {&dout, "do"}});
   const c10::DeviceGuard guard(q.device());
   const int64_t total = q.size(0), Hq = q.size(1), D = q.size(2), Hkv = k.size(1);
-  const at::Tensor qv = as_bhld(q), kv = as_bhld(k), vv = as_bhld(v), ov = as_bhld(o), dov = as_bhld(dout);
+  const int64_t ip = sq.in_place();
+  const at::Tensor qv = as_bhld(q, ip), kv = as_bhld(k, ip), vv = as_bhld(v, ip), ov = as_bhld(o), dov = as_bhld(dout, ip);
   const at::Tensor sinks = sinks_in.defined() ? sinks_ready(sinks_in, Hq, q) : at::Tensor();
   at::Tensor dq = at::empty({total, Hq, D}, q.options());
   at::Tensor dk = at::empty({total, Hkv, D}, q.options());

@@ -214,7 +214,7 @@ def padded_attention(q, k, v, attention_mask, window_size: Optional[int] = None,
         return q.new_zeros(B, L, Hq, D)
     W = max_len if window_size is None else int(window_size)
     b = _ops.autograd_binding(q)
-    if b is not None and starts is not None:
+    if b is not None and starts is not None and B * L < 2 ** 31:  # (int32 row numbers)
         # contiguous tokens: the kernels read each sequence's rows where they are
         rows = lambda x: x.transpose(1, 2).reshape(B * L, x.shape[1], D)
         qr, kr, vr = rows(q), rows(k), rows(v)

@@ -89,6 +89,26 @@ def test_bad_ranges_stay_inside_the_tensors(gpu):
     assert torch.equal(o, ref) and bool((o[20:60] == 0).all())
 
 
+def test_rows_far_apart(gpu):
+    """q, k and v as slices of one wide buffer whose rows span more than the kernels' 32-bit offsets reach:
+    copied closer together, as gathering does."""
+    gpt_oss = load_mod("gpt_oss")
+    B, L, Hq, Hkv, D, lens = 2, 16500, 4, 1, 64, (16500, 16391)
+    wide = torch.empty(B, L, 1 << 16, dtype=BF, device="cuda")
+    cut = lambda H, c: wide[..., c:c + H * D].normal_().view(B, L, H, D).transpose(1, 2)
+    q, k, v = cut(Hq, 0), cut(Hkv, Hq * D), cut(Hkv, (Hq + 1) * D)
+    assert (max(lens) - 1) * q.stride(2) * 2 >= 1 << 31
+    do = wide[..., 512:512 + Hq * D].normal_().view(B, L, Hq, D)
+    mask = mask_of(lens, L, False)
+    results = []
+    for x in ((q, k, v), [t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v)]):
+        leaves = [t.detach().requires_grad_() for t in x]
+        o = gpt_oss.padded_attention(*leaves, mask, window_size=100)
+        results.append([o, *torch.autograd.grad(o, leaves, do)])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("Hq,Hkv,D,dtype", [(64, 8, 64, BF), (6, 3, 128, FP), (5, 1, 16, BF), (7, 7, 32, F32)])
 def test_rows_of_no_sequence(gpu, Hq, Hkv, D, dtype):
     """A packed buffer with long unused stretches before, between and after its sequences: o, dq, dk and dv are
