@@ -1,7 +1,8 @@
 """GPU parity of dQ with one tile per workgroup (bwd_dq_split_kernel): shapes for which 1, 2 or 4 waves
 share a tile's keys, one or more row tiles per workgroup, ragged lengths, windows and sink keys whose
 gradients the dK/dV kernel takes, against the float32 oracle with the bar of tests/test_gpu_parity.py.
-dK, dV (which read this kernel's row statistics) and the learned sinks' gradient are checked too.
+dK, dV (which read this kernel's row statistics; the sink keys' rows, which chunk workgroups add up, with that
+file's wider bar) and the learned sinks' gradient are checked too.
 """
 import math
 
@@ -10,7 +11,7 @@ import torch
 
 from conftest import load_mod
 from oracle import naive
-from test_gpu_parity import assert_close, make_inputs
+from test_gpu_parity import assert_close, make_inputs, naive_reference, sink_rows
 from test_gpu_sinks import check_dsinks
 
 pytestmark = pytest.mark.gpu
@@ -37,6 +38,7 @@ CASES = [
     pytest.param(2, 6, 2, 1153, 128, 300, 3, FP, id="D128-G3-sinks-in-chunks"),
     pytest.param(1, 4, 1, 1090, 64, 1024, 1, BF, id="D64-G4-one-ragged-chunk"),
     pytest.param(1, 16, 2, 2500, 64, 1100, 16, FP, id="D64-G8-sinks-in-chunks"),
+    pytest.param(2, 8, 1, 1200, 64, 1024, 5, BF, id="D64-G8-two-chunks"),
     pytest.param(1, 6, 6, 511, 16, 511, 0, FP, id="4w-D16"),
     pytest.param(4, 16, 16, 3001, 16, 3001, 0, FP, id="D16-row-tiles"),
     pytest.param(1, 16, 1, 900, 32, 900, 0, BF, id="4w-D32"),
@@ -62,8 +64,10 @@ def test_dq_split(gpu, B, Hq, Hkv, L, D, W, S, dtype):
             ref = naive.attention_fwd_bwd_sinks(q, k, v, sk, do, W, S, scale=sc, compute_dtype=torch.float32,
                                                 row_chunk=512)
         assert_close("dQ", grads[0], ref[2])
-        keys = slice(S, None)  # (the sink keys' rows sum every row's rounded terms: see test_gpu_parity.py)
-        assert_close("dK", grads[1][:, :, keys], ref[3][:, :, keys])
-        assert_close("dV", grads[2][:, :, keys], ref[4][:, :, keys])
+        # the sink keys' rows sum every row's rounded terms, whatever the learned sinks: without those
+        nv = naive_reference(q, k, v, do, W, S, sc) if S > 0 and sk is None else (None,) * 4
+        keys = slice(0 if sk is None else S, None)
+        assert_close("dK", grads[1][:, :, keys], ref[3][:, :, keys], nv[2], sink_rows(L, S))
+        assert_close("dV", grads[2][:, :, keys], ref[4][:, :, keys], nv[3], sink_rows(L, S))
         if sk is not None:
             check_dsinks(grads[3], ref[5], ref[1], ref[0], do, sk, range(Hq))

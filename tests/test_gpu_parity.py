@@ -240,7 +240,8 @@ KV_LDS_CASES = [
 @pytest.mark.parametrize("B,Hq,Hkv,L,D,W,S,dtype", KV_LDS_CASES)
 def test_kv_operands_in_lds_path(gpu, B, Hq, Hkv, L, D, W, S, dtype):
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    assert B * Hkv * -(-L // 64) >= 6 * cus and W <= 512, "the shape no longer takes the K/V-in-LDS variant"
+    wgs = B * Hkv * (-(-L // 64) + (-(-(L - (63 + W) // 32 * 32) // 64) if S > 16 else 0))
+    assert W <= 1024 and 1.12 * -(-wgs // (3 * cus)) < -(-wgs // (2 * cus)), "the shape no longer takes the K/V-in-LDS variant"
     print(f"case B={B} Hq={Hq} Hkv={Hkv} L={L} D={D} W={W} S={S} {dtype}", flush=True)
     run_case(B, Hq, Hkv, L, D, W, S, dtype, seed=W + S)
 
@@ -308,8 +309,10 @@ def test_backward_is_deterministic(gpu):
 # partial sums in a fixed order and use no atomics, whichever path the C ABI picks.
 DETERMINISM_CASES = [
     pytest.param(1, 64, 8, 4096, 64, 128, 4, BF, id="c2-slide-dq-64key-dkdv"),
-    pytest.param(1, 8, 2, 2048, 64, 2048, 0, BF, id="full-causal-generic-dq"),
-    pytest.param(2, 8, 2, 1024, 128, 256, 16, FP, id="D128-sink-rows-in-dq"),
+    pytest.param(1, 8, 2, 2048, 64, 2048, 0, BF, id="full-causal-split-dq"),
+    pytest.param(2, 8, 2, 1024, 128, 256, 16, FP, id="D128-sinks-in-chunks"),
+    pytest.param(2, 8, 2, 1024, 128, 100, 16, FP, id="D128-sink-rows-in-dq"),
+    pytest.param(1, 16, 16, 2048, 16, 256, 0, FP, id="D16-resident-dq-no-sinks"),
     pytest.param(1, 16, 16, 2048, 16, 256, 4, FP, id="D16-G1"),
     pytest.param(1, 8, 2, 1500, 64, 64, 40, BF, id="S40-chunks-and-fold"),
     pytest.param(1, 4, 2, 600, 64, 100, 4, torch.float32, id="float32"),

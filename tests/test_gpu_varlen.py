@@ -95,6 +95,9 @@ def run_varlen(cu, Hq, Hkv, D, W, S, dtype, seed=0, sinks=False, with_naive=True
     pytest.param([0, 500, 1200], 4, 1, 32, None, 0, BF, id="full-causal-D32"),
     pytest.param([0, 64, 128, 192, 256], 16, 2, 64, 32, 4, BF, id="equal-lengths"),
     pytest.param([0, 0, 1, 1, 2], 2, 1, 64, 8, 1, FP, id="tiny-and-empty"),
+    # few sink keys under long windows: their gradients are added up by the dK/dV kernel's chunks
+    pytest.param([0, 1150, 1151, 2500, 2560], 4, 1, 64, 1024, 3, BF, id="few-sinks-in-chunks"),
+    pytest.param([0, 400, 400, 1033], 4, 2, 128, 256, 16, FP, id="few-sinks-in-chunks-D128"),
     pytest.param([0, 2048, 4096], 64, 8, 64, 128, 4, BF, id="gpt-oss-shape-two-sequences"),
     # short sequences beside long ones on the sliding kernels, whose units are sized by the rows
     # the batch holds (not by B x the longest sequence): sink rows in the dQ kernel, then in
