@@ -403,7 +403,7 @@ __global__ __launch_bounds__(256) void fwd_kernel(const Args a) {
   // (with a fixed stride the last workgroup of an XCD got 1.66x the first's at full causal).
   const int hwg = HPW * a.wh;
   const int n_tiles = a.n_qtiles * a.B * (a.Hq / hwg);
-  if (blockIdx.x >= a.main_wgs) return fwd_aux<D, 2>(a, blockIdx.x);
+  if (F8 == 0 && blockIdx.x >= a.main_wgs) return fwd_aux<D, 2>(a, blockIdx.x);  // (no packed fp8 batches)
   const int xcd = blockIdx.x % NX, pos = blockIdx.x / NX, wgs_x = int(a.main_wgs) / NX;
   const int per = n_tiles / NX, rem = n_tiles % NX;
   const int t_lo = xcd * per + min(xcd, rem), t_hi = t_lo + per + (xcd < rem ? 1 : 0);
