@@ -212,20 +212,24 @@ extern "C" int fa_quantize_fp8_amax(const void* x, int32_t dtype, int64_t n, voi
   if (!parts || !host_parts || !amax) return FA_ERR_NULL;
   const dim3 grid(FA_AMAX_PARTS), block(fa::kThreads);
   const hipStream_t s = static_cast<hipStream_t>(stream);
+  hipStreamCaptureStatus capture;  // (the host cannot wait for a captured kernel, which would write `host_parts` at replays)
+  if (hipStreamIsCapturing(s, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return FA_ERR_LAUNCH;
   if (dtype == FA_DTYPE_BF16) hipLaunchKernelGGL(fa::amax_kernel<fa::LoadBF16>, grid, block, 0, s, x, n, parts, host_parts);
   else if (dtype == FA_DTYPE_F16) hipLaunchKernelGGL(fa::amax_kernel<fa::LoadF16>, grid, block, 0, s, x, n, parts, host_parts);
   else hipLaunchKernelGGL(fa::amax_kernel<fa::LoadF32>, grid, block, 0, s, x, n, parts, host_parts);
   if (hipGetLastError() != hipSuccess) return FA_ERR_LAUNCH;
   // the host waits for the first kernel only, while the second runs
-  hipEvent_t known;
-  if (hipEventCreateWithFlags(&known, hipEventDisableTiming) != hipSuccess) return FA_ERR_LAUNCH;
-  bool good = hipEventRecord(known, s) == hipSuccess;
+  hipEvent_t known = nullptr;
+  bool good = hipEventCreateWithFlags(&known, hipEventDisableTiming) == hipSuccess && hipEventRecord(known, s) == hipSuccess;
   if (good) {
     fa::launch_quantize(x, dtype, n, out, 0.f, parts, s);
     good = hipGetLastError() == hipSuccess && hipEventSynchronize(known) == hipSuccess;
   }
-  (void)hipEventDestroy(known);
-  if (!good) return FA_ERR_LAUNCH;
+  if (known) (void)hipEventDestroy(known);
+  if (!good) {
+    (void)hipStreamSynchronize(s);  // the caller takes `host_parts` back
+    return FA_ERR_LAUNCH;
+  }
   uint32_t m = 0;
   for (int i = 0; i < FA_AMAX_PARTS; ++i) {
     uint32_t v;

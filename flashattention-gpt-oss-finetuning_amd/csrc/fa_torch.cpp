@@ -15,6 +15,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
@@ -480,6 +481,8 @@ py::object quantize_fp8(const at::Tensor& x_in, c10::optional<double> descale) {
                      "fa_quantize_fp8");
     return py::make_tuple(x8, *descale);
   }
+  if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None)
+    raise_for_status(FA_ERR_LAUNCH, "fa_quantize_fp8_amax under graph capture, where the host cannot read the maximum");
   at::Tensor parts = at::empty({FA_AMAX_PARTS}, x.options().dtype(at::kFloat));
   at::Tensor host = at::empty({FA_AMAX_PARTS}, at::TensorOptions().dtype(at::kFloat).pinned_memory(true));
   float amax = 0.f;

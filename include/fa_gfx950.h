@@ -230,7 +230,8 @@ int fa_bwd_ranges(const fa_bwd_params* p, const int32_t* starts, const int32_t* 
  * that maximum is 0 or NaN) and returns the maximum (NaN if x holds one) in *amax: it enqueues
  * everything, then blocks the host until the maximum is known, while the codes are still being
  * written.  `parts` is FA_AMAX_PARTS floats of device memory, `host_parts` as many of pinned host
- * memory; both are free again when the codes are written (stream order) and at return. */
+ * memory; both are free again when the codes are written (stream order) and at return.  It returns
+ * FA_ERR_LAUNCH in a stream that is being captured. */
 #define FA_AMAX_PARTS 1024
 int fa_quantize_fp8(const void* x, int32_t dtype, int64_t n, void* out, double descale, void* stream);
 int fa_quantize_fp8_amax(const void* x, int32_t dtype, int64_t n, void* out, float* parts, float* host_parts,

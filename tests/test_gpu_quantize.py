@@ -106,3 +106,24 @@ def test_traced_and_transformed_calls(gpu):
         assert f(fake).shape == (4, 64)
     assert f(fake).dtype == torch.float8_e4m3fn
     assert type(f(x.as_subclass(_Sub))) is _Sub and same(f(x.as_subclass(_Sub)).as_subclass(torch.Tensor), x)
+
+
+def test_graph_capture(gpu):
+    """Under capture a given scale quantises in the graph; without one, which the host would have to read
+    back, the call is refused before it enqueues anything."""
+    fa = load_pkg()
+    x = torch.randn(3, 1000, device=gpu).bfloat16()
+    check(x, 0.02)
+    count = torch.zeros(1, device=gpu)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        count.add_(1)
+        codes = fa.quantize_fp8(x, 0.02)[0]
+        with pytest.raises(RuntimeError, match="capture"):
+            fa.quantize_fp8(x)
+    for i in range(3):
+        x.normal_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(codes.view(torch.uint8), reference(x, 0.02)[0].view(torch.uint8)) and int(count) == i + 1
+    check(x)
