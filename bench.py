@@ -95,10 +95,12 @@ def kernel_accounting(cfg):
     }
 
 
-# Kernels launched by each stage of the C ABI: the forward and dQ stages run one of two kernels
-# (the sliding ones for the GPT-OSS sliding layers); fa_bwd_dkdv may also launch the sink fold.
-STAGE_KERNELS = {"fwd": ["fwd_kernel", "fwd_slide_kernel"], "bwd_dq": ["bwd_dq_kernel", "bwd_dq_slide_kernel"],
-                 "bwd_dkdv": ["bwd_dkdv_kernel", "bwd_sink_fold_kernel"]}
+# Kernels launched by each stage of the C ABI: the forward and dQ stages run one of three kernels
+# (the sliding ones for the GPT-OSS sliding layers); fa_bwd_dkdv may also launch the folds of its key
+# blocks' pieces and of the sink keys.
+STAGE_KERNELS = {"fwd": ["fwd_kernel", "fwd_slide_kernel", "fwd_split_kernel"],
+                 "bwd_dq": ["bwd_dq_kernel", "bwd_dq_slide_kernel", "bwd_dq_split_kernel"],
+                 "bwd_dkdv": ["bwd_dkdv_kernel", "bwd_dkdv4_kernel", "bwd_dkdv_fold_kernel", "bwd_sink_fold_kernel"]}
 
 
 def measured_traffic(config, stage):
