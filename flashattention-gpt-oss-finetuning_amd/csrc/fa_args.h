@@ -77,7 +77,7 @@ struct Args {
   // B x n_kblocks blocks).
   int vl_units;
   int vl_kblocks;
-  // dK/dV split (kv_split > 1, see kv_split_plan in fa_capi.cpp): every key block's steps are cut into
+  // dK/dV split (kv_split > 1, see plan_kv_split in fa_capi.cpp): every key block's steps are cut into
   // kv_split pieces, one workgroup each, whose fp32 sums go to kv_part [key block][piece][dK, dV]
   // [64 D]; bwd_dkdv_fold_kernel adds the pieces in order.
   int kv_split;
@@ -195,7 +195,7 @@ __device__ __forceinline__ KvPiece kv_piece(int id, int streams, int ns) {
 // With `rotate` (a packed batch) the streams take turns: an XCD's workgroups go to its shader engines in
 // turn, so where the streams of an XCD are a multiple of them, one engine would get every tile of the same
 // sequences.  Full causal forward, Hq = 64, Hkv = 8, D = 64, without -> with: sequences of 1536, 1187, 640 and
-// 933 rows 91 -> 74 us; of 4096, 2048, 1024, 512, 3000, 1500, 700 and 3504 rows 763 -> 442 us.
+// 933 rows 83 -> 66 us; of 4096, 2048, 1024, 512, 3000, 1500, 700 and 3504 rows 727 -> 413 us.
 struct QStream {
   int stream, pos;
 };

@@ -754,7 +754,8 @@ __global__ __launch_bounds__(256) void fwd_kernel(const Args a) {
 //
 // Against fwd_kernel, which walks tiles with resident workgroups (register-staged key blocks, Q stashed in
 // LDS, mask patterns: 64 KB of LDS, 208 VGPRs, two workgroups per CU at D = 64): one tile per workgroup
-// needs 16 KB and 168 VGPRs, three per CU, and the dispatcher evens out the tiles' lengths.  In us, bf16,
+// needs 16 KB and 168 VGPRs, three per CU (KSP = 2 holds two registers more, which spill to scratch memory), and
+// the dispatcher evens out the tiles' lengths.  In us, bf16,
 // D = 64, Hq = 64, Hkv = 8, full causal, KSP = 1 / 2 / 4: L = 512 17.8 / 13.0 / 11.5 (fwd_kernel 18.8);
 // L = 1024 29.7 / 23.4 / 25.0 (31.4); L = 2048 63 / 48 / 65 (69); L = 4096 152 / 160 / 206 (160); L = 8192
 // 551 / 582 / 734 (600).  KSP = 1 gives fwd_kernel's results bit for bit.
