@@ -85,13 +85,14 @@ def _padding_facts(attention_mask: torch.Tensor):
     first = i.argmax(1)
     last = L - 1 - i.flip(1).argmax(1)
     whole = ((last - first + 1 == lens) | (lens == 0)).all()
+    starts = (first + L * torch.arange(B, device=m.device)).to(torch.int32)
+    # the host waits here, after everything that it hands out is enqueued: layers on other streams use it at once
     full, whole, longest, tokens = torch.stack((m.all().to(torch.int64), whole.to(torch.int64), lens.max().to(torch.int64),
                                                 lens.sum())).tolist()
     if full:
         return True, None, None, L, tokens, None
     if not whole:
         return False, None, None, longest, tokens, _mask_facts(m)
-    starts = (first + L * torch.arange(B, device=m.device)).to(torch.int32)
     return False, starts, lens, longest, tokens, None
 
 

@@ -19,6 +19,36 @@ def test_mask_facts_padded_and_full():
     assert gpt_oss._mask_facts(torch.ones(2, 5, dtype=torch.long))[0] is True
 
 
+def test_padding_facts_are_complete_when_the_host_has_them(monkeypatch):
+    """Layers on other streams use the facts at once, so nothing may be enqueued for them after the host's
+    wait (the tolist of the summary)."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    late, waited = [], []
+    plain = torch.Tensor.tolist
+
+    def tolist(t):
+        r = plain(t)
+        waited.append(True)
+        return r
+
+    class Log(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if waited:
+                late.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    m = torch.tensor([[1, 1, 1, 0, 0], [0, 1, 1, 1, 1], [0, 0, 0, 0, 0]], dtype=torch.bool)
+    monkeypatch.setattr(torch.Tensor, "tolist", tolist)
+    with Log():
+        full, starts, lens, longest, tokens, packed = gpt_oss._padding_facts(m)
+    monkeypatch.undo()
+    assert waited and not late, late
+    assert (full, longest, tokens, packed) == (0, 4, 7, None)
+    assert starts.tolist() == [0, 6, 10] and lens.tolist() == [3, 4, 0]
+    assert starts.dtype == lens.dtype == torch.int32
+
+
 def test_position_facts_packed_row():
     # three sequences of 4, 2 and 3 tokens packed into one row
     p = torch.tensor([[0, 1, 2, 3, 0, 1, 0, 1, 2]])
