@@ -19,34 +19,30 @@ def test_mask_facts_padded_and_full():
     assert gpt_oss._mask_facts(torch.ones(2, 5, dtype=torch.long))[0] is True
 
 
-def test_padding_facts_are_complete_when_the_host_has_them(monkeypatch):
-    """Layers on other streams use the facts at once, so nothing may be enqueued for them after the host's
-    wait (the tolist of the summary)."""
-    from torch.utils._python_dispatch import TorchDispatchMode
-
-    late, waited = [], []
-    plain = torch.Tensor.tolist
-
-    def tolist(t):
-        r = plain(t)
-        waited.append(True)
-        return r
-
-    class Log(TorchDispatchMode):
-        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
-            if waited:
-                late.append(str(func))
-            return func(*args, **(kwargs or {}))
-
-    m = torch.tensor([[1, 1, 1, 0, 0], [0, 1, 1, 1, 1], [0, 0, 0, 0, 0]], dtype=torch.bool)
-    monkeypatch.setattr(torch.Tensor, "tolist", tolist)
-    with Log():
-        full, starts, lens, longest, tokens, packed = gpt_oss._padding_facts(m)
-    monkeypatch.undo()
-    assert waited and not late, late
-    assert (full, longest, tokens, packed) == (0, 4, 7, None)
-    assert starts.tolist() == [0, 6, 10] and lens.tolist() == [3, 4, 0]
-    assert starts.dtype == lens.dtype == torch.int32
+@pytest.mark.parametrize("seed", range(6))
+def test_padding_facts_against_loops(seed):
+    g = torch.Generator().manual_seed(seed)
+    B, L = 1 + seed, (1, 2, 31, 64, 65, 300)[seed]
+    for kind in ("runs", "left", "right", "gaps", "empty"):
+        rows = []
+        for b in range(B):
+            n = int(torch.randint(0, L + 1, (1,), generator=g)) if kind != "empty" else 0
+            s = {"left": L - n, "right": 0}.get(kind, int(torch.randint(0, L - n + 1, (1,), generator=g)))
+            r = torch.zeros(L, dtype=torch.long)
+            r[s:s + n] = 1
+            rows.append(torch.randint(0, 2, (L,), generator=g) if kind == "gaps" else r)
+        mask = torch.stack(rows)
+        full, starts, lens, longest, tokens, packed = gpt_oss._padding_facts(mask)
+        where = [r.nonzero().view(-1).tolist() for r in mask]
+        assert full == (mask.sum() == B * L)
+        if full:
+            continue
+        assert longest == max(len(w) for w in where) and tokens == sum(len(w) for w in where)
+        if any(w and w != list(range(w[0], w[0] + len(w))) for w in where):
+            assert starts is lens is None and packed[1].tolist() == mask.view(-1).nonzero().view(-1).tolist()
+        else:
+            assert packed is None and lens.tolist() == [len(w) for w in where]
+            assert [x for x, w in zip(starts.tolist(), where) if w] == [b * L + w[0] for b, w in enumerate(where) if w]
 
 
 def test_position_facts_packed_row():

@@ -159,3 +159,27 @@ def test_packed_function_equals_the_python_one(gpu, D, window, sinks):
         fa.flash_swda_with_sink_varlen(leaves[0], leaves[1][:, :, :32], leaves[2], cu, 549, window)
     with pytest.raises(ValueError, match="max_seqlen is required"):
         fa.flash_swda_with_sink_varlen(*leaves, cu, None, window)
+
+
+@pytest.mark.parametrize("L", [700, 20000])
+def test_mask_facts_are_complete_when_the_host_has_them(gpu, L):
+    """Layers on other streams use a mask's facts at once, so nothing may be left to run for them; masks that
+    the host works out and, larger, the device."""
+    facts = load_mod("gpt_oss")._padding_facts
+    mask = torch.zeros(3, L, dtype=torch.long, device=gpu)
+    mask[0], mask[1, 50:60] = 1, 1
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        for _ in range(3):
+            full, starts, lens, longest, tokens, packed = facts(mask)
+            assert stream.query()
+            assert (full, longest, tokens, packed) == (False, L, L + 10, None)
+            assert starts.tolist() == [0, L + 50, 2 * L] and lens.tolist() == [L, 10, 0]
+            assert starts.dtype == lens.dtype == torch.int32 and starts.is_cuda
+            mask[0, 5] = 0
+            full, starts, lens, longest, tokens, packed = facts(mask)
+            assert stream.query() and not full and starts is lens is None
+            assert (longest, tokens, packed[3]) == (L - 1, L + 9, L - 1) and packed[2].tolist() == [0, L - 1, L + 9, L + 9]
+            mask[0, 5] = 1
+            assert facts(torch.ones_like(mask)) == (True, None, None, L, 3 * L, None)
