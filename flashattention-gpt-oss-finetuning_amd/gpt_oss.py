@@ -29,7 +29,7 @@ from .attention import _check_packed_shapes, _swda, flash_swda_with_sink_varlen
 class _BatchFacts:
     """Host-side facts about one batch's padding mask or position ids (which rows hold tokens,
     where the packed sequences start, the longest one).  Working them out reads device memory,
-    i.e. synchronises the host once; transformers hands the same tensor object to every attention
+    i.e. the host waits for the GPU; transformers hands the same tensor object to every attention
     layer of a forward pass, so the facts are kept for that tensor (while it lives and is not
     modified in place) and the other layers enqueue their kernels without waiting for the GPU.
 
