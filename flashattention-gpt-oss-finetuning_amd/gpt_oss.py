@@ -87,7 +87,7 @@ def _padding_facts(attention_mask: torch.Tensor):
     h = m.cpu() if m.numel() <= 32768 else m
     if m.numel() == 0 or bool(h.all()):
         return True, None, None, L, m.numel(), None
-    i = h.view(torch.uint8)
+    i = h.to(torch.uint8)
     lens = i.sum(1)
     first = i.argmax(1)
     gaps = ((L - i.flip(1).argmax(1) - first != lens) & (lens > 0)).any()
