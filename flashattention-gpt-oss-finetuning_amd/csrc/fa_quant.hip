@@ -4,7 +4,7 @@
 // reads it for max |x|, one reads it again and writes the e4m3 codes.  Both are bound by memory.  As
 // chained elementwise PyTorch operations (to float32, abs, max, divide, clamp, convert) the same work
 // moved about eight times the bytes.  Quantising q, k and v and the fp8 forward of a full causal layer
-// (L = 8192, Hq = 64, Hkv = 8, D = 64, bfloat16 in): 884 -> 605 us, of which the forward is 520.  The
+// (L = 8192, Hq = 64, Hkv = 8, D = 64, bfloat16 in): 882 -> 599 us, of which the forward is 515.  The
 // host waits for the maximum only, behind which the codes are already being written, so three
 // tensors in a row keep the GPU busy but for the launches.
 //
